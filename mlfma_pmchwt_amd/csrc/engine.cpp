@@ -456,6 +456,7 @@ void Engine::build_near() {
         };
         return work(a) > work(b);
     });
+    build_near_split(planes);
     nd_.nitem = (int)items.size();
     nd_.items = upload(items);
     nd_.planes = planes;
@@ -510,6 +511,47 @@ void Engine::build_near() {
         launch_narrow(st, nunk, d_dinv_, d_dinvf_);
     }
     MLFMA_HIP(hipGetLastError());
+}
+
+// Items of the single-vector near product when the leaves alone do not fill
+// the chip.  A workgroup streams one block row at about 20-25 GB/s, so a leaf
+// of B bytes takes B / 22 GB/s however idle the rest of the chip is: 15,360
+// PMCHWT unknowns in 56 leaves of 25 MB took 1.27 ms (1.1 TB/s).  With column
+// ranges of about 1/1024 of all entries (at least 128 KB, at least 16 columns)
+// every CU holds several (the same product: 0.19 ms); their partial sums cost
+// a second, small launch (about 4 us), so leaves under 512 KB (or 2,048 and more of them: 300,000 RWG
+// in 3,200 leaves of 2.1 MB stream at 5.9 TB/s unsplit) stay whole.
+void Engine::build_near_split(int planes) {
+    const std::vector<int>& lp = tree.leaf_ptr;
+    const size_t esize = sizeof(double2);
+    size_t total = 0, most = 0;
+    for (int t = 0; t < nleaf; ++t) {
+        const size_t b = (size_t)planes * tgt_cols[t] * (lp[t + 1] - lp[t]) * esize;
+        total += b;
+        most = std::max(most, b);
+    }
+    nd_.nsplit = 0;
+    if (nleaf >= 2048 || most < (512u << 10)) return;
+    const size_t target = std::max<size_t>(total / 1024, 128u << 10);
+    std::vector<int4> split;
+    std::vector<long long> part_ptr(nleaf + 1, 0);
+    const int nx = planes == 3 ? 2 : 1;
+    for (int t = 0; t < nleaf; ++t) {
+        const int nt = lp[t + 1] - lp[t], C = tgt_cols[t];
+        const size_t bytes = (size_t)planes * C * nt * esize;
+        const int n = (int)std::max<size_t>(1, std::min<size_t>((bytes + target - 1) / target, (C + 15) / 16));
+        for (int k = 0; k < n; ++k)
+            split.push_back(make_int4(t, (int)((long long)C * k / n), (int)((long long)C * (k + 1) / n), k));
+        part_ptr[t + 1] = part_ptr[t] + (long long)n * nx * nt;
+    }
+    std::stable_sort(split.begin(), split.end(), [&](int4 a, int4 b) {
+        return (long long)(a.z - a.y) * (lp[a.x + 1] - lp[a.x]) > (long long)(b.z - b.y) * (lp[b.x + 1] - lp[b.x]);
+    });
+    nd_.nsplit = (int)split.size();
+    nd_.split = upload(split);
+    nd_.part_ptr = upload(part_ptr);
+    nd_.part = dalloc<double2>((size_t)part_ptr[nleaf]);
+    nd_.leaf_of = d_leaf_of_;
 }
 
 // Copy of one leaf-pair block, planes x (ns x nt column-major).

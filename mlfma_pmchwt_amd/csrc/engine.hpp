@@ -238,6 +238,7 @@ private:
     void build_device_tree();
     void build_wave(int w);
     void build_near();
+    void build_near_split(int planes);
     template <typename R>
     FarDev<R>& far(int w);
     template <typename R>

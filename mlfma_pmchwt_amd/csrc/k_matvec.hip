@@ -1153,17 +1153,23 @@ MLFMA_FAR_INSTANTIATE(float)
 // consecutive addresses; U columns per thread are in flight at once.  The
 // group partials are summed in LDS in a fixed order.  x is gathered into LDS
 // CH columns at a time.  Entries are stored in S (double or float) and
-// accumulated in FP64.
-template <typename S, int P, int BS, int U, int CH>
+// accumulated in FP64.  SPLIT: a workgroup takes the column range of one
+// NearDev::split item instead of the whole block row and leaves its rows'
+// partial sums in `part`, which k_near_fold adds up.
+template <typename S, int P, int BS, int U, int CH, bool SPLIT>
 __global__ __launch_bounds__(BS) void k_near(NearDev nd, const cplx_t<S>* __restrict__ Z,
-                                             const double2* __restrict__ x, double2* __restrict__ y) {
+                                             const double2* __restrict__ x, double2* __restrict__ y,
+                                             double2* __restrict__ part) {
     constexpr int NX = (P == 3) ? 2 : 1;
     __shared__ double2 xs[NX][CH];
     __shared__ double2 red[NX][BS];
-    const int t = nd.order[blockIdx.x];
+    const int4 it = SPLIT ? nd.split[blockIdx.x] : make_int4(nd.order[blockIdx.x], 0, 0, 0);
+    const int t = it.x;
     const int i0 = nd.leaf_ptr[t], nt = nd.leaf_ptr[t + 1] - i0;
     if (nt == 0) return;
     const int C = nd.tgt_cols[t];
+    const int ca = SPLIT ? it.y : 0, cb = SPLIT ? it.z : C;   // this workgroup's columns
+    if (SPLIT) part += nd.part_ptr[t] + (size_t)it.w * NX * nt;
     const int* cref = nd.colref + nd.col_ptr[t];
     const int plane = C * nt;   // < 2^31: one target's block row
     const cplx_t<S>* Zt = Z + nd.tgt_off[t];
@@ -1174,8 +1180,8 @@ __global__ __launch_bounds__(BS) void k_near(NearDev nd, const cplx_t<S>* __rest
         const int row = r0 + rl;
         const bool act = g < G && row < nt;
         double2 aJ = {0, 0}, aM = {0, 0};
-        for (int c0 = 0; c0 < C; c0 += CH) {
-            const int cl = min(CH, C - c0);
+        for (int c0 = ca; c0 < cb; c0 += CH) {
+            const int cl = min(CH, cb - c0);
             __syncthreads();
             for (int c = threadIdx.x; c < cl; c += BS) {
                 const int r = cref[c0 + c];
@@ -1227,6 +1233,17 @@ __global__ __launch_bounds__(BS) void k_near(NearDev nd, const cplx_t<S>* __rest
                 }
             }
         }
+        // row `q` of the leaf is done (column groups folded)
+        auto put = [&](int q, double2 sJ, double2 sM) {
+            if (SPLIT) {
+                part[q] = sJ;
+                if (P == 3) part[nt + q] = sM;
+            } else {
+                const int r = nd.perm[i0 + q];
+                y[r] = sJ;
+                if (P == 3) y[nd.N + r] = sM;
+            }
+        };
         if (G > 1) {   // nt < BS: a single row pass, fold the column groups
             red[0][threadIdx.x] = aJ;
             if (P == 3) red[NX - 1][threadIdx.x] = aM;
@@ -1237,23 +1254,47 @@ __global__ __launch_bounds__(BS) void k_near(NearDev nd, const cplx_t<S>* __rest
                     sJ = cadd(sJ, red[0][h * nt + threadIdx.x]);
                     if (P == 3) sM = cadd(sM, red[NX - 1][h * nt + threadIdx.x]);
                 }
-                const int r = nd.perm[i0 + threadIdx.x];
-                y[r] = sJ;
-                if (P == 3) y[nd.N + r] = sM;
+                put(threadIdx.x, sJ, sM);
             }
         } else if (act) {   // G == 1: threads past nt hold no row
-            const int r = nd.perm[i0 + row];
-            y[r] = aJ;
-            if (P == 3) y[nd.N + r] = aM;
+            put(row, aJ, aM);
         }
     }
+}
+
+// y of the split near product: each row's partial sums in item order.
+template <int P>
+__global__ __launch_bounds__(256) void k_near_fold(NearDev nd, const int* __restrict__ leaf_of,
+                                                   const double2* __restrict__ part, double2* __restrict__ y) {
+    constexpr int NX = (P == 3) ? 2 : 1;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= NX * nd.N) return;
+    const int cur = e / nd.N, i = e - cur * nd.N;
+    const int t = leaf_of[i], i0 = nd.leaf_ptr[t], nt = nd.leaf_ptr[t + 1] - i0;
+    const size_t p0 = nd.part_ptr[t];
+    const int cnt = (int)((nd.part_ptr[t + 1] - p0) / ((size_t)NX * nt));
+    const double2* p = part + p0 + (size_t)cur * nt + (i - i0);
+    double2 s = p[0];
+    for (int k = 1; k < cnt; ++k) s = cadd(s, p[(size_t)k * NX * nt]);
+    y[(size_t)cur * nd.N + nd.perm[i]] = s;
 }
 
 template <typename S>
 void launch_near(hipStream_t st, const NearDev& nd, const cplx_t<S>* Z, const double2* x, double2* y) {
     if (nd.nleaf == 0) return;
-    if (nd.planes == 1) k_near<S, 1, 512, 8, 1024><<<nd.nleaf, 512, 0, st>>>(nd, Z, x, y);
-    else k_near<S, 3, 512, 4, 512><<<nd.nleaf, 512, 0, st>>>(nd, Z, x, y);
+    if (nd.nsplit > 0) {   // few or large leaves (Engine::build_near)
+        const int NX = nd.planes == 1 ? 1 : 2, fb = (NX * nd.N + 255) / 256;
+        if (nd.planes == 1) {
+            k_near<S, 1, 512, 8, 1024, true><<<nd.nsplit, 512, 0, st>>>(nd, Z, x, y, nd.part);
+            k_near_fold<1><<<fb, 256, 0, st>>>(nd, nd.leaf_of, nd.part, y);
+        } else {
+            k_near<S, 3, 512, 4, 512, true><<<nd.nsplit, 512, 0, st>>>(nd, Z, x, y, nd.part);
+            k_near_fold<3><<<fb, 256, 0, st>>>(nd, nd.leaf_of, nd.part, y);
+        }
+        return;
+    }
+    if (nd.planes == 1) k_near<S, 1, 512, 8, 1024, false><<<nd.nleaf, 512, 0, st>>>(nd, Z, x, y, nullptr);
+    else k_near<S, 3, 512, 4, 512, false><<<nd.nleaf, 512, 0, st>>>(nd, Z, x, y, nullptr);
 }
 template void launch_near<double>(hipStream_t, const NearDev&, const double2*, const double2*, double2*);
 template void launch_near<float>(hipStream_t, const NearDev&, const float2*, const double2*, double2*);
