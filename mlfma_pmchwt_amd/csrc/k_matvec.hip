@@ -114,11 +114,97 @@ __global__ __launch_bounds__(512) void k_aggregate(int K, int N, int ldr, int r0
     }
 }
 
+// The single-vector aggregation where there are few leaves: a workgroup takes
+// 64 samples of one leaf and its four wavefronts every fourth RWG each, so a
+// leaf is spread over K / 64 workgroups; the wavefronts' sums are added in a
+// fixed order through LDS.
+template <typename R, int NCUR>
+__global__ __launch_bounds__(256) void k_aggregate_t(int K, int N, int tiles, const int* __restrict__ order,
+                                                     const int* __restrict__ leaf_ptr, const int* __restrict__ perm,
+                                                     const cplx_t<R>* __restrict__ Vs, const double2* __restrict__ x,
+                                                     cplx_t<R>* __restrict__ Sm) {
+    using C = cplx_t<R>;
+    constexpr int CHUNK = 256, D = NCUR * 3;
+    __shared__ C xl[NCUR][CHUNK];
+    __shared__ C red[3][D][64];
+    const int leaf = order[blockIdx.x / tiles];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int q = (blockIdx.x % tiles) * 64 + lane;
+    const bool act = q < K;
+    const int i0 = leaf_ptr[leaf], i1 = leaf_ptr[leaf + 1];
+    C acc[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) acc[d] = C{0, 0};
+    const size_t s3 = (size_t)3 * K;
+    for (int b = i0; b < i1; b += CHUNK) {
+        const int n = min(CHUNK, i1 - b);
+        __syncthreads();
+        for (int e = threadIdx.x; e < n; e += 256) {
+            const int r = perm[b + e];
+#pragma unroll
+            for (int c = 0; c < NCUR; ++c) narrow(x[(size_t)c * N + r], xl[c][e]);
+        }
+        __syncthreads();
+        if (act) {
+            const C* v = Vs + (size_t)(b + wave) * s3 + q;
+            int j = wave;
+            for (; j + 12 < n; j += 16, v += 16 * s3) {
+                C a[4][3];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) a[u][d] = v[(size_t)(4 * u) * s3 + (size_t)d * K];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int c = 0; c < NCUR; ++c)
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) cfma(acc[c * 3 + d], a[u][d], xl[c][j + 4 * u]);
+            }
+            for (; j < n; j += 4, v += 4 * s3) {
+                const C a0 = v[0], a1 = v[K], a2 = v[2 * (size_t)K];
+#pragma unroll
+                for (int c = 0; c < NCUR; ++c) {
+                    cfma(acc[c * 3 + 0], a0, xl[c][j]);
+                    cfma(acc[c * 3 + 1], a1, xl[c][j]);
+                    cfma(acc[c * 3 + 2], a2, xl[c][j]);
+                }
+            }
+        }
+    }
+    if (wave > 0)
+#pragma unroll
+        for (int d = 0; d < D; ++d) red[wave - 1][d][lane] = acc[d];
+    __syncthreads();
+    if (wave == 0 && act) {
+        C* s = Sm + (size_t)leaf * D * K + q;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            C a = acc[d];
+#pragma unroll
+            for (int w = 0; w < 3; ++w) a.x += red[w][d][lane].x, a.y += red[w][d][lane].y;
+            s[(size_t)d * K] = a;
+        }
+    }
+}
+
+// One workgroup per leaf needs enough leaves: 7,680 RWG in 56 leaves (PMCHWT,
+// FP64, both wavenumbers, 346 MB of patterns) take 310 us that way and 88 us in
+// sample tiles, 480 RWG 7.1 and 5.0 us.  With 3,200 leaves (300,000 RWG,
+// 4.9 GB) whole rows stream slightly better, 917 against 944 us.
+constexpr int kAggTileLeaves = 1024;
+
 template <typename R>
 void launch_aggregate_b(hipStream_t st, int ncur, int rb, int nleaf, int K, int N, int ldr, int r0, const int* order,
                         const int* leaf_ptr, const int* perm, const cplx_t<R>* Vs, const double2* x,
                         cplx_t<R>* Sm) {
     if (nleaf == 0) return;
+    if (rb == 1 && ldr == 1 && nleaf < kAggTileLeaves) {
+        const int tiles = (K + 63) / 64;
+        if (ncur == 1) k_aggregate_t<R, 1><<<nleaf * tiles, 256, 0, st>>>(K, N, tiles, order, leaf_ptr, perm, Vs, x, Sm);
+        else k_aggregate_t<R, 2><<<nleaf * tiles, 256, 0, st>>>(K, N, tiles, order, leaf_ptr, perm, Vs, x, Sm);
+        return;
+    }
     const int threads = std::min(512, (K + 63) / 64 * 64);
 #define AGG(NCUR, RB) k_aggregate<R, NCUR, RB><<<nleaf, threads, 0, st>>>(K, N, ldr, r0, order, leaf_ptr, perm, Vs, x, Sm)
     if (ncur == 1) {
