@@ -7,6 +7,7 @@
 // the real type R of the patterns, tables and workspaces (double or float);
 // they accumulate in R.  Solver vectors x, y and the near field stay FP64.
 #include <algorithm>
+#include <complex>
 
 #include "kernels.hpp"
 #include <stdexcept>
@@ -1058,14 +1059,147 @@ __global__ __launch_bounds__(256) void k_disagg_pec(int N, int K, int ldr, int r
     }
 }
 
+// Single-vector disaggregation, both equations (Code/MLFMM.cpp:211-227,
+// :285-351).  A wavefront streams ROWS consecutive RWG rows together; rows of
+// one leaf share its effective vectors: PEC E = B, PMCHWT (the K integral
+// sum (-khat x V).B with khat = -kp is sum V.(kp x B)) for the J and M outputs
+//   E_J = a B_J - c kp x B_M,   E_M = c kp x B_J + b B_M
+// with a, b, c the wavenumber's constants over the common factor `scale`, which
+// multiplies the sums in FP64 (k1: a = b = c = 1).  Forming E once per ROWS rows in
+// place of one row's L and K sums cuts the L2 reads of B, which bounded the
+// row-per-wavefront form (7,680 RWG, 346 MB of patterns: 98 us, now 76).  KS = 4:
+// the block's wavefronts split the samples of the same rows instead, for few
+// rows (480 RWG, PEC: 11.7 us with four rows a wavefront, 4.1 with one a block).
+template <typename R>
+struct DisaggWave {
+    int K;
+    const cplx_t<R>*Vf, *Bm;
+    const R* kp;
+    double2 a, b, c;
+};
+
+template <typename R, bool PM, int ROWS, int KS>
+__global__ __launch_bounds__(256) void k_disagg_one(int N, int nw, int ldr, int r0, const int* __restrict__ leaf_of,
+                                                    const int* __restrict__ perm, DisaggWave<R> w0, DisaggWave<R> w1,
+                                                    double2 scale, double2* __restrict__ y) {
+    using C = cplx_t<R>;
+    constexpr int NO = PM ? 2 : 1;
+    __shared__ C red[KS == 1 ? 1 : 4][ROWS * NO];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int i00 = (KS == 1 ? blockIdx.x * 4 + wave : blockIdx.x) * ROWS;
+    if (KS == 1 && i00 >= N) return;
+    int leaf[ROWS];
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) leaf[u] = __builtin_amdgcn_readfirstlane(leaf_of[min(i00 + u, N - 1)]);
+    C s[ROWS][NO];
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+        for (int o = 0; o < NO; ++o) s[u][o] = C{0, 0};
+    for (int w = 0; w < nw; ++w) {
+        const DisaggWave<R> W = w == 0 ? w0 : w1;
+        const int K = W.K;
+        const C ca = C{(R)W.a.x, (R)W.a.y}, cb = C{(R)W.b.x, (R)W.b.y}, cc = C{(R)W.c.x, (R)W.c.y};
+        for (int q = lane + (KS == 1 ? 0 : 64 * wave); q < K; q += 64 * KS) {
+            C v[ROWS][3];
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                const C* V = W.Vf + (size_t)min(i00 + u, N - 1) * 3 * K + q;   // rows past N repeat N-1
+#pragma unroll
+                for (int d = 0; d < 3; ++d) v[u][d] = V[(size_t)d * K];
+            }
+            C e[NO][3];
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u) {
+                if (u == 0 || leaf[u] != leaf[u - 1]) {   // uniform over the wavefront
+                    const C* B = W.Bm + (size_t)leaf[u] * NO * 3 * K + q;
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) e[0][d] = B[(size_t)d * K];
+                    if constexpr (PM) {
+                        const R kx = W.kp[q], ky = W.kp[K + q], kz = W.kp[2 * K + q];
+                        const C j0 = e[0][0], j1 = e[0][1], j2 = e[0][2];
+                        const C m0 = B[(size_t)3 * K], m1 = B[(size_t)4 * K], m2 = B[(size_t)5 * K];
+                        // kp x B
+                        const C cj[3] = {csub(cscale(j2, ky), cscale(j1, kz)), csub(cscale(j0, kz), cscale(j2, kx)),
+                                         csub(cscale(j1, kx), cscale(j0, ky))};
+                        const C cm[3] = {csub(cscale(m2, ky), cscale(m1, kz)), csub(cscale(m0, kz), cscale(m2, kx)),
+                                         csub(cscale(m1, kx), cscale(m0, ky))};
+                        const C m[3] = {m0, m1, m2};
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) {
+                            e[0][d] = csub(cmul(ca, e[0][d]), cmul(cc, cm[d]));
+                            e[NO - 1][d] = cadd(cmul(cc, cj[d]), cmul(cb, m[d]));
+                        }
+                    }
+                }
+#pragma unroll
+                for (int o = 0; o < NO; ++o)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) cfma(s[u][o], v[u][d], e[o][d]);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+        for (int o = 0; o < NO; ++o) s[u][o] = wave_sum(s[u][o]);
+    if (KS > 1) {
+        if (lane == 0)
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+                for (int o = 0; o < NO; ++o) red[wave][u * NO + o] = s[u][o];
+        __syncthreads();
+        if (wave > 0) return;
+    }
+    if (lane < ROWS * NO) {   // lane u * NO + o writes row u, output o
+        const int u = lane / NO, o = lane - u * NO;
+        C v = s[0][0];
+        if (KS > 1) {
+            v = red[0][lane];
+            for (int k = 1; k < 4; ++k) v.x += red[k][lane].x, v.y += red[k][lane].y;
+        } else {
+#pragma unroll
+            for (int uu = 0; uu < ROWS; ++uu)
+#pragma unroll
+                for (int oo = 0; oo < NO; ++oo)
+                    if (uu == u && oo == o) v = s[uu][oo];
+        }
+        if (i00 + u < N) {
+            double2* yp = y + ((size_t)o * N + perm[i00 + u]) * ldr + r0;
+            double2 t = *yp;
+            cfma(t, scale, widen(v));
+            *yp = t;
+        }
+    }
+}
+
+// Rows per wavefront and sample split by the number of rows: from 16,384 rows
+// whole rows by fours give every SIMD four wavefronts and more (300,000 RWG:
+// 809 us, 6.0 TB/s), fewer take all four wavefronts of a block for the same
+// rows, very few one row a block.
+template <typename R, bool PM>
+void disagg_one(hipStream_t st, int N, int nw, int ldr, int r0, const int* leaf_of, const int* perm,
+                const DisaggWave<R>& w0, const DisaggWave<R>& w1, double2 scale, double2* y) {
+    if (N >= 16384)
+        k_disagg_one<R, PM, 4, 1><<<(N + 15) / 16, 256, 0, st>>>(N, nw, ldr, r0, leaf_of, perm, w0, w1, scale, y);
+    else if (N >= 2048)
+        k_disagg_one<R, PM, 4, 4><<<(N + 3) / 4, 256, 0, st>>>(N, nw, ldr, r0, leaf_of, perm, w0, w1, scale, y);
+    else
+        k_disagg_one<R, PM, 1, 4><<<N, 256, 0, st>>>(N, nw, ldr, r0, leaf_of, perm, w0, w1, scale, y);
+}
+
 template <typename R>
 void launch_disagg_pec_b(hipStream_t st, int rb, int N, int K, int ldr, int r0, const int* leaf_of, const int* perm,
                          const cplx_t<R>* Vf, const cplx_t<R>* Bm, double2 c, double2* y) {
 #define DIS(ROWS, RB)                                                                                      \
     k_disagg_pec<R, ROWS, RB><<<(N + 4 * ROWS - 1) / (4 * ROWS), 256, 0, st>>>(N, K, ldr, r0, leaf_of, perm, Vf, \
                                                                                Bm, c, y)
-    if (rb == 1) DIS(4, 1);
-    else if (rb == 2) DIS(2, 2);
+    if (rb == 1) {
+        const double2 one = make_double2(1.0, 0.0);
+        const DisaggWave<R> w{K, Vf, Bm, nullptr, one, one, one};
+        disagg_one<R, false>(st, N, 1, ldr, r0, leaf_of, perm, w, w, c, y);
+    } else if (rb == 2) DIS(2, 2);
     else if (rb == 4) DIS(1, 4);
     else DIS(1, 8);
 #undef DIS
@@ -1172,8 +1306,16 @@ template <typename R>
 void launch_disagg_pmchwt_b(hipStream_t st, int rb, int ldr, int r0, const int* leaf_of, const int* perm,
                             const PmchwtFarArgs<R>& a, double2* y) {
     const int blocks = (a.N + 3) / 4;
-    if (rb == 1) k_disagg_pmchwt<R, 1><<<blocks, 256, 0, st>>>(ldr, r0, leaf_of, perm, a, y);
-    else if (rb == 2) k_disagg_pmchwt<R, 2><<<blocks, 256, 0, st>>>(ldr, r0, leaf_of, perm, a, y);
+    if (rb == 1) {
+        using Z = std::complex<double>;
+        auto z = [](double2 v) { return Z(v.x, v.y); };
+        auto d = [](Z v) { return make_double2(v.real(), v.imag()); };
+        const double2 one = make_double2(1.0, 0.0);
+        const Z c = z(a.c2) / z(a.c1);
+        const DisaggWave<R> w0{a.K1, a.Vf1, a.B1, a.kp1, one, one, one};
+        const DisaggWave<R> w1{a.K2, a.Vf2, a.B2, a.kp2, d(c * z(a.etai)), d(c * z(a.inv_etai)), d(c)};
+        disagg_one<R, true>(st, a.N, 2, ldr, r0, leaf_of, perm, w0, w1, a.c1, y);
+    } else if (rb == 2) k_disagg_pmchwt<R, 2><<<blocks, 256, 0, st>>>(ldr, r0, leaf_of, perm, a, y);
     else if (rb == 4) k_disagg_pmchwt<R, 4><<<blocks, 256, 0, st>>>(ldr, r0, leaf_of, perm, a, y);
     else if constexpr (sizeof(R) == 4) k_disagg_pmchwt<R, 8><<<blocks, 256, 0, st>>>(ldr, r0, leaf_of, perm, a, y);
     else throw std::invalid_argument("FP64 disaggregation: at most 4 right-hand sides per pass");
@@ -1360,8 +1502,17 @@ __global__ __launch_bounds__(256) void k_near_fold(NearDev nd, const int* __rest
     const size_t p0 = nd.part_ptr[t];
     const int cnt = (int)((nd.part_ptr[t + 1] - p0) / ((size_t)NX * nt));
     const double2* p = part + p0 + (size_t)cur * nt + (i - i0);
+    const size_t step = (size_t)NX * nt;
     double2 s = p[0];
-    for (int k = 1; k < cnt; ++k) s = cadd(s, p[(size_t)k * NX * nt]);
+    int k = 1;
+    for (; k + 7 < cnt; k += 8) {   // eight loads in flight
+        double2 a[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a[u] = p[(size_t)(k + u) * step];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s = cadd(s, a[u]);
+    }
+    for (; k < cnt; ++k) s = cadd(s, p[(size_t)k * step]);
     y[(size_t)cur * nd.N + nd.perm[i]] = s;
 }
 

@@ -30,3 +30,45 @@ def test_aggregation_tiles(freq, radius, leaf, ie):
                 bound = 2 * len(xs) * np.finfo(float).eps * np.einsum("nqc,n->qc", np.abs(v), np.abs(xs))
                 got = op.workspace(wn, cur, 0, op.max_level, t)
                 assert np.all(np.abs(got - want) <= bound + 1e-300), (t, wn, cur)
+
+
+# fewer than 2,048 rows (one row a block), up to 16,384 (four rows, samples split), above (rows by
+# fours), with row counts and sample counts that are no multiple of the tiles
+@pytest.mark.parametrize("ie", [api.EFIE, api.PMCHWT])
+@pytest.mark.parametrize("freq,radius", [(5, 0.7), (13, 0.9), (25, 1.3)])
+def test_disaggregation_rows(freq, radius, ie):
+    op = api.Operator(geometry.geodesic_sphere(freq, radius), integral_equation=ie, eps_r_re=3.0, eps_r_im=-0.2)
+    n = op.n_rwg
+    rng = np.random.default_rng(freq + ie)
+    op.stage(api.STAGE_AGGREGATE, rng.standard_normal(op.n) + 1j * rng.standard_normal(op.n))
+    op.stage(api.STAGE_M2M)
+    op.stage(api.STAGE_M2L_L2L)
+    y = op.stage(api.STAGE_FAR)
+    ptr, rwg = op.level_list(op.max_level, 4)
+    box = np.empty(n, dtype=int)
+    for t in range(len(ptr) - 1):
+        box[rwg[ptr[t]:ptr[t + 1]]] = t
+    order = np.argsort(box, kind="stable")        # internal rows are leaf by leaf
+    k0, eta0 = 2 * np.pi, 119.9169832 * np.pi
+    er = 3.0 - 0.2j
+    for i in np.unique(np.concatenate([order[:5], order[-5:], order[ptr[1] - 3:ptr[1] + 3], rng.integers(0, n, 8)])):
+        want, size = np.zeros(2, complex), np.zeros(2)
+        for wn, k in enumerate([k0, k0 * np.sqrt(er)] if ie == api.PMCHWT else [k0], 1):
+            v = op.pattern(wn, 1, int(i))
+            b = [op.workspace(wn, c, 1, op.max_level, box[i]) for c in range(2 if ie == api.PMCHWT else 1)]
+            if ie != api.PMCHWT:
+                c = (k * eta0 / (4 * np.pi)) * (k / (4 * np.pi))
+                want[0], size[0] = c * np.sum(v * b[0]), abs(c) * np.sum(np.abs(v * b[0]))
+                continue
+            _, th, ph, _, _ = op.grid(wn, op.max_level)
+            T, P = np.meshgrid(th, ph, indexing="ij")
+            kp = np.stack([np.sin(T) * np.cos(P), np.sin(T) * np.sin(P), np.cos(T)], -1).reshape(-1, 3)
+            c, z = k * k / (16 * np.pi * np.pi), 1.0 if wn == 1 else np.sqrt(1.0 / er)
+            lj, lm = (np.sum(v * b[q]) for q in (0, 1))
+            kj, km = (np.sum(v * np.cross(kp, b[q])) for q in (0, 1))
+            want += [c * (z * lj - km), c * (kj + lm / z)]
+            size += abs(c) * 4 * np.sum(np.abs(v)) * max(np.abs(b[0]).max(), np.abs(b[1]).max())
+        got = [y[i]] + ([y[n + i]] if ie == api.PMCHWT else [])
+        # sums of 3K products in two orders, a few roundings per product
+        bound = (6 * v.size + 64) * np.finfo(float).eps * size
+        assert np.all(np.abs(np.array(got) - want[:len(got)]) <= bound[:len(got)]), i
