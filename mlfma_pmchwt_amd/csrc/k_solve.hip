@@ -193,18 +193,35 @@ void launch_multidot_b(hipStream_t st, int n, int R, int m, const float2* V, siz
     k_multidot_b<float2><<<dim3(nblk, (m + kDotJ - 1) / kDotJ), 256, 0, st>>>(n, R, m, V, ldv, w, partial);
 }
 
-// out[j * R + r] = sum_b partial[(j * nblk + b) * R + r], b ascending
-__global__ void k_reduce_partials_b(int nblk, int R, const double2* __restrict__ partial, double2* __restrict__ out) {
-    const int j = blockIdx.x;
-    for (int r = threadIdx.x; r < R; r += blockDim.x) {
-        double2 s = make_double2(0, 0);
-        for (int b = 0; b < nblk; ++b) s = cadd(s, partial[((size_t)j * nblk + b) * R + r]);
-        out[(size_t)j * R + r] = s;
+// out[j * R + r] = sum_b partial[(j * nblk + b) * R + r].  A block takes one
+// vector j and 8 right-hand sides (128-byte reads); its 32 slices take every
+// 32nd partial sum and are added pairwise in a fixed order.  One thread per
+// right-hand side walking all 256 partial sums was a chain of 256 dependent
+// adds behind their loads: 60 us per call at 8 right-hand sides, a quarter of
+// the inner near-field solve; in slices 4 us.
+__global__ __launch_bounds__(256) void k_reduce_partials_b(int nblk, int R, const double2* __restrict__ partial,
+                                                           double2* __restrict__ out) {
+    __shared__ double2 red[4][8];
+    const int j = blockIdx.x, rl = threadIdx.x & 7, r = blockIdx.y * 8 + rl;
+    double2 s = make_double2(0, 0);
+    if (r < R) {
+        const double2* p = partial + (size_t)j * nblk * R + r;
+#pragma unroll 8
+        for (int b = threadIdx.x >> 3; b < nblk; b += 32) s = cadd(s, p[(size_t)b * R]);
     }
+#pragma unroll
+    for (int d = 8; d < 64; d <<= 1) {
+        s.x += __shfl_xor(s.x, d);
+        s.y += __shfl_xor(s.y, d);
+    }
+    if ((threadIdx.x & 63) < 8) red[threadIdx.x >> 6][rl] = s;
+    __syncthreads();
+    if (threadIdx.x < 8 && r < R)
+        out[(size_t)j * R + r] = cadd(cadd(red[0][rl], red[1][rl]), cadd(red[2][rl], red[3][rl]));
 }
 
 void launch_reduce_partials_b(hipStream_t st, int m, int R, int nblk, const double2* partial, double2* out) {
-    k_reduce_partials_b<<<m, 256, 0, st>>>(nblk, R, partial, out);
+    k_reduce_partials_b<<<dim3(m, (R + 7) / 8), 256, 0, st>>>(nblk, R, partial, out);
 }
 
 // partial[b * R + r] = sum over block b of |x[u][r]|^2
