@@ -461,7 +461,6 @@ void Engine::build_near() {
     nd_.items = upload(items);
     nd_.planes = planes;
     nd_.nleaf = nleaf;
-    nd_.npairs = (int)pair_src.size();
     nd_.N = N;
     nd_.leaf_ptr = d_leaf_ptr_;
     nd_.perm = d_perm_;
@@ -470,9 +469,6 @@ void Engine::build_near() {
     nd_.tgt_cols = upload(tgt_cols);
     nd_.col_ptr = upload(col_ptr);
     nd_.colref = upload(colref);
-    nd_.pair_tgt = upload(pair_tgt);
-    nd_.pair_src = upload(pair_src);
-    nd_.pair_col = upload(pair_col);
     d_Z_ = dalloc<double2>((size_t)near_entries);
     NearConsts c;
     c.k1 = d2(med.k1);
@@ -481,8 +477,7 @@ void Engine::build_near() {
     c.etai = d2(med.etai);
     c.inv_etai = d2(1.0 / med.etai);
     c.alpha = P.cfie_alpha;
-    launch_near_fill(st, ie, nd_, d_geo_, gauss_, c, d_Z_);
-    MLFMA_HIP(hipGetLastError());
+    fill_near(planes, c);
     if (P.near_precision != MLFMA_FP64) {   // FP32 storage (also the single-vector products of MLFMA_BF16)
         d_Z32_ = dalloc<float2>((size_t)near_entries);
         launch_narrow(st, (size_t)near_entries, d_Z_, d_Z32_);
@@ -511,6 +506,130 @@ void Engine::build_near() {
         launch_narrow(st, nunk, d_dinv_, d_dinvf_);
     }
     MLFMA_HIP(hipGetLastError());
+}
+
+// The near field's entries, in batches of leaf-pair blocks whose face-pair
+// integrals fit the scratch array (256 MB: it stays in the last-level cache
+// between the two kernels; a block of two full groups takes at most 113 MB).
+void Engine::fill_near(int planes, const NearConsts& c) {
+    constexpr int kFillRows = 256;
+    const std::vector<int>& lp = tree.leaf_ptr;
+    // groups of at most kFillRows RWG, and the faces of each in order of appearance
+    std::vector<int> leaf_group(nleaf + 1, 0), row_ptr(1, 0), face_ptr(1, 0), face_idx;
+    std::vector<int2> side(N);
+    std::vector<double> len(N);
+    std::vector<int> stamp(mesh.face_id.size(), -1), local(mesh.face_id.size(), 0);
+    for (int t = 0; t < nleaf; ++t) {
+        const int nt = lp[t + 1] - lp[t], ng = std::max(1, (nt + kFillRows - 1) / kFillRows);
+        for (int k = 0; k < ng; ++k) {
+            const int g = (int)row_ptr.size() - 1;
+            const int i0 = lp[t] + (int)((long long)nt * k / ng), i1 = lp[t] + (int)((long long)nt * (k + 1) / ng);
+            auto ref = [&](int f, int free) {
+                if (stamp[f] != g) {
+                    stamp[f] = g;
+                    local[f] = (int)face_idx.size() - face_ptr[g];
+                    face_idx.push_back(f);
+                }
+                int v = 0;
+                while (v < 2 && mesh.tri[3 * f + v] != free) ++v;
+                return local[f] * 4 + v;
+            };
+            for (int i = i0; i < i1; ++i) {
+                const int r = tree.perm[i];
+                const int neg = ref(basis.fneg[r], basis.vneg[r]);
+                side[i] = make_int2(neg, ref(basis.fpos[r], basis.vpos[r]));
+                len[i] = basis.len[r];
+            }
+            row_ptr.push_back(i1);
+            face_ptr.push_back((int)face_idx.size());
+        }
+        leaf_group[t + 1] = (int)row_ptr.size() - 1;
+    }
+    std::vector<FaceGeo> faces(mesh.face_id.size());
+    for (size_t f = 0; f < faces.size(); ++f) {
+        for (int v = 0; v < 3; ++v) {
+            const Vec3& p = mesh.pts[mesh.tri[3 * f + v]];
+            faces[f].tri[3 * v] = p.x, faces[f].tri[3 * v + 1] = p.y, faces[f].tri[3 * v + 2] = p.z;
+        }
+        faces[f].nrm[0] = mesh.normal[f].x, faces[f].nrm[1] = mesh.normal[f].y, faces[f].nrm[2] = mesh.normal[f].z;
+        faces[f].area = mesh.area[f];
+        faces[f].id = mesh.face_id[f];
+    }
+    // faces with one id count as identical: the same small number for each id
+    std::vector<int> ids(mesh.face_id), key(faces.size());
+    std::sort(ids.begin(), ids.end());
+    for (size_t f = 0; f < faces.size(); ++f)
+        key[f] = (int)(std::lower_bound(ids.begin(), ids.end(), mesh.face_id[f]) - ids.begin());
+    // blocks, and per batch their face-pair, identical-face and entry items
+    const size_t per = (size_t)9 * planes * sizeof(double2);
+    const long long cap = (256ll << 20) / (long long)per;
+    struct Batch {
+        size_t pair0, same0, entry0;
+    };
+    std::vector<FillBlock> blocks;
+    std::vector<int2> pairs, same, entries;
+    std::vector<Batch> batches;
+    std::vector<int> head(faces.size(), -1), next(faces.size(), -1);
+    long long slots = cap + 1, most = 0;
+    for (size_t p = 0; p < pair_tgt.size(); ++p) {
+        const int t = pair_tgt[p], s = pair_src[p], nt = lp[t + 1] - lp[t];
+        for (int gs = leaf_group[s]; gs < leaf_group[s + 1]; ++gs) {
+            const int s0 = face_ptr[gs], nS = face_ptr[gs + 1] - s0;
+            for (int k = nS - 1; k >= 0; --k) {   // source faces by id
+                next[k] = head[key[face_idx[s0 + k]]];
+                head[key[face_idx[s0 + k]]] = k;
+            }
+            for (int gt = leaf_group[t]; gt < leaf_group[t + 1]; ++gt) {
+                const int f0 = face_ptr[gt], nF = face_ptr[gt + 1] - f0;
+                const long long cnt = (long long)nF * nS;
+                if (slots + cnt > cap) {
+                    batches.push_back({pairs.size(), same.size(), entries.size()});
+                    slots = 0;
+                }
+                const int b = (int)blocks.size();
+                FillBlock B;
+                B.gt = gt, B.gs = gs, B.ld = nt;
+                B.plane = (long long)tgt_cols[t] * nt;
+                B.out = tgt_off[t] + (long long)(pair_col[p] + row_ptr[gs] - lp[s]) * nt + row_ptr[gt] - lp[t];
+                B.slot0 = slots;
+                blocks.push_back(B);
+                slots += cnt;
+                most = std::max(most, slots);
+                for (int k = 0; k < (cnt + 63) / 64; ++k) pairs.push_back(make_int2(b, k));
+                for (int k = 0; k < nF; ++k)
+                    for (int q = head[key[face_idx[f0 + k]]]; q >= 0; q = next[q])
+                        same.push_back(make_int2(b, q * nF + k));
+                const long long ne = (long long)(row_ptr[gt + 1] - row_ptr[gt]) * (row_ptr[gs + 1] - row_ptr[gs]);
+                for (int k = 0; k < (ne + 255) / 256; ++k) entries.push_back(make_int2(b, k));
+            }
+            for (int k = 0; k < nS; ++k) head[key[face_idx[s0 + k]]] = -1;
+        }
+    }
+    batches.push_back({pairs.size(), same.size(), entries.size()});
+    NearFill nf;
+    nf.faces = upload(faces);
+    nf.face_ptr = upload(face_ptr);
+    nf.face_idx = upload(face_idx);
+    nf.row_ptr = upload(row_ptr);
+    nf.side = upload(side);
+    nf.len = upload(len);
+    nf.blocks = upload(blocks);
+    int2* d_pairs = upload(pairs);
+    int2* d_same = upload(same);
+    int2* d_entries = upload(entries);
+    double2* scr = dalloc<double2>((size_t)9 * planes * std::max(most, 1ll));
+    for (size_t b = 0; b + 1 < batches.size(); ++b) {
+        const Batch &u = batches[b], &v = batches[b + 1];
+        launch_near_fill(st, ie, nf, d_pairs + u.pair0, (int)(v.pair0 - u.pair0), d_same + u.same0,
+                         (int)(v.same0 - u.same0), d_entries + u.entry0, (int)(v.entry0 - u.entry0), gauss_, c,
+                         (size_t)most, scr, d_Z_);
+        MLFMA_HIP(hipGetLastError());
+    }
+    MLFMA_HIP(hipStreamSynchronize(st));
+    for (const void* q : {(const void*)nf.faces, (const void*)nf.face_ptr, (const void*)nf.face_idx,
+                          (const void*)nf.row_ptr, (const void*)nf.side, (const void*)nf.len, (const void*)nf.blocks,
+                          (const void*)d_pairs, (const void*)d_same, (const void*)d_entries, (const void*)scr})
+        dfree(const_cast<void*>(q));
 }
 
 // Items of the single-vector near product when the leaves alone do not fill

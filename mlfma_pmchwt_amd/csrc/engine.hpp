@@ -239,6 +239,7 @@ private:
     void build_wave(int w);
     void build_near();
     void build_near_split(int planes);
+    void fill_near(int planes, const struct NearConsts& c);
     template <typename R>
     FarDev<R>& far(int w);
     template <typename R>

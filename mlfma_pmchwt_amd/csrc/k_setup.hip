@@ -110,203 +110,328 @@ __device__ void sing_point(R3 r, const double* t, const SingFrame& f, bool want3
     }
 }
 
-// Galerkin entries between field RWG F and source RWG S.
+// Galerkin integrals between one half of field RWG F and one half of source RWG
+// S on the same face (identical-face singular extraction), free vertices vF, vS:
 //   L(k):  Code/Operator.h:709-881     (EFIE = eta * L, Code/EFIE.cpp:6-194)
 //   K(k):  Code/Operator.h:883-1046
 //   M(k):  MFIE, Code/MFIE.cpp:6-212
+// without the factor len_F len_S / (4 pi) and the halves' signs.
 template <int NK, bool WL, bool WK, bool WM>
-__device__ void pair_ops(const RwgGeo& F, const RwgGeo& S, const GaussRule& g, const double2* ks, double2* Lo,
-                         double2* Ko, double2* Mo) {
-    for (int q = 0; q < NK; ++q) Lo[q] = Ko[q] = make_double2(0, 0);
-    *Mo = make_double2(0, 0);
-    for (int i = 0; i < 2; ++i) {
-        const double* tF = F.tri[i];
-        const R3 vF = mk(F.vf[i]);
-        const R3 nF = mk(F.nrm[i]);
-        const double AF = F.area[i], recAf = 1.0 / (2.0 * AF);
-        for (int j = 0; j < 2; ++j) {
-            const double* tS = S.tri[j];
-            const R3 vS = mk(S.vf[j]);
-            const double AS = S.area[j], recAs = 1.0 / (2.0 * AS);
-            const bool same = (F.face[i] == S.face[j]);
-            double2 aL[NK], aK[NK], aM = make_double2(0, 0);
-            for (int q = 0; q < NK; ++q) aL[q] = aK[q] = make_double2(0, 0);
-            for (int a = 0; a < g.n; ++a) {
-                const R3 rf = gpt(g, a, tF);
-                const R3 pf = sub3(rf, vF);
-                const double wF = g.w[a];
-                for (int b = 0; b < g.n; ++b) {
-                    const R3 rs = gpt(g, b, tS);
-                    const R3 ps = sub3(rs, vS);
-                    const R3 Rv = sub3(rf, rs);
-                    const double R = nrm3(Rv);
-                    const double w = wF * g.w[b];
-                    const double dL = WL ? dot3(pf, ps) : 0.0;
-                    const double dK = (WK || (WM && !same)) ? dot3(pf, crs3(Rv, ps)) : 0.0;
-                    double dM = 0.0;
-                    if (WM) dM = same ? dot3(crs3(sub3(rf, vS), ps), crs3(pf, nF)) : dot3(pf, crs3(nF, crs3(Rv, ps)));
+__device__ void same_face_ops(const FaceGeo& F, R3 vF, const FaceGeo& S, R3 vS, const GaussRule& g, const double2* ks,
+                              double2* aL, double2* aK, double2* aM) {
+    const R3 nF = mk(F.nrm);
+    const double AF = F.area, recAf = 1.0 / (2.0 * AF), AS = S.area, recAs = 1.0 / (2.0 * AS);
+    *aM = make_double2(0, 0);
+    for (int q = 0; q < NK; ++q) aL[q] = aK[q] = make_double2(0, 0);
+    for (int a = 0; a < g.n; ++a) {
+        const R3 rf = gpt(g, a, F.tri);
+        const R3 pf = sub3(rf, vF);
+        for (int b = 0; b < g.n; ++b) {
+            const R3 rs = gpt(g, b, S.tri);
+            const R3 ps = sub3(rs, vS);
+            const R3 Rv = sub3(rf, rs);
+            const double R = nrm3(Rv);
+            const double w = g.w[a] * g.w[b];
+            const double dL = WL ? dot3(pf, ps) : 0.0;
+            const double dK = WK ? dot3(pf, crs3(Rv, ps)) : 0.0;
+            const double dM = WM ? dot3(crs3(sub3(rf, vS), ps), crs3(pf, nF)) : 0.0;
 #pragma unroll
-                    for (int q = 0; q < NK; ++q) {
-                        const double2 k = ks[q];
-                        const double2 jk = make_double2(-k.y, k.x);
-                        double2 G, G3;
-                        if (!same) {
-                            const double2 e = expmjk(k, R);
-                            G = cscale(e, 1.0 / R);
-                            // e / R^3 * (1 + j k R)
-                            G3 = cscale(cmul(e, make_double2(1.0 - k.y * R, k.x * R)), 1.0 / (R * R * R));
-                        } else if (R < kEps0D) {
-                            G = make_double2(k.y, -k.x);   // -j k
-                            G3 = make_double2(0, 0);
-                        } else {
-                            const double2 e = expmjk(k, R);
-                            G = make_double2(e.x / R - 1.0 / R, e.y / R);
-                            G3 = cscale(cmul(e, make_double2(1.0 - k.y * R, k.x * R)), 1.0 / (R * R * R));
-                            const double2 k2 = cmul(k, k);
-                            G3.x -= 1.0 / (R * R * R) + 0.5 * k2.x / R;
-                            G3.y -= 0.5 * k2.y / R;
-                        }
-                        if (WL) {
-                            // jk w (G pf.ps - 4 G / k^2)
-                            const double2 c4 = cdiv(make_double2(4.0, 0.0), cmul(k, k));
-                            const double2 t = csub(cscale(G, dL), cmul(G, c4));
-                            cfma(aL[q], cscale(jk, w), t);
-                        }
-                        if (WK) cfma(aK[q], make_double2(w, 0.0), cscale(G3, dK));
-                        if (WM && q == 0) cfma(aM, make_double2(w, 0.0), cscale(G3, dM));
-                    }
-                }
-            }
-            if (same) {
-                SingFrame fr;
-                sing_frame(tS, S.nrm[j], fr);
-                const R3 nS = fr.n;
-                const R3 rho0N = sub3(vS, scl3(nS, dot3(nS, vS)));
-                for (int a = 0; a < g.n; ++a) {
-                    const R3 rf = gpt(g, a, tF);
-                    const double wF = g.w[a];
-                    SingPt sp;
-                    sing_point(rf, tS, fr, WK || WM, sp);
-                    const R3 RWGf = scl3(sub3(rf, vF), recAf);
-                    const R3 pv1 = sub3(sp.rho, rho0N);
-                    const R3 Ri = sub3(rf, vS);
-                    if (WM) {   // identity term, Code/MFIE.cpp:175-192
-                        const R3 RWGs = scl3(Ri, recAs);
-                        aM.x += 4.0 * kPiD * wF * AF * dot3(RWGf, RWGs);
-                    }
-#pragma unroll
-                    for (int q = 0; q < NK; ++q) {
-                        const double2 k = ks[q];
-                        const double2 jk = make_double2(-k.y, k.x);
-                        const double2 k2 = cmul(k, k);
-                        if (WL) {
-                            const R3 Ikon = scl3(add3(sp.Iv, scl3(pv1, sp.Is)), recAs);
-                            const double2 t =
-                                csub(make_double2(dot3(RWGf, Ikon), 0.0),
-                                     cscale(cdiv(make_double2(1.0, 0.0), k2), sp.Is / (AF * AS)));
-                            cfma(aL[q], cscale(jk, wF * 2.0 * AF), t);
-                        }
-                        if (WK || (WM && q == 0)) {
-                            // Ikon = (k^2/2)(Iv + pv1 Is)/(2As) + (Iv3 + pv1 Is3)/(2As)
-                            const double2 h = cscale(k2, 0.5);
-                            const R3 a1 = add3(sp.Iv, scl3(pv1, sp.Is));
-                            const R3 a3 = add3(sp.Iv3, scl3(pv1, sp.Is3));
-                            const double2 I0 = make_double2(h.x * a1.x * recAs + a3.x * recAs, h.y * a1.x * recAs);
-                            const double2 I1 = make_double2(h.x * a1.y * recAs + a3.y * recAs, h.y * a1.y * recAs);
-                            const double2 I2 = make_double2(h.x * a1.z * recAs + a3.z * recAs, h.y * a1.z * recAs);
-                            // Ri x Ikon
-                            const double2 X0 = csub(cscale(I2, Ri.y), cscale(I1, Ri.z));
-                            const double2 X1 = csub(cscale(I0, Ri.z), cscale(I2, Ri.x));
-                            const double2 X2 = csub(cscale(I1, Ri.x), cscale(I0, Ri.y));
-                            if (WK) {
-                                double2 d = cadd(cadd(cscale(X0, RWGf.x), cscale(X1, RWGf.y)), cscale(X2, RWGf.z));
-                                aK[q] = cadd(aK[q], cscale(d, wF * 2.0 * AF));
-                            }
-                            if (WM && q == 0) {
-                                const R3 c2 = crs3(RWGf, nF);
-                                double2 d = cadd(cadd(cscale(X0, c2.x), cscale(X1, c2.y)), cscale(X2, c2.z));
-                                aM = cadd(aM, cscale(d, wF * 2.0 * AF));
-                            }
-                        }
-                    }
-                }
-            }
-            const double sg = ((i == 0) ? -1.0 : 1.0) * ((j == 0) ? -1.0 : 1.0);
-            const double sc = (F.len * S.len) / (4.0 * kPiD) * sg;
             for (int q = 0; q < NK; ++q) {
-                if (WL) Lo[q] = cadd(Lo[q], cscale(aL[q], sc));
-                if (WK) Ko[q] = cadd(Ko[q], cscale(aK[q], sc));
+                const double2 k = ks[q];
+                const double2 jk = make_double2(-k.y, k.x);
+                double2 G, G3;
+                if (R < kEps0D) {
+                    G = make_double2(k.y, -k.x);   // -j k
+                    G3 = make_double2(0, 0);
+                } else {
+                    const double2 e = expmjk(k, R);
+                    G = make_double2(e.x / R - 1.0 / R, e.y / R);
+                    G3 = cscale(cmul(e, make_double2(1.0 - k.y * R, k.x * R)), 1.0 / (R * R * R));
+                    const double2 k2 = cmul(k, k);
+                    G3.x -= 1.0 / (R * R * R) + 0.5 * k2.x / R;
+                    G3.y -= 0.5 * k2.y / R;
+                }
+                if (WL) {
+                    // jk w (G pf.ps - 4 G / k^2)
+                    const double2 c4 = cdiv(make_double2(4.0, 0.0), cmul(k, k));
+                    cfma(aL[q], cscale(jk, w), csub(cscale(G, dL), cmul(G, c4)));
+                }
+                if (WK) cfma(aK[q], make_double2(w, 0.0), cscale(G3, dK));
+                if (WM && q == 0) cfma(*aM, make_double2(w, 0.0), cscale(G3, dM));
             }
-            if (WM) *Mo = cadd(*Mo, cscale(aM, sc));
         }
     }
+    SingFrame fr;
+    sing_frame(S.tri, S.nrm, fr);
+    const R3 rho0N = sub3(vS, scl3(fr.n, dot3(fr.n, vS)));
+    for (int a = 0; a < g.n; ++a) {
+        const R3 rf = gpt(g, a, F.tri);
+        const double wF = g.w[a];
+        SingPt sp;
+        sing_point(rf, S.tri, fr, WK || WM, sp);
+        const R3 RWGf = scl3(sub3(rf, vF), recAf);
+        const R3 pv1 = sub3(sp.rho, rho0N);
+        const R3 Ri = sub3(rf, vS);
+        if (WM) {   // identity term, Code/MFIE.cpp:175-192
+            const R3 RWGs = scl3(Ri, recAs);
+            aM->x += 4.0 * kPiD * wF * AF * dot3(RWGf, RWGs);
+        }
+#pragma unroll
+        for (int q = 0; q < NK; ++q) {
+            const double2 k = ks[q];
+            const double2 jk = make_double2(-k.y, k.x);
+            const double2 k2 = cmul(k, k);
+            if (WL) {
+                const R3 Ikon = scl3(add3(sp.Iv, scl3(pv1, sp.Is)), recAs);
+                const double2 t = csub(make_double2(dot3(RWGf, Ikon), 0.0),
+                                       cscale(cdiv(make_double2(1.0, 0.0), k2), sp.Is / (AF * AS)));
+                cfma(aL[q], cscale(jk, wF * 2.0 * AF), t);
+            }
+            if (WK || (WM && q == 0)) {
+                // Ikon = (k^2/2)(Iv + pv1 Is)/(2As) + (Iv3 + pv1 Is3)/(2As)
+                const double2 h = cscale(k2, 0.5);
+                const R3 a1 = add3(sp.Iv, scl3(pv1, sp.Is));
+                const R3 a3 = add3(sp.Iv3, scl3(pv1, sp.Is3));
+                const double2 I0 = make_double2(h.x * a1.x * recAs + a3.x * recAs, h.y * a1.x * recAs);
+                const double2 I1 = make_double2(h.x * a1.y * recAs + a3.y * recAs, h.y * a1.y * recAs);
+                const double2 I2 = make_double2(h.x * a1.z * recAs + a3.z * recAs, h.y * a1.z * recAs);
+                // Ri x Ikon
+                const double2 X0 = csub(cscale(I2, Ri.y), cscale(I1, Ri.z));
+                const double2 X1 = csub(cscale(I0, Ri.z), cscale(I2, Ri.x));
+                const double2 X2 = csub(cscale(I1, Ri.x), cscale(I0, Ri.y));
+                if (WK) {
+                    double2 d = cadd(cadd(cscale(X0, RWGf.x), cscale(X1, RWGf.y)), cscale(X2, RWGf.z));
+                    aK[q] = cadd(aK[q], cscale(d, wF * 2.0 * AF));
+                }
+                if (WM && q == 0) {
+                    const R3 c2 = crs3(RWGf, nF);
+                    double2 d = cadd(cadd(cscale(X0, c2.x), cscale(X1, c2.y)), cscale(X2, c2.z));
+                    *aM = cadd(*aM, cscale(d, wF * 2.0 * AF));
+                }
+            }
+        }
+    }
+}
+
+// complex 3-vectors of the face-pair sums
+struct C3 {
+    double2 x, y, z;
+};
+__device__ __forceinline__ void acc3(C3& s, double2 g, R3 p) {
+    s.x.x = fma(g.x, p.x, s.x.x), s.x.y = fma(g.y, p.x, s.x.y);
+    s.y.x = fma(g.x, p.y, s.y.x), s.y.y = fma(g.y, p.y, s.y.y);
+    s.z.x = fma(g.x, p.z, s.z.x), s.z.y = fma(g.y, p.z, s.z.y);
+}
+__device__ __forceinline__ double2 dotc(R3 p, const C3& s) {
+    return make_double2(fma(p.z, s.z.x, fma(p.y, s.y.x, p.x * s.x.x)), fma(p.z, s.z.y, fma(p.y, s.y.y, p.x * s.x.y)));
+}
+__device__ __forceinline__ C3 crossc(R3 p, const C3& s) {
+    C3 o;
+    o.x = make_double2(p.y * s.z.x - p.z * s.y.x, p.y * s.z.y - p.z * s.y.y);
+    o.y = make_double2(p.z * s.x.x - p.x * s.z.x, p.z * s.x.y - p.x * s.z.y);
+    o.z = make_double2(p.x * s.y.x - p.y * s.x.x, p.x * s.y.y - p.y * s.x.y);
+    return o;
 }
 
 }  // namespace
 
 // ---------------------------------------------------------------- near field
-// One workgroup per (target leaf, source leaf) block, written into its
-// columns of the target's block row (layout of NearDev, geo.hpp).
-// Code/Zmartix.h:188-278 (EFIE), :372-465 (CFIE), :541-643 (PMCHWT).
+// Code/Zmartix.h:188-278 (EFIE), :372-465 (CFIE), :541-643 (PMCHWT).  An entry
+// is the signed sum over the two halves of each RWG, and every (face, free
+// vertex) pair is a half of one RWG only, so a pair of faces with its 49
+// kernel evaluations (sincos, 1/R; exp in a lossy medium) serves 9 entries'
+// halves: evaluating per entry repeated it up to nine times.  9,720 PMCHWT RWG
+// in 40 leaves: 113 ms per entry, 11 ms by face pairs; 151,230 RWG: 1.4 and
+// 0.2 s; 300,000 RWG CFIE: 1.2 and 0.14 s; 48,000 RWG in leaves of up to 18
+// (faces shared least): 50 and 8 ms.  k_face_pairs takes one pair of faces per thread and leaves
+// the integrals for the 3 x 3 free-vertex pairs in a bounded scratch array,
+// k_face_same those of identical faces (singular extraction), and
+// k_near_assemble sums each entry's four in a fixed order.
+//
+// The sums over the source points need the kernels only against 1 and r' - v_0:
+// with T_n = sum G (r' - v_n), L wants (r - v_m).T_n, and since
+// (r - r') x (r' - v_n) = (r - v_n) x (r' - v_n), K and the MFIE want
+// (r - v_n) x T_n of the gradient kernel.
 template <int MODE>
-__global__ __launch_bounds__(256) void k_near_fill(NearDev nd, const RwgGeo* __restrict__ geo, GaussRule g,
-                                                   NearConsts c, double2* __restrict__ Z) {
-    const int p = blockIdx.x;
-    const int t = nd.pair_tgt[p], s = nd.pair_src[p];
-    const int i0 = nd.leaf_ptr[t], nt = nd.leaf_ptr[t + 1] - i0;
-    const int j0 = nd.leaf_ptr[s], ns = nd.leaf_ptr[s + 1] - j0;
-    const size_t plane = (size_t)nd.tgt_cols[t] * nt;
-    double2* out = Z + nd.tgt_off[t] + (size_t)nd.pair_col[p] * nt;
-    for (int e = threadIdx.x; e < nt * ns; e += blockDim.x) {
-        const int row = e % nt, col = e / nt;
-        const RwgGeo& F = geo[i0 + row];
-        const RwgGeo& S = geo[j0 + col];
-        if (MODE == 2) {
-            double2 L[2], K[2], M;
-            const double2 ks[2] = {c.k1, c.k2};
-            pair_ops<2, true, true, false>(F, S, g, ks, L, K, &M);
-            const double2 z11 = cadd(L[0], cmul(c.etai, L[1]));
-            const double2 zk = cadd(K[0], K[1]);
-            const double2 z22 = cadd(L[0], cmul(c.inv_etai, L[1]));
-            out[(size_t)col * nt + row] = z11;
-            out[plane + (size_t)col * nt + row] = zk;
-            out[2 * plane + (size_t)col * nt + row] = z22;
-        } else if (MODE == 0) {
-            double2 L, K, M;
-            pair_ops<1, true, false, false>(F, S, g, &c.k1, &L, &K, &M);
-            out[(size_t)col * nt + row] = cmul(c.eta1, L);
-        } else {
-            double2 L, K, M;
-            pair_ops<1, true, false, true>(F, S, g, &c.k1, &L, &K, &M);
-            // alpha E + (1 - alpha) eta M, E = eta L  (Code/Zmartix.h:432)
-            const double2 E = cmul(c.eta1, L);
-            out[(size_t)col * nt + row] = cadd(cscale(E, c.alpha), cscale(cmul(c.eta1, M), 1.0 - c.alpha));
+__global__ __launch_bounds__(64) void k_face_pairs(NearFill nf, const int2* __restrict__ items, GaussRule g,
+                                                   NearConsts c, size_t cap, double2* __restrict__ scr) {
+    constexpr int PL = MODE == 2 ? 3 : 1;
+    const int2 it = items[blockIdx.x];
+    const FillBlock& B = nf.blocks[it.x];
+    const int f0 = nf.face_ptr[B.gt], nF = nf.face_ptr[B.gt + 1] - f0;
+    const int s0 = nf.face_ptr[B.gs], nS = nf.face_ptr[B.gs + 1] - s0;
+    const int e = it.y * 64 + threadIdx.x;
+    if (e >= nF * nS) return;
+    const int sl = e / nF, fl = e - sl * nF;
+    const FaceGeo& F = nf.faces[nf.face_idx[f0 + fl]];
+    const FaceGeo& S = nf.faces[nf.face_idx[s0 + sl]];
+    if (F.id == S.id) return;   // k_face_same
+    double tS[9], tF[9];
+    for (int v = 0; v < 9; ++v) tS[v] = S.tri[v], tF[v] = F.tri[v];
+    const R3 vS0 = mk(tS);
+    double2 D1[3][3], D2[3][3], DK[3][3];   // [field vertex][source vertex]
+    for (int m = 0; m < 3; ++m)
+        for (int n = 0; n < 3; ++n) D1[m][n] = D2[m][n] = DK[m][n] = make_double2(0, 0);
+    double2 E1 = {0, 0}, E2 = {0, 0};
+    const R3 nrm = mk(F.nrm);
+    for (int a = 0; a < g.n; ++a) {
+        const R3 rf = gpt(g, a, tF);
+        const double wF = g.w[a];
+        double2 g1 = {0, 0}, g2 = {0, 0}, h = {0, 0};
+        C3 G1 = {{0, 0}, {0, 0}, {0, 0}}, G2 = G1, H = G1;
+        for (int b = 0; b < g.n; ++b) {
+            const R3 rs = gpt(g, b, tS);
+            const R3 ps = sub3(rs, vS0);
+            const double R2 = dot3(sub3(rf, rs), sub3(rf, rs));
+            const double R = sqrt(R2), ri = 1.0 / R;
+            const double w = g.w[b];
+            const double wi = w * ri, wi3 = wi * (ri * ri);
+            const double2 e1 = expmjk(c.k1, R);
+            const double2 u1 = cscale(e1, wi);
+            g1 = cadd(g1, u1);
+            acc3(G1, u1, ps);
+            if (MODE >= 1) {   // gradient kernel e (1 + j k R) / R^3, both media of PMCHWT together
+                double2 q = cmul(e1, make_double2(1.0 - c.k1.y * R, c.k1.x * R));
+                if (MODE == 2) {
+                    const double2 e2 = expmjk(c.k2, R);
+                    const double2 u2 = cscale(e2, wi);
+                    g2 = cadd(g2, u2);
+                    acc3(G2, u2, ps);
+                    q = cadd(q, cmul(e2, make_double2(1.0 - c.k2.y * R, c.k2.x * R)));
+                }
+                q = cscale(q, wi3);
+                h = cadd(h, q);
+                acc3(H, q, ps);
+            }
         }
+        E1 = cadd(E1, cscale(g1, wF));
+        if (MODE == 2) E2 = cadd(E2, cscale(g2, wF));
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            const R3 vn = mk(tS + 3 * n), d = sub3(vS0, vn);
+            C3 T1 = G1, T2 = G2, TH = H;
+            acc3(T1, g1, d);
+            if (MODE == 2) acc3(T2, g2, d);
+            if (MODE >= 1) {
+                acc3(TH, h, d);
+                TH = crossc(sub3(rf, vn), TH);
+            }
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                const R3 pf = scl3(sub3(rf, mk(tF + 3 * m)), wF);
+                D1[m][n] = cadd(D1[m][n], dotc(pf, T1));
+                if (MODE == 2) D2[m][n] = cadd(D2[m][n], dotc(pf, T2));
+                if (MODE == 2) DK[m][n] = cadd(DK[m][n], dotc(pf, TH));
+                if (MODE == 1) DK[m][n] = cadd(DK[m][n], dotc(crs3(pf, nrm), TH));
+            }
+        }
+    }
+    // L = jk (sum G pf.ps - 4 / k^2 sum G)
+    const double2 four = make_double2(4.0, 0.0);
+    const double2 jk1 = make_double2(-c.k1.y, c.k1.x), jk2 = make_double2(-c.k2.y, c.k2.x);
+    E1 = cmul(E1, cdiv(four, cmul(c.k1, c.k1)));
+    if (MODE == 2) E2 = cmul(E2, cdiv(four, cmul(c.k2, c.k2)));
+    double2* o = scr + B.slot0 + e;
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            double2* q = o + (size_t)(m * 3 + n) * PL * cap;
+            const double2 L1 = cmul(jk1, csub(D1[m][n], E1));
+            if (MODE == 2) {
+                const double2 L2 = cmul(jk2, csub(D2[m][n], E2));
+                q[0] = cadd(L1, cmul(c.etai, L2));
+                q[cap] = DK[m][n];
+                q[2 * cap] = cadd(L1, cmul(c.inv_etai, L2));
+            } else if (MODE == 0) {
+                q[0] = cmul(c.eta1, L1);
+            } else {   // alpha E + (1 - alpha) eta M, E = eta L  (Code/Zmartix.h:432)
+                q[0] = cadd(cscale(cmul(c.eta1, L1), c.alpha), cscale(cmul(c.eta1, DK[m][n]), 1.0 - c.alpha));
+            }
+        }
+}
+
+// Identical faces: one thread per (listed pair, free-vertex pair).
+template <int MODE>
+__global__ __launch_bounds__(64) void k_face_same(NearFill nf, int count, const int2* __restrict__ same, GaussRule g,
+                                                  NearConsts c, size_t cap, double2* __restrict__ scr) {
+    constexpr int PL = MODE == 2 ? 3 : 1;
+    const int idx = blockIdx.x * 64 + threadIdx.x;
+    if (idx >= count * 9) return;
+    const int p = idx / 9, m = (idx - p * 9) / 3, n = idx - p * 9 - m * 3;
+    const FillBlock& B = nf.blocks[same[p].x];
+    const int e = same[p].y;
+    const int f0 = nf.face_ptr[B.gt], nF = nf.face_ptr[B.gt + 1] - f0, s0 = nf.face_ptr[B.gs];
+    const int sl = e / nF, fl = e - sl * nF;
+    const FaceGeo& F = nf.faces[nf.face_idx[f0 + fl]];
+    const FaceGeo& S = nf.faces[nf.face_idx[s0 + sl]];
+    const R3 vF = mk(F.tri + 3 * m), vS = mk(S.tri + 3 * n);
+    double2* q = scr + (size_t)(m * 3 + n) * PL * cap + B.slot0 + e;
+    double2 L[2], K[2], M;
+    if (MODE == 2) {
+        const double2 ks[2] = {c.k1, c.k2};
+        same_face_ops<2, true, true, false>(F, vF, S, vS, g, ks, L, K, &M);
+        q[0] = cadd(L[0], cmul(c.etai, L[1]));
+        q[cap] = cadd(K[0], K[1]);
+        q[2 * cap] = cadd(L[0], cmul(c.inv_etai, L[1]));
+    } else if (MODE == 0) {
+        same_face_ops<1, true, false, false>(F, vF, S, vS, g, &c.k1, L, K, &M);
+        q[0] = cmul(c.eta1, L[0]);
+    } else {
+        same_face_ops<1, true, false, true>(F, vF, S, vS, g, &c.k1, L, K, &M);
+        q[0] = cadd(cscale(cmul(c.eta1, L[0]), c.alpha), cscale(cmul(c.eta1, M), 1.0 - c.alpha));
     }
 }
 
-void launch_near_fill(hipStream_t st, int mode, const NearDev& nd, const RwgGeo* geo, const GaussRule& g,
-                      const NearConsts& c, double2* Z) {
-    if (nd.npairs == 0) return;
-    if (mode == 2) k_near_fill<2><<<nd.npairs, 256, 0, st>>>(nd, geo, g, c, Z);
-    else if (mode == 1) k_near_fill<1><<<nd.npairs, 256, 0, st>>>(nd, geo, g, c, Z);
-    else k_near_fill<0><<<nd.npairs, 256, 0, st>>>(nd, geo, g, c, Z);
+// Entries of the blocks: rows of the target group x columns of the source
+// group, 256 per workgroup, rows fastest (layout of NearDev, geo.hpp).
+template <int PL>
+__global__ __launch_bounds__(256) void k_near_assemble(NearFill nf, const int2* __restrict__ items, size_t cap,
+                                                       const double2* __restrict__ scr, double2* __restrict__ Z) {
+    const int2 it = items[blockIdx.x];
+    const FillBlock& B = nf.blocks[it.x];
+    const int i0 = nf.row_ptr[B.gt], nr = nf.row_ptr[B.gt + 1] - i0;
+    const int j0 = nf.row_ptr[B.gs], nc = nf.row_ptr[B.gs + 1] - j0;
+    const int e = it.y * 256 + threadIdx.x;
+    if (e >= nr * nc) return;
+    const int col = e / nr, row = e - col * nr;
+    const int nF = nf.face_ptr[B.gt + 1] - nf.face_ptr[B.gt];
+    const int2 sf = nf.side[i0 + row], ss = nf.side[j0 + col];   // face * 4 + free vertex of the - and + halves
+    const double sc = nf.len[i0 + row] * nf.len[j0 + col] / (4.0 * kPiD);
+    double2 z[PL];
+    for (int p = 0; p < PL; ++p) z[p] = make_double2(0, 0);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int f = a == 0 ? sf.x : sf.y, s = b == 0 ? ss.x : ss.y;
+            const double2* v = scr + (size_t)((f & 3) * 3 + (s & 3)) * PL * cap + B.slot0 + (s >> 2) * nF + (f >> 2);
+            const double w = a == b ? sc : -sc;
+#pragma unroll
+            for (int p = 0; p < PL; ++p) z[p] = cadd(z[p], cscale(v[(size_t)p * cap], w));
+        }
+    double2* o = Z + B.out + (size_t)col * B.ld + row;
+#pragma unroll
+    for (int p = 0; p < PL; ++p) o[(size_t)p * B.plane] = z[p];
 }
 
-// Single-entry evaluation (tests): out[0..3] = L(k1), L(k2), K(k1), K(k2); out[4] = MFIE(k1)
-__global__ void k_pair_probe(const RwgGeo* geo, int f, int s, GaussRule g, NearConsts c, double2* out) {
-    double2 L[2], K[2], M;
-    const double2 ks[2] = {c.k1, c.k2};
-    pair_ops<2, true, true, false>(geo[f], geo[s], g, ks, L, K, &M);
-    out[0] = L[0], out[1] = L[1], out[2] = K[0], out[3] = K[1];
-    double2 L1, K1;
-    pair_ops<1, false, false, true>(geo[f], geo[s], g, &c.k1, &L1, &K1, &M);
-    out[4] = M;
-}
-
-void launch_pair_probe(hipStream_t st, const RwgGeo* geo, int f, int s, const GaussRule& g, const NearConsts& c,
-                       double2* out) {
-    k_pair_probe<<<1, 1, 0, st>>>(geo, f, s, g, c, out);
+void launch_near_fill(hipStream_t st, int mode, const NearFill& nf, const int2* pair_items, int npair,
+                      const int2* same, int nsame, const int2* entry_items, int nentry, const GaussRule& g,
+                      const NearConsts& c, size_t cap, double2* scr, double2* Z) {
+    const unsigned sb = (unsigned)(((long long)nsame * 9 + 63) / 64);
+#define FILL(M)                                                                        \
+    k_face_pairs<M><<<npair, 64, 0, st>>>(nf, pair_items, g, c, cap, scr);             \
+    if (nsame > 0) k_face_same<M><<<sb, 64, 0, st>>>(nf, nsame, same, g, c, cap, scr); \
+    k_near_assemble<M == 2 ? 3 : 1><<<nentry, 256, 0, st>>>(nf, entry_items, cap, scr, Z)
+    if (npair == 0) return;
+    if (mode == 2) {
+        FILL(2);
+    } else if (mode == 1) {
+        FILL(1);
+    } else {
+        FILL(0);
+    }
+#undef FILL
 }
 
 // ---------------------------------------------------------------- patterns

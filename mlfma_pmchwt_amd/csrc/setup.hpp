@@ -17,11 +17,13 @@ struct ExcitationArgs {
     double alpha;
 };
 
-// mode 0 EFIE, 1 CFIE, 2 PMCHWT; one workgroup per leaf-pair block.
-void launch_near_fill(hipStream_t st, int mode, const NearDev& nd, const RwgGeo* geo, const GaussRule& g,
-                      const NearConsts& c, double2* Z);
-void launch_pair_probe(hipStream_t st, const RwgGeo* geo, int f, int s, const GaussRule& g, const NearConsts& c,
-                       double2* out);
+// mode 0 EFIE, 1 CFIE, 2 PMCHWT.  One batch of blocks of the near field: the
+// face-pair integrals (pair_items: block, chunk of 64 face pairs; same: block,
+// face pair with identical faces) into scr ([free-vertex pair][plane][cap]),
+// then the entries (entry_items: block, chunk of 256 entries) into Z.
+void launch_near_fill(hipStream_t st, int mode, const NearFill& nf, const int2* pair_items, int npair,
+                      const int2* same, int nsame, const int2* entry_items, int nentry, const GaussRule& g,
+                      const NearConsts& c, size_t cap, double2* scr, double2* Z);
 void launch_patterns(hipStream_t st, bool cfie, int N, int K, const RwgGeo* geo, const int* leaf_of,
                      const double* centre, const double* kp, double2 k, const GaussRule& g, double alpha, double2* Vs,
                      double2* Vf);
