@@ -708,10 +708,8 @@ void Engine::far_pass(int w, const double2* x, int ldr, int r0, int rb) {
     const int nc = ncur * rb;
     mark(6 * w + 0);
     cplx_t<R>* leaf_ws = F.Sm[L];
-    if constexpr (std::is_same<R, float>::value) {
-        if (eall_R_ > 0)   // aggregated for all right-hand sides already: this pass's leaf workspaces
-            F.Sm[L] = d_Sall_[w] + (size_t)nleaf * ncur * r0 * 3 * D.K[L];
-    }
+    if (eall_R_ > 0)   // aggregated for all right-hand sides already: this pass's leaf workspaces
+        F.Sm[L] = reinterpret_cast<cplx_t<R>*>(d_Sall_[w]) + (size_t)nleaf * ncur * r0 * 3 * D.K[L];
     if (F.Sm[L] == leaf_ws)
         launch_aggregate_b<R>(st, ncur, rb, nleaf, D.K[L], N, ldr, r0, d_leaf_order_, d_leaf_ptr_, d_perm_, F.Vs, x,
                               F.Sm[L]);
@@ -772,22 +770,25 @@ void Engine::translate(int w, int l, int nc) {
 template <typename R>
 void Engine::disaggregate(double2* y, int ldr, int r0, int rb) {
     const int L = tree.max_level;
-    if (std::is_same<R, float>::value && eall_R_ > 0) {   // deferred: this pass's columns of Eall only
+    if (eall_R_ > 0) {   // deferred: this pass's columns of Eall only
         const bool pm = ie == MLFMA_PMCHWT;
-        const bool split = d_Vb_[0] != nullptr;   // the split-pair product reads Eall as BF16 pairs
-        const FarDev<float>& F1 = far<float>(0);
+        // the split-pair product reads Eall as BF16 pairs
+        const bool split = std::is_same<R, float>::value && d_Vb_[0] != nullptr;
+        const int lde = eall_ld(eall_R_);
+        cplx_t<R>* E[2] = {reinterpret_cast<cplx_t<R>*>(d_Eall_[0]), reinterpret_cast<cplx_t<R>*>(d_Eall_[1])};
+        const FarDev<R>& F1 = far<R>(0);
         if (!pm) {
             const cplx c = (med.k1 * med.eta1 / (4.0 * kPi)) * (med.k1 / (4.0 * kPi));   // Code/MLFMM.cpp:226
             const double2 z = make_double2(0, 0);
-            launch_beff_all(st, nleaf, rb, wd_[0].K[L], false, F1.Bm[L], F1.kp0, d2(c), z, z, z, eall_R_, r0, split,
-                            d_Eall_[0]);
+            launch_beff_all<R>(st, nleaf, rb, wd_[0].K[L], false, F1.Bm[L], F1.kp0, d2(c), z, z, z, lde, r0, split,
+                               E[0]);
         } else {
-            const FarDev<float>& F2 = far<float>(1);
+            const FarDev<R>& F2 = far<R>(1);
             const cplx c1 = med.k1 * med.k1 / (16.0 * kPi * kPi), c2 = med.k2 * med.k2 / (16.0 * kPi * kPi);
-            launch_beff_all(st, nleaf, rb, wd_[0].K[L], true, F1.Bm[L], F1.kp0, d2(c1), d2(c1), d2(c1), d2(c1),
-                            eall_R_, r0, split, d_Eall_[0]);
-            launch_beff_all(st, nleaf, rb, wd_[1].K[L], true, F2.Bm[L], F2.kp0, d2(c2 * med.etai), d2(c2), d2(c2),
-                            d2(c2 / med.etai), eall_R_, r0, split, d_Eall_[1]);
+            launch_beff_all<R>(st, nleaf, rb, wd_[0].K[L], true, F1.Bm[L], F1.kp0, d2(c1), d2(c1), d2(c1), d2(c1),
+                               lde, r0, split, E[0]);
+            launch_beff_all<R>(st, nleaf, rb, wd_[1].K[L], true, F2.Bm[L], F2.kp0, d2(c2 * med.etai), d2(c2), d2(c2),
+                               d2(c2 / med.etai), lde, r0, split, E[1]);
         }
         return;
     }
@@ -948,13 +949,22 @@ void Engine::apply_block(const double2* X, double2* Y, int R, int prec, const fl
             prof_ms[3] += ms;
         }
     }
-    // FP32 far field with the matrix-core disaggregation: one product
-    // aggregates all R into the passes' leaf workspaces, the passes write
-    // their effective matrices into Eall, and one product disaggregates all R,
-    // so each pattern row is read once per matvec in each direction
-    // (with profiling on, the two all-R products are timed into the
-    // aggregation and disaggregation groups)
-    const bool all = f32 && mfma_near && disagg_mfma_;
+    // matrix-core near product and disaggregation: one product aggregates all
+    // right-hand sides into the passes' leaf workspaces, the passes write their
+    // effective matrices into Eall, and one product disaggregates all of them,
+    // so each pattern row is read once per matvec in each direction instead of
+    // once per pass.  FP64 does so for up to 32 at a time (kAll64; passes of 4
+    // read 3.6 GB of patterns per direction 16 times for 64 right-hand sides of
+    // 75,000 lossy PMCHWT RWG: 36 + 22 ms of two residuals, now 10.7 + 10.8).
+    // (with profiling on, the all-R products are timed into the aggregation
+    // and disaggregation groups)
+    if (!f32 && !capturing_) ensure_eall(R);
+    // columns per all-RHS product: whole passes, so that the passes are the same either way
+    const int width = f32 ? R : std::min({R, kAll64, all64_cols_});
+    const int step = width >= R ? R : width / cap * cap;
+    const bool all = mfma_near && disagg_mfma_ && step > 0;
+    const int L = tree.max_level;
+    const bool pm = ie == MLFMA_PMCHWT;
     auto timed = [&](int group, int launches, auto&& body) {
         if (prof_on_) MLFMA_HIP(hipEventRecord(ev_[16], st));
         body();
@@ -967,65 +977,106 @@ void Engine::apply_block(const double2* X, double2* Y, int R, int prec, const fl
             prof_launch[group] += launches;
         }
     };
-    if (all) {
-        ensure_eall(R);
-        const int L = tree.max_level;
+    auto passes = [&](const double2* x, double2* y, int n) {
+        for (int r0 = 0; r0 < n;) {
+            int rb = 1;
+            while (rb * 2 <= cap && r0 + rb * 2 <= n) rb *= 2;
+            apply_pass(x, y, R, r0, rb, prec, !mfma_near);
+            if (prof_on_) collect_profile(rb);
+            r0 += rb;
+        }
+    };
+    if (!all) {
+        passes(X, Y, R);
+        return;
+    }
+    if (f32) ensure_eall(R);
+    for (int s0 = 0; s0 < R; s0 += step) {
+        const int n = std::min(step, R - s0);
         timed(0, nw, [&] {
             for (int w = 0; w < nw; ++w) {
-                if (d_Va_[w] && xsplit)   // split-pair BF16 (near_precision = MLFMA_BF16), X split above
+                if (!f32)
+                    launch_aggregate_all<double>(st, ncur, nleaf, wd_[w].K[L], N, n, R, cap, d_leaf_ptr_, d_perm_,
+                                                 far<double>(w).Vs, X + s0, reinterpret_cast<double2*>(d_Sall_[w]));
+                else if (d_Va_[w] && xsplit)   // split-pair BF16 (near_precision = MLFMA_BF16), X split above
                     launch_aggregate_bf3(st, ncur, nleaf, wd_[w].K[L], N, R, cap, Qa_[w], Np_, d_leaf_ptr_, d_joff_,
                                          d_perm_, d_Va_[w], reinterpret_cast<const uint2*>(d_xf_), d_Sall_[w]);
                 else if (d_Va_[w])
                     launch_aggregate_bf3(st, ncur, nleaf, wd_[w].K[L], N, R, cap, Qa_[w], Np_, d_leaf_ptr_, d_joff_,
                                          d_perm_, d_Va_[w], X, d_Sall_[w]);
                 else
-                    launch_aggregate_all(st, ncur, nleaf, wd_[w].K[L], N, R, cap, d_leaf_ptr_, d_perm_,
-                                         far<float>(w).Vs, X, d_Sall_[w]);
+                    launch_aggregate_all<float>(st, ncur, nleaf, wd_[w].K[L], N, R, R, cap, d_leaf_ptr_, d_perm_,
+                                                far<float>(w).Vs, X, d_Sall_[w]);
             }
         });
-        eall_R_ = R;
-    }
-    try {
-        for (int r0 = 0; r0 < R;) {
-            int rb = 1;
-            while (rb * 2 <= cap && r0 + rb * 2 <= R) rb *= 2;
-            apply_pass(X, Y, R, r0, rb, prec, !mfma_near);
-            if (prof_on_) collect_profile(rb);
-            r0 += rb;
+        eall_R_ = n;
+        try {
+            passes(X + s0, Y + s0, n);
+        } catch (...) {
+            eall_R_ = 0;
+            throw;
         }
-    } catch (...) {
         eall_R_ = 0;
-        throw;
-    }
-    eall_R_ = 0;
-    if (all) {
-        const int L = tree.max_level;
-        const bool pm = ie == MLFMA_PMCHWT;
         timed(4, 1, [&] {
-            if (d_Vb_[0])   // split-pair BF16 (near_precision = MLFMA_BF16)
-                launch_disagg_bf3(st, R, nd_, pm, wd_[0].K[L], d_Vb_[0], reinterpret_cast<const uint2*>(d_Eall_[0]),
+            if (!f32)
+                launch_disagg_all<double>(st, n, eall_ld(n), R, nd_, pm, wd_[0].K[L], far<double>(0).Vf,
+                                          reinterpret_cast<const double2*>(d_Eall_[0]), pm ? wd_[1].K[L] : 0,
+                                          pm ? far<double>(1).Vf : nullptr,
+                                          reinterpret_cast<const double2*>(d_Eall_[1]), Y + s0);
+            else if (d_Vb_[0])   // split-pair BF16 (near_precision = MLFMA_BF16)
+                launch_disagg_bf3(st, R, eall_ld(R), nd_, pm, wd_[0].K[L], d_Vb_[0], reinterpret_cast<const uint2*>(d_Eall_[0]),
                                   pm ? wd_[1].K[L] : 0, pm ? d_Vb_[1] : nullptr,
                                   reinterpret_cast<const uint2*>(d_Eall_[1]), Y);
             else
-                launch_disagg_all(st, R, nd_, pm, wd_[0].K[L], far<float>(0).Vf, d_Eall_[0], pm ? wd_[1].K[L] : 0,
-                                  pm ? far<float>(1).Vf : nullptr, d_Eall_[1], Y);
+                launch_disagg_all<float>(st, R, eall_ld(R), R, nd_, pm, wd_[0].K[L], far<float>(0).Vf, d_Eall_[0],
+                                         pm ? wd_[1].K[L] : 0, pm ? far<float>(1).Vf : nullptr, d_Eall_[1], Y);
         });
     }
 }
 
-// All-RHS effective matrices of the FP32 far field (sized before any
-// recording: the recorded sequences hold their addresses)
+// All-RHS leaf workspaces and effective matrices (sized before any recording:
+// the recorded sequences hold their addresses): R columns of FP32 for the FP32
+// far field, and of FP64 for up to kAll64 columns, in the same buffers (64
+// columns of FP32 hold 32 of FP64).  Where the FP64 columns do not fit the
+// device, the FP64 matvec keeps to passes.
 void Engine::ensure_eall(int R) {
-    if (P.far_precision != MLFMA_FP32 || R <= eall_cap_) return;
+    if (R <= eall_cap_ || R < 2) return;
     clear_graphs();
     const int L = tree.max_level, no = ie == MLFMA_PMCHWT ? 2 : 1;
     for (int w = 0; w < nw; ++w) {
         dfree(d_Eall_[w]);
         dfree(d_Sall_[w]);
-        d_Eall_[w] = dalloc<float2>((size_t)nleaf * no * 3 * wd_[w].K[L] * R);
-        d_Sall_[w] = dalloc<float2>((size_t)nleaf * ncur * 3 * wd_[w].K[L] * R);
+        d_Eall_[w] = d_Sall_[w] = nullptr;
     }
-    eall_cap_ = R;
+    const int c32 = P.far_precision == MLFMA_FP32 ? eall_ld(R) : 0;
+    auto take = [&](int cols) {   // cols of FP32
+        for (int w = 0; w < nw; ++w) {
+            d_Eall_[w] = dalloc<float2>((size_t)nleaf * no * 3 * wd_[w].K[L] * cols);   // cols: a multiple of 8
+            d_Sall_[w] = dalloc<float2>((size_t)nleaf * ncur * 3 * wd_[w].K[L] * cols);
+        }
+        all64_cols_ = cols / 2 & ~7;   // whole padded columns (eall_ld)
+        eall_cap_ = R;
+    };
+    eall_cap_ = all64_cols_ = 0;
+    const int cols = std::max(c32, 2 * eall_ld(std::min(R, kAll64)));
+    try {
+        take(cols);
+        return;
+    } catch (const Error& e) {
+        if (e.code != MLFMA_ERR_OOM || cols == c32) throw;
+        (void)hipGetLastError();
+    }
+    for (int w = 0; w < nw; ++w) {
+        dfree(d_Eall_[w]);
+        dfree(d_Sall_[w]);
+        d_Eall_[w] = d_Sall_[w] = nullptr;
+    }
+    if (c32 > 0) {
+        take(c32);
+    } else {
+        all64_cols_ = 0;
+        eall_cap_ = R;
+    }
 }
 
 // Column-major device vectors (vector j at x + j * nunk), as the C ABI passes them.
@@ -2331,7 +2382,7 @@ void Engine::ensure_xf(int R) {
 // both large enough, as the FP64 polynomial does not run at the same time)
 void Engine::ensure_poly(int R) {
     ensure_xf(R);
-    ensure_eall(R);
+    if (P.far_precision == MLFMA_FP32) ensure_eall(R);
     if (R <= poly_cap_) return;
     clear_graphs();
     dfree(d_pt_);

@@ -302,7 +302,11 @@ private:
     int* d_jmap_ = nullptr;                          // RWG of each column, -1 for padding
     float2* d_Sall_[2] = {nullptr, nullptr};   // all-RHS leaf radiation workspaces of the passes, nleaf x ncur x 3K x eall_cap_
     int eall_cap_ = 0;
-    int eall_R_ = 0;   // > 0 while a batched FP32 matvec defers its disaggregation to one all-RHS product
+    int eall_R_ = 0;   // > 0 while a batched matvec defers its disaggregation to one all-RHS product
+    static constexpr int kAll64 = 32;   // FP64 columns of an all-RHS product
+    // columns of Eall, padded so that the passes' 2 to 8 columns start on 64-byte boundaries
+    static int eall_ld(int R) { return (R + 7) & ~7; }
+    int all64_cols_ = 0;                // FP64 columns that the all-RHS buffers hold
     float2* d_xf_ = nullptr;    // FP32 copy of the matrix-core near product's input, nunk x xf_cap_
     int xf_cap_ = 0;
     unsigned* d_xb_ = nullptr;  // BF16 copy of the preconditioner's near-product input, nunk x poly_cap_

@@ -194,12 +194,12 @@ void launch_disagg_mfma(hipStream_t st, int nleaf, int N, int ldr, int r0, int r
                                                    y);
 }
 
-// ---------------------------------------------------------------- all right-hand sides at once (FP32)
+// ---------------------------------------------------------------- all right-hand sides at once
 // The far-field passes write their effective matrices into one block
 // Eall[w][leaf][o][q][R] (q = d K + k as in E, right-hand sides fastest,
 // pass columns r0 .. r0 + rb - 1), and one product per matvec then reads
-// each pattern row once for all R right-hand sides instead of once per pass.
-// SPLIT (the split-pair disaggregation): each element is stored as its BF16
+// each pattern row once for all R right-hand sides instead of once per pass
+// (FP64: once per 32 right-hand sides, Engine::apply_block).  SPLIT (the split-pair disaggregation): each element is stored as its BF16
 // pairs, .x = hi Re | hi Im << 16, .y = lo Re | lo Im << 16 (8 bytes, as the
 // FP32 value), so the product stages them without converting.
 __device__ __forceinline__ unsigned bf16r(float f) {   // round to nearest even (finite inputs)
@@ -207,8 +207,8 @@ __device__ __forceinline__ unsigned bf16r(float f) {   // round to nearest even 
     u += 0x7fffu + ((u >> 16) & 1u);
     return u >> 16;
 }
-template <bool SPLIT>
-__device__ __forceinline__ void put_e(float2* E, size_t i, float2 v) {
+template <bool SPLIT, typename C2>
+__device__ __forceinline__ void put_e(C2* E, size_t i, C2 v) {
     if constexpr (SPLIT) {
         const unsigned hr = bf16r(v.x), hi = bf16r(v.y);
         const unsigned lr = bf16r(v.x - __uint_as_float(hr << 16)), li = bf16r(v.y - __uint_as_float(hi << 16));
@@ -217,66 +217,73 @@ __device__ __forceinline__ void put_e(float2* E, size_t i, float2 v) {
         E[i] = v;
     }
 }
-template <bool SPLIT>
-__global__ void k_beff_all(int nleaf, int rb, int K, int pmchwt, const float2* __restrict__ Bm,
-                           const float* __restrict__ kp, double2 ca, double2 cb, double2 cc, double2 cd, int R,
-                           int r0, float2* __restrict__ Eall) {
-    using M = Mx<float>;
+template <typename T, bool SPLIT>
+__global__ void k_beff_all(int nleaf, int rb, int K, int pmchwt, const cplx_t<T>* __restrict__ Bm,
+                           const T* __restrict__ kp, double2 ca, double2 cb, double2 cc, double2 cd, int lde,
+                           int r0, cplx_t<T>* __restrict__ Eall) {
+    using M = Mx<T>;
+    using C2 = cplx_t<T>;
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= (size_t)nleaf * rb * K) return;
     const int rr = (int)(e % rb);   // right-hand side fastest: the writes below are contiguous in it
     const int k = (int)((e / rb) % K), leaf = (int)(e / ((size_t)K * rb));
     const int ncur = pmchwt ? 2 : 1, no = pmchwt ? 2 : 1;
     const size_t Q = 3 * (size_t)K;
-    const float2* BJ = Bm + ((size_t)leaf * rb * ncur + (size_t)rr * ncur) * Q;
-    float2* EJ = Eall + (size_t)leaf * no * Q * R + r0 + rr;   // element (o, q) at EJ[(o Q + q) R]
+    const C2* BJ = Bm + ((size_t)leaf * rb * ncur + (size_t)rr * ncur) * Q;
+    C2* EJ = Eall + (size_t)leaf * no * Q * lde + r0 + rr;   // element (o, q) at EJ[(o Q + q) lde]
     if (!pmchwt) {
-        for (int d = 0; d < 3; ++d) put_e<SPLIT>(EJ, ((size_t)d * K + k) * R, M::mulc(ca, BJ[(size_t)d * K + k]));
+        for (int d = 0; d < 3; ++d) put_e<SPLIT>(EJ, ((size_t)d * K + k) * lde, M::mulc(ca, BJ[(size_t)d * K + k]));
         return;
     }
-    const float2* BM = BJ + Q;
-    float2* EM = EJ + Q * R;
-    const float kx = kp[k], ky = kp[K + k], kz = kp[2 * K + k];
-    float2 j[3], m[3];
+    const C2* BM = BJ + Q;
+    C2* EM = EJ + Q * lde;
+    const T kx = kp[k], ky = kp[K + k], kz = kp[2 * K + k];
+    C2 j[3], m[3];
     for (int d = 0; d < 3; ++d) j[d] = BJ[(size_t)d * K + k], m[d] = BM[(size_t)d * K + k];
-    const float2 cj[3] = {csub(cscale(j[2], ky), cscale(j[1], kz)), csub(cscale(j[0], kz), cscale(j[2], kx)),
+    const C2 cj[3] = {csub(cscale(j[2], ky), cscale(j[1], kz)), csub(cscale(j[0], kz), cscale(j[2], kx)),
                           csub(cscale(j[1], kx), cscale(j[0], ky))};
-    const float2 cm[3] = {csub(cscale(m[2], ky), cscale(m[1], kz)), csub(cscale(m[0], kz), cscale(m[2], kx)),
+    const C2 cm[3] = {csub(cscale(m[2], ky), cscale(m[1], kz)), csub(cscale(m[0], kz), cscale(m[2], kx)),
                           csub(cscale(m[1], kx), cscale(m[0], ky))};
     for (int d = 0; d < 3; ++d) {
-        put_e<SPLIT>(EJ, ((size_t)d * K + k) * R, csub(M::mulc(ca, j[d]), M::mulc(cb, cm[d])));
-        put_e<SPLIT>(EM, ((size_t)d * K + k) * R, cadd(M::mulc(cc, cj[d]), M::mulc(cd, m[d])));
+        put_e<SPLIT>(EJ, ((size_t)d * K + k) * lde, csub(M::mulc(ca, j[d]), M::mulc(cb, cm[d])));
+        put_e<SPLIT>(EM, ((size_t)d * K + k) * lde, cadd(M::mulc(cc, cj[d]), M::mulc(cd, m[d])));
     }
 }
 
-void launch_beff_all(hipStream_t st, int nleaf, int rb, int K, bool pmchwt, const float2* Bm, const float* kp,
-                     double2 ca, double2 cb, double2 cc, double2 cd, int R, int r0, bool split, float2* Eall) {
+template <typename T>
+void launch_beff_all(hipStream_t st, int nleaf, int rb, int K, bool pmchwt, const cplx_t<T>* Bm, const T* kp,
+                     double2 ca, double2 cb, double2 cc, double2 cd, int lde, int r0, bool split, cplx_t<T>* Eall) {
     if (nleaf == 0) return;
     const size_t total = (size_t)nleaf * rb * K;
     const unsigned grid = (unsigned)((total + 255) / 256);
-    if (split)
-        k_beff_all<true><<<grid, 256, 0, st>>>(nleaf, rb, K, pmchwt ? 1 : 0, Bm, kp, ca, cb, cc, cd, R, r0, Eall);
-    else
-        k_beff_all<false><<<grid, 256, 0, st>>>(nleaf, rb, K, pmchwt ? 1 : 0, Bm, kp, ca, cb, cc, cd, R, r0, Eall);
+    if constexpr (sizeof(T) == 4) {
+        if (split) {
+            k_beff_all<T, true><<<grid, 256, 0, st>>>(nleaf, rb, K, pmchwt ? 1 : 0, Bm, kp, ca, cb, cc, cd, lde, r0, Eall);
+            return;
+        }
+    }
+    k_beff_all<T, false><<<grid, 256, 0, st>>>(nleaf, rb, K, pmchwt ? 1 : 0, Bm, kp, ca, cb, cc, cd, lde, r0, Eall);
 }
 
 // Y[perm[i] (+N for output 1)][r] += sum_w V_w[i] . Eall_w[leaf][o][.][r] for all R.
 // The work items of the matrix-core near product (a leaf's range of up to 4
 // 16-row tiles, largest first); wavefront w owns row tile w and CT column
-// tiles of 8 right-hand sides, the pattern values of the next k-step are
-// loaded while the current one's products run (alternating register sets,
-// clamped branch-free loads), and Eall is staged in LDS kQ rows at a time,
-// the next chunk loaded into registers during the current one's products.
-template <int NO, int CT>
-__global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int nw, int K1, const float2* __restrict__ V1,
-                                                    const float2* __restrict__ E1, int K2,
-                                                    const float2* __restrict__ V2,
-                                                    const float2* __restrict__ E2, double2* __restrict__ y) {
-    using M = Mx<float>;
+// tiles of 8 right-hand sides.  Eall is staged in LDS kQ rows at a time; the
+// next chunk of it and of the pattern values is loaded during the current
+// one's products (alternating register sets, clamped branch-free loads).
+template <typename T, int NO, int CT>
+__global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int lde, int ldr, int nw, int K1,
+                                                    const cplx_t<T>* __restrict__ V1,
+                                                    const cplx_t<T>* __restrict__ E1, int K2,
+                                                    const cplx_t<T>* __restrict__ V2,
+                                                    const cplx_t<T>* __restrict__ E2, double2* __restrict__ y) {
+    using M = Mx<T>;
+    using C2 = cplx_t<T>;
+    using acc_t = typename M::acc;
     constexpr int RT = 8 * CT;
     constexpr int kQ = 16;
     constexpr int NE = NO * kQ * RT, NU = (NE + 255) / 256;
-    __shared__ float2 es[NO][kQ][RT];
+    __shared__ C2 es[NO][kQ][RT];
     const int2 item = nd.items[blockIdx.x];
     const int t = item.x, rp = item.y;
     const int i0 = nd.leaf_ptr[t], nt = nd.leaf_ptr[t + 1] - i0;
@@ -288,17 +295,17 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int nw, i
     const int part = li >> 3;
     const bool wact = wave < nrp;
     const int arow = min((rp + (wact ? wave : 0)) * 16 + li, nt - 1);
-    floatx4 acc[CT][NO];
+    acc_t acc[CT][NO];
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int o = 0; o < NO; ++o) acc[c][o] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float2 pe[NU];
+        for (int o = 0; o < NO; ++o) acc[c][o] = acc_t{0, 0, 0, 0};
+    C2 pe[NU];
     unsigned pmask = 0;
     for (int w = 0; w < nw; ++w) {
         const int Q = 3 * (w ? K2 : K1);
-        const float2* Vr = (w ? V2 : V1) + ((size_t)i0 + arow) * Q;   // this lane's pattern row
-        const float2* E = (w ? E2 : E1) + (size_t)t * NO * Q * R;
+        const C2* Vr = (w ? V2 : V1) + ((size_t)i0 + arow) * Q;   // this lane's pattern row
+        const C2* E = (w ? E2 : E1) + (size_t)t * NO * Q * lde;
         auto load_e = [&](int q0) {
             pmask = 0;
 #pragma unroll
@@ -306,27 +313,33 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int nw, i
                 const int e = threadIdx.x + 256 * u, ec = min(e, NE - 1);
                 const int o = ec / (kQ * RT), rem = ec - o * (kQ * RT);
                 const int qq = rem / RT, r = rem - qq * RT;
-                pe[u] = E[((size_t)o * Q + min(q0 + qq, Q - 1)) * R + rb0 + min(r, rv - 1)];
+                pe[u] = E[((size_t)o * Q + min(q0 + qq, Q - 1)) * lde + rb0 + min(r, rv - 1)];
                 pmask |= (unsigned)((NE % 256 == 0 || e < NE) & (q0 + qq < Q) & (r < rv)) << u;
             }
         };
-        auto step = [&](int kk, const float2& v) {
+        auto step = [&](int kk, const C2& v) {
             if (!wact) return;
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
                 for (int o = 0; o < NO; ++o) {
-                    const float2 ev = es[o][kk + lk][ct * 8 + (li & 7)];
-                    const float b1 = part ? ev.y : ev.x, b2 = part ? ev.x : -ev.y;
-                    floatx4 a = acc[ct][o];
+                    const C2 ev = es[o][kk + lk][ct * 8 + (li & 7)];
+                    const T b1 = part ? ev.y : ev.x, b2 = part ? ev.x : -ev.y;
+                    acc_t a = acc[ct][o];
                     a = M::op(v.x, b1, a);
                     a = M::op(v.y, b2, a);
                     acc[ct][o] = a;
                 }
         };
-        load_e(0);
-        float2 va = Vr[min(lk, Q - 1)], vb;
-        for (int q0 = 0; q0 < Q; q0 += kQ) {
+        // one chunk: stage Eall's rows, then the next chunk's loads, then the
+        // products from the current patterns; chunks alternate between two
+        // register sets (one past Q reads clamped patterns and meets zero Eall)
+        constexpr int KS = kQ / 4;
+        auto load_v = [&](int q0, C2* v) {
+#pragma unroll
+            for (int u = 0; u < KS; ++u) v[u] = Vr[min(q0 + 4 * u + lk, Q - 1)];
+        };
+        auto chunk = [&](int q0, const C2* cur, C2* nxt) {
             __syncthreads();
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
@@ -334,18 +347,21 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int nw, i
                 if (NE % 256 == 0 || e < NE) {
                     const int o = e / (kQ * RT), rem = e - o * (kQ * RT);
                     const int qq = rem / RT, r = rem - qq * RT;
-                    es[o][qq][r] = ((pmask >> u) & 1u) ? pe[u] : make_float2(0.f, 0.f);
+                    es[o][qq][r] = ((pmask >> u) & 1u) ? pe[u] : C2{0, 0};
                 }
             }
             __syncthreads();
             load_e(q0 + kQ);
+            load_v(q0 + kQ, nxt);
 #pragma unroll
-            for (int kk = 0; kk < kQ; kk += 8) {
-                vb = Vr[min(q0 + kk + 4 + lk, Q - 1)];
-                step(kk, va);
-                va = Vr[min(q0 + kk + 8 + lk, Q - 1)];
-                step(kk + 4, vb);
-            }
+            for (int u = 0; u < KS; ++u) step(4 * u, cur[u]);
+        };
+        C2 va[KS], vb[KS];
+        load_e(0);
+        load_v(0, va);
+        for (int q0 = 0; q0 < Q; q0 += 2 * kQ) {
+            chunk(q0, va, vb);
+            chunk(q0 + kQ, vb, va);
         }
     }
     if (!wact) return;
@@ -355,12 +371,12 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int nw, i
         for (int o = 0; o < NO; ++o)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const float re = acc[ct][o][v];
-                const float im = __shfl_xor(re, 8, 64);
+                const T re = acc[ct][o][v];
+                const T im = __shfl_xor(re, 8, 64);
                 const int row = (rp + wave) * 16 + M::row(lk, v);
                 const int rc = ct * 8 + li;
                 if (part == 0 && rc < rv && row < nt) {
-                    double2* yp = y + ((size_t)nd.perm[i0 + row] + (o ? (size_t)nd.N : 0)) * R + rb0 + rc;
+                    double2* yp = y + ((size_t)nd.perm[i0 + row] + (o ? (size_t)nd.N : 0)) * ldr + rb0 + rc;
                     double2 tt = *yp;
                     tt.x += (double)re;
                     tt.y += (double)im;
@@ -369,17 +385,21 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int nw, i
             }
 }
 
-void launch_disagg_all(hipStream_t st, int R, const NearDev& nd, bool pmchwt, int K1, const float2* V1,
-                       const float2* E1, int K2, const float2* V2, const float2* E2, double2* y) {
+template <typename T>
+void launch_disagg_all(hipStream_t st, int R, int lde, int ldr, const NearDev& nd, bool pmchwt, int K1, const cplx_t<T>* V1,
+                       const cplx_t<T>* E1, int K2, const cplx_t<T>* V2, const cplx_t<T>* E2, double2* y) {
     if (nd.nitem == 0 || R < 1) return;
-    const int ct = R > 32 ? 8 : (R > 16 ? 4 : (R > 8 ? 2 : 1));
+    // FP64: 32 right-hand sides at most per workgroup (64 registers of accumulators)
+    const int ct = R > 32 && sizeof(T) == 4 ? 8 : (R > 16 ? 4 : (R > 8 ? 2 : 1));
     dim3 grid(nd.nitem, (R + 8 * ct - 1) / (8 * ct));
-#define DA(NO, CT) k_disagg_all<NO, CT><<<grid, 256, 0, st>>>(nd, R, NO, K1, V1, E1, K2, V2, E2, y)
+#define DA(NO, CT) k_disagg_all<T, NO, CT><<<grid, 256, 0, st>>>(nd, R, lde, ldr, NO, K1, V1, E1, K2, V2, E2, y)
 #define DAN(NO)                                                                                                       \
-    if (ct == 8) DA(NO, 8);                                                                                           \
-    else if (ct == 4) DA(NO, 4);                                                                                      \
+    if constexpr (sizeof(T) == 4) {                                                                                   \
+        if (ct == 8) DA(NO, 8);                                                                                       \
+    }                                                                                                                 \
+    if (ct == 4) DA(NO, 4);                                                                                           \
     else if (ct == 2) DA(NO, 2);                                                                                      \
-    else DA(NO, 1);
+    else if (ct == 1) DA(NO, 1);
     if (pmchwt) {
         DAN(2)
     } else {
@@ -479,7 +499,7 @@ void launch_split_rows(hipStream_t st, int N, int Q, int Qp, const float2* V, un
 }
 
 template <int NO, int CT>
-__global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int nw, int K1,
+__global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, int nw, int K1,
                                                     const unsigned short* __restrict__ P1,
                                                     const uint2* __restrict__ E1, int K2,
                                                     const unsigned short* __restrict__ P2,
@@ -528,7 +548,7 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int nw, i
         const unsigned short* Pl = w ? P2 : P1;
         const size_t plane = (size_t)nd.N * Qp;
         const unsigned short* arow_p = Pl + ((size_t)i0 + arow) * Qp + 8 * lk;   // this lane's 8 q of plane 0
-        const uint2* E = (w ? E2 : E1) + (size_t)t * NO * Q * R;
+        const uint2* E = (w ? E2 : E1) + (size_t)t * NO * Q * lde;
         auto load_a = [&](int q0, uint4* a) {
             const int qc = min(q0, Qp - kQ);
 #pragma unroll
@@ -536,11 +556,11 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int nw, i
         };
         auto load_e = [&](int q0) {
             pmask = 0;
-            const uint2* Er = E + (size_t)so * Q * R + rb0 + min(sr, rv - 1);
+            const uint2* Er = E + (size_t)so * Q * lde + rb0 + min(sr, rv - 1);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int q = q0 + 8 * sg + i;
-                pe[i] = Er[(size_t)min(q, Q - 1) * R];
+                pe[i] = Er[(size_t)min(q, Q - 1) * lde];
                 pmask |= (unsigned)((q < Q) & (sr < rv)) << i;
             }
         };
@@ -615,13 +635,13 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int nw, i
             }
 }
 
-void launch_disagg_bf3(hipStream_t st, int R, const NearDev& nd, bool pmchwt, int K1, const unsigned short* P1,
+void launch_disagg_bf3(hipStream_t st, int R, int lde, const NearDev& nd, bool pmchwt, int K1, const unsigned short* P1,
                        const uint2* E1, int K2, const unsigned short* P2, const uint2* E2, double2* y) {
     if (nd.nitem == 0 || R < 1) return;
     const int ct = R > 16 ? 4 : (R > 8 ? 2 : 1);
     const int ny = (R + 8 * ct - 1) / (8 * ct);
     const unsigned grid = xcd_chunk_grid(nd.nitem, 4, ny);
-#define DB(NO, CT) k_disagg_bf3<NO, CT><<<grid, 256, 0, st>>>(nd, R, NO, K1, P1, E1, K2, P2, E2, y)
+#define DB(NO, CT) k_disagg_bf3<NO, CT><<<grid, 256, 0, st>>>(nd, R, lde, NO, K1, P1, E1, K2, P2, E2, y)
 #define DBN(NO)                                                                                                       \
     if (ct == 4) DB(NO, 4);                                                                                           \
     else if (ct == 2) DB(NO, 2);                                                                                      \
@@ -635,7 +655,7 @@ void launch_disagg_bf3(hipStream_t st, int R, const NearDev& nd, bool pmchwt, in
 #undef DB
 }
 
-// ---------------------------------------------------------------- aggregation, all right-hand sides (FP32)
+// ---------------------------------------------------------------- aggregation, all right-hand sides
 // Code/ProcessMLFMM.h:33-56 (mexp) for all R right-hand sides in one product:
 // per leaf, S (3K x ncur R) = V^T (3K x nt) X (nt x ncur R) on the matrix
 // cores, so each pattern row is read once per matvec.  Column c is current
@@ -646,16 +666,19 @@ void launch_disagg_bf3(hipStream_t st, int R, const NearDev& nd, bool pmchwt, in
 // single pass's workspace.  A workgroup owns one leaf and 4 16-row q tiles
 // (one per wavefront) and CT column tiles; X is staged in LDS kJ rows at a
 // time, the next chunk in flight during the current one's products.
-template <int NCUR, int CT>
-__global__ __launch_bounds__(256) void k_aggregate_all(int nleaf, int K, int N, int R, int cap,
+template <typename T, int NCUR, int CT>
+__global__ __launch_bounds__(256) void k_aggregate_all(int nleaf, int K, int N, int R, int ldr, int cap,
                                                        const int* __restrict__ leaf_ptr,
-                                                       const int* __restrict__ perm, const float2* __restrict__ Vs,
-                                                       const double2* __restrict__ x, float2* __restrict__ Sall) {
-    using M = Mx<float>;
+                                                       const int* __restrict__ perm,
+                                                       const cplx_t<T>* __restrict__ Vs,
+                                                       const double2* __restrict__ x, cplx_t<T>* __restrict__ Sall) {
+    using M = Mx<T>;
+    using C2 = cplx_t<T>;
+    using acc_t = typename M::acc;
     constexpr int CC = 8 * CT;   // columns per workgroup
     constexpr int kJ = 16;
     constexpr int NE = kJ * CC, NU = (NE + 255) / 256;
-    __shared__ float2 xs[kJ][CC];
+    __shared__ C2 xs[kJ][CC];
     const int Q = 3 * K, QG = (Q + 63) / 64;
     // the sample groups of one leaf (which read the same X rows) with their
     // column groups (which read the same pattern rows) run together on one XCD
@@ -671,12 +694,18 @@ __global__ __launch_bounds__(256) void k_aggregate_all(int nleaf, int K, int N, 
     const int part = li >> 3;
     const int q = (qg * 4 + wave) * 16 + li;   // this lane's row of the A operand (V^T)
     const int qc = min(q, Q - 1);
-    floatx4 acc[CT];
+    acc_t acc[CT];
 #pragma unroll
-    for (int c = 0; c < CT; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < CT; ++c) acc[c] = acc_t{0, 0, 0, 0};
     if (nt > 0) {
-        float2 px[NU];
+        C2 px[NU];
+        int pidx[NU];   // unknowns of the chunk whose X is loaded next (read one chunk earlier)
         unsigned pmask = 0;
+        auto load_perm = [&](int j0) {
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+                pidx[u] = perm[i0 + min(j0 + min((int)threadIdx.x + 256 * u, NE - 1) / CC, nt - 1)];
+        };
         auto load_x = [&](int j0) {
             pmask = 0;
 #pragma unroll
@@ -685,45 +714,54 @@ __global__ __launch_bounds__(256) void k_aggregate_all(int nleaf, int K, int N, 
                 const int jj = ec / CC, cc = ec - jj * CC;
                 const int c = min(cb0 + cc, ncol - 1);
                 const int r = c / NCUR, cur = c - r * NCUR;
-                const double2 v = x[((size_t)cur * N + perm[i0 + min(j0 + jj, nt - 1)]) * R + r];
-                px[u] = make_float2((float)v.x, (float)v.y);
+                const double2 v = x[((size_t)cur * N + pidx[u]) * ldr + r];
+                px[u] = C2{(T)v.x, (T)v.y};
                 pmask |= (unsigned)((NE % 256 == 0 || e < NE) & (j0 + jj < nt) & (cb0 + cc < ncol)) << u;
             }
         };
-        const float2* Vq = Vs + (size_t)i0 * Q + qc;   // element (j, q) at Vq[j Q]
-        auto vload = [&](int j) { return Vq[(size_t)min(j, nt - 1) * Q]; };
-        auto step = [&](int kk, const float2& v) {
+        const C2* Vq = Vs + (size_t)i0 * Q + qc;   // element (j, q) at Vq[j Q]
+        constexpr int KS = kJ / 4;
+        auto load_v = [&](int j0, C2* v) {
+#pragma unroll
+            for (int u = 0; u < KS; ++u) v[u] = Vq[(size_t)min(j0 + 4 * u + lk, nt - 1) * Q];
+        };
+        auto step = [&](int kk, const C2& v) {
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
-                const float2 xv = xs[kk + lk][ct * 8 + (li & 7)];
-                const float b1 = part ? xv.y : xv.x, b2 = part ? xv.x : -xv.y;
-                floatx4 a = acc[ct];
+                const C2 xv = xs[kk + lk][ct * 8 + (li & 7)];
+                const T b1 = part ? xv.y : xv.x, b2 = part ? xv.x : -xv.y;
+                acc_t a = acc[ct];
                 a = M::op(v.x, b1, a);
                 a = M::op(v.y, b2, a);
                 acc[ct] = a;
             }
         };
-        load_x(0);
-        float2 va = vload(lk), vb;
-        for (int j0 = 0; j0 < nt; j0 += kJ) {
+        // chunks alternate between two register sets, as in k_disagg_all
+        auto chunk = [&](int j0, const C2* cur, C2* nxt) {
             __syncthreads();
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
                 const int e = threadIdx.x + 256 * u;
                 if (NE % 256 == 0 || e < NE) {
                     const int jj = e / CC, cc = e - jj * CC;
-                    xs[jj][cc] = ((pmask >> u) & 1u) ? px[u] : make_float2(0.f, 0.f);
+                    xs[jj][cc] = ((pmask >> u) & 1u) ? px[u] : C2{0, 0};
                 }
             }
             __syncthreads();
             load_x(j0 + kJ);
+            load_perm(j0 + 2 * kJ);
+            load_v(j0 + kJ, nxt);
 #pragma unroll
-            for (int kk = 0; kk < kJ; kk += 8) {
-                vb = vload(j0 + kk + 4 + lk);
-                step(kk, va);
-                va = vload(j0 + kk + 8 + lk);
-                step(kk + 4, vb);
-            }
+            for (int u = 0; u < KS; ++u) step(4 * u, cur[u]);
+        };
+        C2 va[KS], vb[KS];
+        load_perm(0);
+        load_x(0);
+        load_perm(kJ);
+        load_v(0, va);
+        for (int j0 = 0; j0 < nt; j0 += 2 * kJ) {
+            chunk(j0, va, vb);
+            chunk(j0 + kJ, vb, va);
         }
     }
     // D[4 lk + v][li]: lanes li < 8 hold Re of column ct * 8 + li, lane li + 8 its Im
@@ -738,31 +776,36 @@ __global__ __launch_bounds__(256) void k_aggregate_all(int nleaf, int K, int N, 
             if (r < p0 + rb || p0 + rb >= R) break;
             p0 += rb;
         }
-        float2* S = Sall + (size_t)nleaf * NCUR * p0 * Q + ((size_t)leaf * rb + (r - p0)) * NCUR * Q +
+        C2* S = Sall + (size_t)nleaf * NCUR * p0 * Q + ((size_t)leaf * rb + (r - p0)) * NCUR * Q +
                     (size_t)cur * Q;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const float re = acc[ct][v];
-            const float im = __shfl_xor(re, 8, 64);
+            const T re = acc[ct][v];
+            const T im = __shfl_xor(re, 8, 64);
             const int qq = (qg * 4 + wave) * 16 + M::row(lk, v);
-            if (part == 0 && c < ncol && qq < Q) S[qq] = make_float2(re, im);
+            if (part == 0 && c < ncol && qq < Q) S[qq] = C2{re, im};
         }
     }
 }
 
-void launch_aggregate_all(hipStream_t st, int ncur, int nleaf, int K, int N, int R, int cap, const int* leaf_ptr,
-                          const int* perm, const float2* Vs, const double2* x, float2* Sall) {
+template <typename T>
+void launch_aggregate_all(hipStream_t st, int ncur, int nleaf, int K, int N, int R, int ldr, int cap,
+                          const int* leaf_ptr, const int* perm, const cplx_t<T>* Vs, const double2* x,
+                          cplx_t<T>* Sall) {
     if (nleaf == 0 || R < 1) return;
     const int ncol = ncur * R;
-    const int ct = ncol > 32 ? 8 : (ncol > 16 ? 4 : (ncol > 8 ? 2 : 1));
+    // FP64: 32 columns at most per workgroup (with 64, one wavefront per SIMD: 1.6 times slower)
+    const int ct = ncol > 32 && sizeof(T) == 4 ? 8 : (ncol > 16 ? 4 : (ncol > 8 ? 2 : 1));
     const int QG = (3 * K + 63) / 64, ncg = (ncol + 8 * ct - 1) / (8 * ct);
     const unsigned grid = xcd_chunk_grid(nleaf * QG, QG, ncg);
-#define AA(NC, CT) k_aggregate_all<NC, CT><<<grid, 256, 0, st>>>(nleaf, K, N, R, cap, leaf_ptr, perm, Vs, x, Sall)
+#define AA(NC, CT) k_aggregate_all<T, NC, CT><<<grid, 256, 0, st>>>(nleaf, K, N, R, ldr, cap, leaf_ptr, perm, Vs, x, Sall)
 #define AAN(NC)                                                                                                       \
-    if (ct == 8) AA(NC, 8);                                                                                           \
-    else if (ct == 4) AA(NC, 4);                                                                                      \
+    if constexpr (sizeof(T) == 4) {                                                                                   \
+        if (ct == 8) AA(NC, 8);                                                                                       \
+    }                                                                                                                 \
+    if (ct == 4) AA(NC, 4);                                                                                           \
     else if (ct == 2) AA(NC, 2);                                                                                      \
-    else AA(NC, 1);
+    else if (ct == 1) AA(NC, 1);
     if (ncur == 2) {
         AAN(2)
     } else {
@@ -989,7 +1032,13 @@ void launch_aggregate_bf3(hipStream_t st, int ncur, int nleaf, int K, int N, int
                                  double2, double2, cplx_t<T>*);                                                     \
     template void launch_disagg_mfma<T>(hipStream_t, int, int, int, int, int, const int*, const int*, const int*,  \
                                         bool, int, const cplx_t<T>*, const cplx_t<T>*, int, const cplx_t<T>*,      \
-                                        const cplx_t<T>*, double2*);
+                                        const cplx_t<T>*, double2*);                                               \
+    template void launch_beff_all<T>(hipStream_t, int, int, int, bool, const cplx_t<T>*, const T*, double2,        \
+                                     double2, double2, double2, int, int, bool, cplx_t<T>*);                        \
+    template void launch_disagg_all<T>(hipStream_t, int, int, int, const NearDev&, bool, int, const cplx_t<T>*,         \
+                                       const cplx_t<T>*, int, const cplx_t<T>*, const cplx_t<T>*, double2*);        \
+    template void launch_aggregate_all<T>(hipStream_t, int, int, int, int, int, int, int, const int*, const int*,  \
+                                          const cplx_t<T>*, const double2*, cplx_t<T>*);
 MLFMA_DISAGG_MFMA_INSTANTIATE(float)
 MLFMA_DISAGG_MFMA_INSTANTIATE(double)
 #undef MLFMA_DISAGG_MFMA_INSTANTIATE

@@ -146,27 +146,30 @@ template <typename T>
 void launch_disagg_mfma(hipStream_t st, int nleaf, int N, int ldr, int r0, int rb, const int* order,
                         const int* leaf_ptr, const int* perm, bool pmchwt, int K1, const cplx_t<T>* V1,
                         const cplx_t<T>* E1, int K2, const cplx_t<T>* V2, const cplx_t<T>* E2, double2* y);
-// All right-hand sides at once (FP32): the passes' effective matrices go into
-// Eall[leaf][o][3K][R] at columns r0 .. r0 + rb - 1, then one product per
-// matvec over the near product's work items (nd.items, leaf rows).
-// (split: each element stored as its BF16 pairs, uint2 .x = hi Re | hi Im << 16,
-// .y = lo Re | lo Im << 16, for launch_disagg_bf3)
-void launch_beff_all(hipStream_t st, int nleaf, int rb, int K, bool pmchwt, const float2* Bm, const float* kp,
-                     double2 ca, double2 cb, double2 cc, double2 cd, int R, int r0, bool split, float2* Eall);
-void launch_disagg_all(hipStream_t st, int R, const NearDev& nd, bool pmchwt, int K1, const float2* V1,
-                       const float2* E1, int K2, const float2* V2, const float2* E2, double2* y);
+// All right-hand sides at once: the passes' effective matrices go into
+// Eall[leaf][o][3K][lde] at columns r0 .. r0 + rb - 1, then one product per
+// matvec over the near product's work items (nd.items, leaf rows); y has
+// stride ldr.  (split, FP32 only: each element stored as its BF16 pairs, uint2
+// .x = hi Re | hi Im << 16, .y = lo Re | lo Im << 16, for launch_disagg_bf3)
+template <typename T>
+void launch_beff_all(hipStream_t st, int nleaf, int rb, int K, bool pmchwt, const cplx_t<T>* Bm, const T* kp,
+                     double2 ca, double2 cb, double2 cc, double2 cd, int lde, int r0, bool split, cplx_t<T>* Eall);
+template <typename T>
+void launch_disagg_all(hipStream_t st, int R, int lde, int ldr, const NearDev& nd, bool pmchwt, int K1, const cplx_t<T>* V1,
+                       const cplx_t<T>* E1, int K2, const cplx_t<T>* V2, const cplx_t<T>* E2, double2* y);
 // Split-pair BF16 disaggregation of all R: pattern planes [Re hi, Im hi,
 // Re lo, Im lo][N][Qp] (Qp = 3K rounded up to 32) from the FP32 patterns,
 // and the product from Eall stored as BF16 pairs (launch_beff_all, split).
 void launch_split_rows(hipStream_t st, int N, int Q, int Qp, const float2* V, unsigned short* planes);
-void launch_disagg_bf3(hipStream_t st, int R, const NearDev& nd, bool pmchwt, int K1, const unsigned short* P1,
+void launch_disagg_bf3(hipStream_t st, int R, int lde, const NearDev& nd, bool pmchwt, int K1, const unsigned short* P1,
                        const uint2* E1, int K2, const unsigned short* P2, const uint2* E2, double2* y);
-// Aggregation of all R right-hand sides (FP32 patterns, x RHS-fastest with
-// stride R) into the leaf workspaces of every pass of the batched matvec
+// Aggregation of all R right-hand sides (x RHS-fastest with stride ldr) into the leaf workspaces of every pass of the batched matvec
 // (passes of rb = largest power of two <= cap, pass (r0, rb) at
 // Sall + nleaf ncur r0 3K).
-void launch_aggregate_all(hipStream_t st, int ncur, int nleaf, int K, int N, int R, int cap, const int* leaf_ptr,
-                          const int* perm, const float2* Vs, const double2* x, float2* Sall);
+template <typename T>
+void launch_aggregate_all(hipStream_t st, int ncur, int nleaf, int K, int N, int R, int ldr, int cap,
+                          const int* leaf_ptr, const int* perm, const cplx_t<T>* Vs, const double2* x,
+                          cplx_t<T>* Sall);
 // The same product on split-pair BF16 from transposed pattern planes
 // [hi Re, hi Im, lo Re, lo Im][Qp][Np] (launch_split_cols; Qp a multiple of
 // 64, leaf t's RWGs from the 32-aligned column joff[t] on, jmap[column] = RWG
