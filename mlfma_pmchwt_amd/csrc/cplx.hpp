@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace mlfma {
 
 __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
@@ -80,6 +82,35 @@ __device__ __forceinline__ void xcd_chunk(int b, int cs, int ng, int& unit, int&
 inline unsigned xcd_chunk_grid(int units, int cs, int ng) {
     return (unsigned)((units + 8 * cs - 1) / (8 * cs)) * 8u * (unsigned)cs * (unsigned)ng;
 }
+
+// Work of a wavefront in an item of nrp <= 4 row tiles: with 1 or 2 tiles the
+// wavefronts without a row tile of their own take a share of another's CT
+// column tiles (of the row tiles of leaves of about 90 RWG a quarter of the
+// wavefronts had none, and held their registers idle): 75,000 lossy PMCHWT RWG,
+// FP64, 64 right-hand sides, near product 5.8 -> 5.0 ms, disaggregation of 32
+// 2.7 -> 2.2 ms; the BF16 products, bound by their loads, gain 1 to 4%.  tile: row tile; cb: first column tile; n: column tiles (CT, CT/2
+// or CT/4); on: whether there is any work.
+template <int CT>
+struct WaveShare {
+    int tile, cb, n;
+    bool on;
+    __device__ __forceinline__ WaveShare(int wave, int nrp) {
+        const int rows = nrp <= 2 ? nrp : 4;             // wavefronts over row tiles
+        const int parts = min(4 / rows, CT);             // wavefronts over column tiles
+        tile = wave % rows;
+        const int p = wave / rows;
+        n = CT / parts;
+        cb = p * n;
+        on = tile < nrp && p < parts;
+    }
+    // f(count) with the count of column tiles a compile-time constant
+    template <typename F>
+    __device__ __forceinline__ void each(F&& f) const {
+        if (n == CT) f(std::integral_constant<int, CT>{});
+        else if (CT >= 2 && n == CT / 2) f(std::integral_constant<int, (CT >= 2 ? CT / 2 : 1)>{});
+        else if (CT >= 4 && n == CT / 4) f(std::integral_constant<int, (CT >= 4 ? CT / 4 : 1)>{});
+    }
+};
 
 // Conversions between the FP64 solver vectors and the far-field precision.
 __device__ __forceinline__ void narrow(double2 a, double2& b) { b = a; }

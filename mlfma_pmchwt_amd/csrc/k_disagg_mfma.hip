@@ -272,7 +272,7 @@ void launch_beff_all(hipStream_t st, int nleaf, int rb, int K, bool pmchwt, cons
 // next chunk of it and of the pattern values is loaded during the current
 // one's products (alternating register sets, clamped branch-free loads).
 template <typename T, int NO, int CT>
-__global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int lde, int ldr, int nw, int K1,
+__global__ __launch_bounds__(256, sizeof(T) == 8 && NO == 2 && CT == 4 ? 3 : 1) void k_disagg_all(NearDev nd, int R, int lde, int ldr, int nw, int K1,
                                                     const cplx_t<T>* __restrict__ V1,
                                                     const cplx_t<T>* __restrict__ E1, int K2,
                                                     const cplx_t<T>* __restrict__ V2,
@@ -293,11 +293,14 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int lde, 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int part = li >> 3;
-    const bool wact = wave < nrp;
-    const int arow = min((rp + (wact ? wave : 0)) * 16 + li, nt - 1);
-    acc_t acc[CT][NO];
+    const WaveShare<CT> ws(wave, nrp);
+    const int arow = min((rp + (ws.on ? ws.tile : 0)) * 16 + li, nt - 1);
+    // the rest for this item's number of column tiles per wavefront
+    ws.each([&](auto cnt) {
+    constexpr int NC = decltype(cnt)::value;
+    acc_t acc[NC][NO];
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int o = 0; o < NO; ++o) acc[c][o] = acc_t{0, 0, 0, 0};
     C2 pe[NU];
@@ -318,12 +321,12 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int lde, 
             }
         };
         auto step = [&](int kk, const C2& v) {
-            if (!wact) return;
+            if (!ws.on) return;
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
+            for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
                 for (int o = 0; o < NO; ++o) {
-                    const C2 ev = es[o][kk + lk][ct * 8 + (li & 7)];
+                    const C2 ev = es[o][kk + lk][(ws.cb + ct) * 8 + (li & 7)];
                     const T b1 = part ? ev.y : ev.x, b2 = part ? ev.x : -ev.y;
                     acc_t a = acc[ct][o];
                     a = M::op(v.x, b1, a);
@@ -364,17 +367,17 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int lde, 
             chunk(q0 + kQ, vb, va);
         }
     }
-    if (!wact) return;
+    if (!ws.on) return;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
         for (int o = 0; o < NO; ++o)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const T re = acc[ct][o][v];
                 const T im = __shfl_xor(re, 8, 64);
-                const int row = (rp + wave) * 16 + M::row(lk, v);
-                const int rc = ct * 8 + li;
+                const int row = (rp + ws.tile) * 16 + M::row(lk, v);
+                const int rc = (ws.cb + ct) * 8 + li;
                 if (part == 0 && rc < rv && row < nt) {
                     double2* yp = y + ((size_t)nd.perm[i0 + row] + (o ? (size_t)nd.N : 0)) * ldr + rb0 + rc;
                     double2 tt = *yp;
@@ -383,6 +386,7 @@ __global__ __launch_bounds__(256) void k_disagg_all(NearDev nd, int R, int lde, 
                     *yp = tt;
                 }
             }
+    });
 }
 
 template <typename T>
@@ -531,11 +535,14 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int part = li >> 3;
-    const bool wact = wave < nrp;
-    const int arow = min((rp + (wact ? wave : 0)) * 16 + li, nt - 1);
-    floatx4 acc[CT][NO];
+    const WaveShare<CT> ws(wave, nrp);
+    const int arow = min((rp + (ws.on ? ws.tile : 0)) * 16 + li, nt - 1);
+    // the rest for this item's number of column tiles per wavefront
+    ws.each([&](auto cnt) {
+    constexpr int NC = decltype(cnt)::value;
+    floatx4 acc[NC][NO];
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int o = 0; o < NO; ++o) acc[c][o] = floatx4{0.f, 0.f, 0.f, 0.f};
     const bool sact = NUS == 256 || (int)threadIdx.x < NUS;
@@ -583,10 +590,10 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
             __syncthreads();
             load_e(q0 + kQ);
             load_a(q0 + kQ, nxt);
-            if (!wact) return;
+            if (!ws.on) return;
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const int rc = ct * 8 + (li & 7);
+            for (int ct = 0; ct < NC; ++ct) {
+                const int rc = (ws.cb + ct) * 8 + (li & 7);
 #pragma unroll
                 for (int o = 0; o < NO; ++o) {
                     floatx4 d = acc[ct][o];
@@ -614,17 +621,17 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
             chunk(q0 + kQ, ab, aa);
         }
     }
-    if (!wact) return;
+    if (!ws.on) return;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
         for (int o = 0; o < NO; ++o)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const float re = acc[ct][o][v];
                 const float im = __shfl_xor(re, 8, 64);
-                const int row = (rp + wave) * 16 + 4 * lk + v;
-                const int rc = ct * 8 + li;
+                const int row = (rp + ws.tile) * 16 + 4 * lk + v;
+                const int rc = (ws.cb + ct) * 8 + li;
                 if (part == 0 && rc < rv && row < nt) {
                     double2* yp = y + ((size_t)nd.perm[i0 + row] + (o ? (size_t)nd.N : 0)) * R + rb0 + rc;
                     double2 tt = *yp;
@@ -633,6 +640,7 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
                     *yp = tt;
                 }
             }
+    });
 }
 
 void launch_disagg_bf3(hipStream_t st, int R, int lde, const NearDev& nd, bool pmchwt, int K1, const unsigned short* P1,

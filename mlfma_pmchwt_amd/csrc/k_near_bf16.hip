@@ -163,7 +163,7 @@ __global__ void k_poly_init_bf16(size_t total, int R, const float2* __restrict__
 // other workgroups still gather from it); every (row, right-hand side) has one
 // owner, so t and y are updated without races.
 template <int P, int CT, bool S, bool F>
-__global__ __launch_bounds__(256) void k_near_bf16(NearDev nd, int R, int ldr, int r0, const uint4* __restrict__ Zb,
+__global__ __launch_bounds__(256, S && P == 3 && CT > 1 ? 2 : 1) void k_near_bf16(NearDev nd, int R, int ldr, int r0, const uint4* __restrict__ Zb,
                                                    const long long* __restrict__ bf_off,
                                                    const void* __restrict__ xbv, double2* __restrict__ y,
                                                    PolyEpi pe) {
@@ -202,8 +202,8 @@ __global__ __launch_bounds__(256) void k_near_bf16(NearDev nd, int R, int ldr, i
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int part = li >> 3;          // 0: real-part column, 1: imaginary-part column
-    const bool wact = wave < nrp;      // this wavefront's row tile exists
-    const uint4* zrec = Zb + bf_off[t] + (size_t)(rp + (wact ? wave : 0)) * P * W + lane;
+    const WaveShare<CT> ws(wave, nrp);
+    const uint4* zrec = Zb + bf_off[t] + (size_t)(rp + (ws.on ? ws.tile : 0)) * P * W + lane;
     const size_t kstride = (size_t)nrt * P * W;   // records of one 32-column block
     // records of block kb (clamped to the last block: a block past nkb is
     // loaded but never used), without bounds branches, which would make the
@@ -221,9 +221,12 @@ __global__ __launch_bounds__(256) void k_near_bf16(NearDev nd, int R, int ldr, i
             }
         }
     };
-    floatx4 acc[CT][NO];
+    // the rest for this item's number of column tiles per wavefront
+    ws.each([&](auto cnt) {
+    constexpr int NC = decltype(cnt)::value;
+    floatx4 acc[NC][NO];
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int o = 0; o < NO; ++o) acc[c][o] = floatx4{0.f, 0.f, 0.f, 0.f};
     // X staging, one chunk ahead: a thread's units (current xj, 8-column group
@@ -270,11 +273,11 @@ __global__ __launch_bounds__(256) void k_near_bf16(NearDev nd, int R, int ldr, i
     load_cref(kKC);
     // products of one 32-column block; zr/zi as filled by load
     auto step = [&](int kb2, const uint4* zr, const uint4* zi) {
-        if (!wact) return;
+        if (!ws.on) return;
         const int kof = kb2 * 32 + 8 * lk;
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const int rc = ct * 8 + (li & 7);
+        for (int ct = 0; ct < NC; ++ct) {
+            const int rc = (ws.cb + ct) * 8 + (li & 7);
             floatx4 a = acc[ct][0], b = acc[ct][NO - 1];
             auto ld = [&](int xp, int xj, int pl) { return *reinterpret_cast<const uint4*>(&xs[xp][xj][pl][rc][kof]); };
             // (Z part, X part) pairs: (hi, hi), and with S also (hi, lo), (lo, hi)
@@ -341,18 +344,18 @@ __global__ __launch_bounds__(256) void k_near_bf16(NearDev nd, int R, int ldr, i
         load(kb + 2, ar, ai);
         step(1, br, bi);
     }
-    if (!wact) return;
+    if (!ws.on) return;
     // D[4 lk + v][li]: lanes li < 8 hold Re of right-hand side ct * 8 + li, lane li + 8 its Im
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
         for (int o = 0; o < NO; ++o)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const float re = acc[ct][o][v];
                 const float im = __shfl_xor(re, 8, 64);
-                const int row = (rp + wave) * 16 + 4 * lk + v;
-                const int rc = ct * 8 + li;
+                const int row = (rp + ws.tile) * 16 + 4 * lk + v;
+                const int rc = (ws.cb + ct) * 8 + li;
                 if (part == 0 && rc < rv && row < nt) {
                     const size_t u = (size_t)nd.perm[i0 + row] + (o ? (size_t)nd.N : 0);
                     const size_t e = u * ldr + r0 + rb0 + rc;
@@ -369,6 +372,7 @@ __global__ __launch_bounds__(256) void k_near_bf16(NearDev nd, int R, int ldr, i
                     }
                 }
             }
+    });
 }
 
 long long bf16_near_layout(const std::vector<int>& leaf_ptr, const std::vector<int>& tgt_cols, int planes,

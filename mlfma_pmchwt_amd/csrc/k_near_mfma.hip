@@ -97,12 +97,12 @@ __global__ __launch_bounds__(256) void k_near_mfma(NearDev nd, int ldr, int r0, 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int part = li >> 3;   // 0: real-part column, 1: imaginary-part column
-    const bool wact = wave < nrp;   // this wavefront's row tile exists
+    const WaveShare<CT> ws(wave, nrp);
     // this lane's row of the A operand, clamped into the leaf: rows past nt
     // give output rows that are not stored, columns past C meet zero-staged X,
     // so the loads need no bounds branches (which would make the compiler wait
     // for the prefetched values before the current products)
-    const int arow = min((rp + (wact ? wave : 0)) * 16 + li, nt - 1);
+    const int arow = min((rp + (ws.on ? ws.tile : 0)) * 16 + li, nt - 1);
     // near-field values of global column gc for this lane's row
     auto load = [&](int gc, C2& z1, C2& zk, C2& z2) {
         const int off = min(gc, C - 1) * nt + arow;
@@ -112,9 +112,12 @@ __global__ __launch_bounds__(256) void k_near_mfma(NearDev nd, int ldr, int r0, 
             z2 = Zt[2 * plane + off];
         }
     };
-    acc_t acc[CT][NO];
+    // the rest for this item's number of column tiles per wavefront
+    ws.each([&](auto cnt) {
+    constexpr int NC = decltype(cnt)::value;
+    acc_t acc[NC][NO];
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int o = 0; o < NO; ++o) acc[c][o] = acc_t{0, 0, 0, 0};
     // FP32 staging units of this thread: element e = threadIdx.x + 256 u of
@@ -159,11 +162,11 @@ __global__ __launch_bounds__(256) void k_near_mfma(NearDev nd, int ldr, int r0, 
     // k-steps alternate between two register sets (no copies, so the next
     // step's values stay in flight during the current step's products)
     auto step = [&](int kk, const C2& z1, const C2& zk, const C2& z2) {
-        if (!wact) return;
+        if (!ws.on) return;
         const int cl = kk + lk;   // this lane's column in the chunk (< kCC); zero-staged past kend
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const int rc = ct * 8 + (li & 7);
+        for (int ct = 0; ct < NC; ++ct) {
+            const int rc = (ws.cb + ct) * 8 + (li & 7);
             const C2 xj = xs[0][cl][rc];
             const T bJ1 = part ? xj.y : xj.x, bJ2 = part ? xj.x : -xj.y;
             acc_t a = acc[ct][0];
@@ -227,23 +230,24 @@ __global__ __launch_bounds__(256) void k_near_mfma(NearDev nd, int ldr, int r0, 
             step(kk + 4, b1, bk, b2);
         }
     }
-    if (!wact) return;
+    if (!ws.on) return;
     // D[row(lk, v)][li]: lanes li < 8 hold Re of right-hand side ct * 8 + li, lane li + 8 its Im
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
         for (int o = 0; o < NO; ++o)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const T re = acc[ct][o][v];
                 const T im = __shfl_xor(re, 8, 64);
-                const int row = (rp + wave) * 16 + M::row(lk, v);
-                const int rc = ct * 8 + li;
+                const int row = (rp + ws.tile) * 16 + M::row(lk, v);
+                const int rc = (ws.cb + ct) * 8 + li;
                 if (part == 0 && rc < rv && row < nt) {
                     const size_t u = (size_t)nd.perm[i0 + row] + (o ? (size_t)nd.N : 0);
                     y[u * ldr + r0 + rb0 + rc] = make_double2((double)re, (double)im);
                 }
             }
+    });
 }
 
 template <typename T>
