@@ -24,6 +24,11 @@ double wall() {
 inline double2 d2(cplx c) { return make_double2(c.real(), c.imag()); }
 inline cplx cx(double2 d) { return cplx(d.x, d.y); }
 constexpr int kRedBlocks = 256;   // fixed partition of every reduction
+std::vector<int> three_each(int rows) {   // CSR offsets of a 3-point stencil
+    std::vector<int> p(rows + 1);
+    for (int i = 0; i <= rows; ++i) p[i] = 3 * i;
+    return p;
+}
 }  // namespace
 
 // Code/EMSource.cpp:34-72: incidence -r_hat, v = -theta_hat, h = phi_hat,
@@ -256,24 +261,40 @@ void Engine::build_wave(int w) {
     D.tap.assign(L + 1, nullptr);
     D.t_ptr.assign(L + 1, nullptr);
     D.t_kp.assign(L + 1, nullptr);
-    D.th_tap.assign(L + 1, nullptr);
+    D.up_rows.assign(L + 1, 0);
+    D.up_ptr.assign(L + 1, nullptr);
+    D.up_row.assign(L + 1, nullptr);
     D.ph_tap.assign(L + 1, nullptr);
-    D.at_ptr.assign(L + 1, nullptr);
-    D.at_idx.assign(L + 1, nullptr);
-    D.ap_ptr.assign(L + 1, nullptr);
-    D.ap_idx.assign(L + 1, nullptr);
+    D.dn_rows.assign(L + 1, 0);
+    D.ap_taps.assign(L + 1, 0);
+    D.dn_ptr.assign(L + 1, nullptr);
+    D.dn_row.assign(L + 1, nullptr);
+    D.ap_tap.assign(L + 1, nullptr);
     D.Lp.assign(L + 1, 0);
     D.Lc.assign(L + 1, 0);
     for (int l = 2; l <= L; ++l) D.K[l] = T.grid[l].K();
     for (int c = 3; c <= L; ++c) {
         const InterpTable& it = T.interp[c];
         D.tap[c] = upload(it.tap);
-        D.th_tap[c] = upload(it.th_tap);
         D.ph_tap[c] = upload(it.ph_tap);
-        D.at_ptr[c] = upload(it.at_ptr);
-        D.at_idx[c] = upload(it.at_idx);
-        D.ap_ptr[c] = upload(it.ap_ptr);
-        D.ap_idx[c] = upload(it.ap_idx);
+        std::vector<int> tap, win_ptr, win_row;
+        std::vector<double> tw;
+        D.up_rows[c] = m2m_rows(it.Lp, it.Lc);
+        if (D.up_rows[c] > 0) {
+            row_windows(three_each(it.Lp), it.th_tap, it.th_w, D.up_rows[c], win_ptr, win_row, tw);
+            D.up_ptr[c] = upload(win_ptr);
+            D.up_row[c] = upload(win_row);
+        }
+        const int taps = padded_taps(it.ap_ptr, it.ap_idx, it.ap_w, 1, tap, tw);
+        D.dn_rows[c] = l2l_rows(it.Lp, taps);
+        if (D.dn_rows[c] > 0) {
+            D.ap_taps[c] = l2l_taps(D.dn_rows[c], taps);
+            padded_taps(it.ap_ptr, it.ap_idx, it.ap_w, D.ap_taps[c], tap, tw);
+            D.ap_tap[c] = upload(tap);
+            row_windows(it.at_ptr, it.at_idx, it.at_w, D.dn_rows[c], win_ptr, win_row, tw);
+            D.dn_ptr[c] = upload(win_ptr);
+            D.dn_row[c] = upload(win_row);
+        }
         D.Lp[c] = it.Lp;
         D.Lc[c] = it.Lc;
         D.t_ptr[c] = upload(it.t_ptr);
@@ -350,9 +371,9 @@ void Engine::build_far(int w, const WaveTables& T) {
     F.Bm.assign(L + 1, nullptr);
     F.TFw.assign(L + 1, nullptr);
     F.tw.assign(L + 1, nullptr);
-    F.th_w.assign(L + 1, nullptr);
+    F.up_w.assign(L + 1, nullptr);
     F.ph_w.assign(L + 1, nullptr);
-    F.at_w.assign(L + 1, nullptr);
+    F.dn_w.assign(L + 1, nullptr);
     F.ap_w.assign(L + 1, nullptr);
     F.t_w.assign(L + 1, nullptr);
     F.sh_up.assign(L + 1, nullptr);
@@ -392,10 +413,19 @@ void Engine::build_far(int w, const WaveTables& T) {
     for (int c = 3; c <= L; ++c) {
         const InterpTable& it = T.interp[c];
         F.tw[c] = upload(to_real<R>(it.w));
-        F.th_w[c] = upload(to_real<R>(it.th_w));
         F.ph_w[c] = upload(to_real<R>(it.ph_w));
-        F.at_w[c] = upload(to_real<R>(it.at_w));
-        F.ap_w[c] = upload(to_real<R>(it.ap_w));
+        std::vector<int> tap, win_ptr, win_row;
+        std::vector<double> tw;
+        if (D.up_rows[c] > 0) {
+            row_windows(three_each(it.Lp), it.th_tap, it.th_w, D.up_rows[c], win_ptr, win_row, tw);
+            F.up_w[c] = upload(to_real<R>(tw));
+        }
+        if (D.dn_rows[c] > 0) {
+            padded_taps(it.ap_ptr, it.ap_idx, it.ap_w, D.ap_taps[c], tap, tw);
+            F.ap_w[c] = upload(to_real<R>(tw));
+            row_windows(it.at_ptr, it.at_idx, it.at_w, D.dn_rows[c], win_ptr, win_row, tw);
+            F.dn_w[c] = upload(to_real<R>(tw));
+        }
         F.t_w[c] = upload(to_real<R>(it.t_w));
         std::vector<cplx_t<R>> su(T.shift_up[c].size()), sd(T.shift_down[c].size());
         for (size_t e = 0; e < su.size(); ++e) su[e] = to_cx<R>(T.shift_up[c][e]);
@@ -730,10 +760,12 @@ void Engine::interpolate(int w, int l, int nc) {
     WaveDev& D = wd_[w];
     FarDev<R>& F = far<R>(w);
     const int c = l + 1;
-    if (m2m_separable_ && launch_m2m_sep<R>(st, nc, lv_[l].n, D.Lp[c], D.Lc[c], lv_[l].son_ptr, lv_[l].son_idx,
-                                            lv_[c].oct, D.th_tap[c], F.th_w[c], D.ph_tap[c], F.ph_w[c], F.sh_up[c],
-                                            F.Sm[c], F.Sm[l]))
+    if (m2m_separable_ && D.up_rows[c] > 0) {
+        launch_m2m_row<R>(st, nc, lv_[l].n, D.Lp[c], D.Lc[c], D.up_rows[c], lv_[l].son_ptr, lv_[l].son_idx,
+                          lv_[c].oct, D.up_ptr[c], D.up_row[c], F.up_w[c], D.ph_tap[c], F.ph_w[c], F.sh_up[c],
+                          F.Sm[c], F.Sm[l]);
         return;
+    }
     launch_m2m<R>(st, nc, lv_[l].n, D.K[l], D.K[c], lv_[l].son_ptr, lv_[l].son_idx, lv_[c].oct, D.tap[c], F.tw[c],
                   F.sh_up[c], F.Sm[c], F.Sm[l]);
 }
@@ -747,8 +779,8 @@ void Engine::translate(int w, int l, int nc) {
     const LevelDev& v = lv_[l];
     // the anterpolation from the parents either fused into the translation
     // (gather over the 9-tap stencil's transpose) or as a separable pass after it
-    const int rw = (l > 2 && l2l_separable_) ? l2l_sep_rows(nc, D.Lp[l], D.Lc[l], sizeof(cplx_t<R>)) : 0;
-    const bool up = l > 2 && rw == 0;
+    const bool sep = l > 2 && l2l_separable_ && D.dn_rows[l] > 0;
+    const bool up = l > 2 && !sep;
     if (m2l_cluster_ && m2l_variant_ == 2 && std::is_same<R, float>::value && (nc == 4 || nc == 8 || nc == 16))
         launch_m2l_cls<R>(st, nc, v.ncl8, D.K[l], v.cl8_child, v.cl8_ptr, v.cl8_src, v.cl8_vec, F.TFw[l], F.Sm[l],
                           up ? D.K[l - 1] : 0, v.parent, v.oct, D.t_ptr[l], D.t_kp[l], F.t_w[l], F.sh_dn[l],
@@ -761,9 +793,9 @@ void Engine::translate(int w, int l, int nc) {
         launch_m2l_l2l<R>(st, nc, v.n, D.K[l], v.dr_ptr, v.dr_idx, v.dr_vec, F.TFw[l], F.Sm[l], up ? D.K[l - 1] : 0,
                           v.parent, v.oct, D.t_ptr[l], D.t_kp[l], F.t_w[l], F.sh_dn[l], up ? F.Bm[l - 1] : nullptr,
                           F.Bm[l]);
-    if (rw > 0)
-        launch_l2l_sep<R>(st, nc, v.n, D.Lp[l], D.Lc[l], rw, v.parent, v.oct, D.at_ptr[l], D.at_idx[l], F.at_w[l],
-                          D.ap_ptr[l], D.ap_idx[l], F.ap_w[l], F.sh_dn[l], F.Bm[l - 1], F.Bm[l]);
+    if (sep)
+        launch_l2l_row<R>(st, nc, v.n, D.Lp[l], D.Lc[l], D.dn_rows[l], D.ap_taps[l], v.parent, v.oct, D.dn_ptr[l],
+                          D.dn_row[l], F.dn_w[l], D.ap_tap[l], F.ap_w[l], F.sh_dn[l], F.Bm[l - 1], F.Bm[l]);
 }
 
 // y += far field (finest Bm of every wavenumber), same right-hand-side range

@@ -63,16 +63,22 @@ struct FarDev {
     R* kp0 = nullptr;                    // [3][K0] finest-level directions
     std::vector<cplx_t<R>*> Sm, Bm, TFw;     // per tree level
     std::vector<R*> tw, t_w;             // per child tree level
-    std::vector<R*> th_w, ph_w;          // per child tree level: the stencil's weights by direction
-    std::vector<R*> at_w, ap_w;          // per child tree level: the transposed stencils' weights
+    std::vector<R*> up_w, ph_w;          // per child tree level: weights of the interpolation's row windows, phi weights
+    std::vector<R*> dn_w, ap_w;          // per child tree level: weights of the anterpolation's row windows and taps
     std::vector<cplx_t<R>*> sh_up, sh_dn;
 };
 
 struct WaveDev {
     std::vector<int> K;                  // per tree level
     std::vector<int*> tap, t_ptr, t_kp;  // per child tree level
-    std::vector<int*> th_tap, ph_tap;    // per child tree level: the stencil's taps by direction
-    std::vector<int*> at_ptr, at_idx, ap_ptr, ap_idx;   // per child tree level: transposed, by direction
+    // per child tree level, separable interpolation: parent rows per group (0: does not apply), the groups'
+    // windows of child rows, the phi taps
+    std::vector<int> up_rows;
+    std::vector<int*> up_ptr, up_row, ph_tap;
+    // per child tree level, separable anterpolation: child rows per group (0: does not apply), the groups'
+    // windows of parent rows, the padded phi taps per child column
+    std::vector<int> dn_rows, ap_taps;
+    std::vector<int*> dn_ptr, dn_row, ap_tap;
     std::vector<int> Lp, Lc;             // per child tree level: theta rows of the parent and child grids
     FarDev<double> f64;                  // always built (true residuals, stage API)
     FarDev<float> f32;                   // built when far_precision = MLFMA_FP32

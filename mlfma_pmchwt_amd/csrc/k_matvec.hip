@@ -298,285 +298,326 @@ void launch_m2m(hipStream_t st, int ncur, int nparent, int Kp, int Kc, const int
 #undef M2M
 }
 
-// Separable form of the same interpolation: the 3 x 3 stencil of a parent
+// Code/ProcessMLFMM.h:61-107 (m2m) in separable form: the 3x3 stencil of parent
 // sample (i, j) is child rows th_tap[i][a] x child columns ph_tap[j][b] with
-// weights th_w[i][a] ph_w[j][b], so a workgroup owning RW consecutive rows of
-// parent p first interpolates in theta, U(i, m) = sum_a th_w[i][a]
-// S_c(th_tap[i][a], m), for all 2 Lc child columns m of each of its CPT
-// columns into LDS (contiguous rows of the child workspace), then in phi,
-// r(i, j) = sum_b ph_w[j][b] U(i, ph_tap[j][b]), and adds shift x r, child
-// after child.  About half the loads and multiply-adds of the 9-tap form; the
-// sums are regrouped (theta inside), which changes only rounding.  The lanes
-// of a wavefront run over (row, column) pairs of its rows, so short rows
-// still fill the wavefront and a workgroup's barriers serve RW rows; a thread
-// owns outputs t = lane + 64 jj (jj < JJ) of the RW x 2 Lp block.  G = nc x 3 /
-// CPT wavefronts, one per column group, each with its own LDS rows.
-template <typename R, int NC, int CPT, int JJ>
-__global__ __launch_bounds__(64 * NC * 3 / CPT) void k_m2m_sep(int Lp, int Lc, int RW, const int* __restrict__ son_ptr,
-                                                        const int* __restrict__ son_idx,
-                                                        const int* __restrict__ oct_child,
-                                                        const int* __restrict__ th_tap, const R* __restrict__ th_w,
-                                                        const int* __restrict__ ph_tap, const R* __restrict__ ph_w,
-                                                        const cplx_t<R>* __restrict__ shup,
-                                                        const cplx_t<R>* __restrict__ Smc,
-                                                        cplx_t<R>* __restrict__ Smp) {
+// weights th_w[i][a] ph_w[j][b], so theta comes first, U(i, m) = sum_a th_w[i][a]
+// S_c(th_tap[i][a], m), then phi, r(i, j) = sum_b ph_w[j][b] U(i, ph_tap[j][b]),
+// and shift x r is added child after child.  About half the loads and
+// multiply-adds of the 9-tap form; the sums are regrouped, which changes only
+// rounding.  A wavefront takes RW rows of a parent and CPT of the nc x 3
+// columns.  Theta: its lanes run over the child's columns and it walks the
+// window of child rows that its parent rows take (win_*: row_windows of the
+// theta stencil), so a child sample is loaded once per group of RW rows and
+// added to the RW rows in registers, the next row's loads in flight.  (Parent
+// row by parent row each child sample was loaded about four times: C5, 64
+// right-hand sides, 4.4 ms per matvec, now 3.3.)  Phi: the rows go through the
+// wavefront's own LDS (no barrier), lanes over (row, parent column) pairs, JJ
+// outputs per thread kept in registers over the children.
+template <typename R, int CPT, int RW, int JJ>
+__global__ __launch_bounds__(256) void k_m2m_row(int nc, int Lp, int Lc, int ncb, const int* __restrict__ son_ptr,
+                                                 const int* __restrict__ son_idx,
+                                                 const int* __restrict__ oct_child,
+                                                 const int* __restrict__ win_ptr, const int* __restrict__ win_row,
+                                                 const R* __restrict__ win_w, const int* __restrict__ ph_tap,
+                                                 const R* __restrict__ ph_w, const cplx_t<R>* __restrict__ shup,
+                                                 const cplx_t<R>* __restrict__ Smc, cplx_t<R>* __restrict__ Smp) {
     using C = cplx_t<R>;
     extern __shared__ __align__(16) unsigned char m2m_lds[];
     const int pfn = 2 * Lp, psn = 2 * Lc, Kp = Lp * pfn, Kc = Lc * psn;
     const int nrg = (Lp + RW - 1) / RW;   // row groups per parent
     const int lin = xcd_remap(blockIdx.x, (int)gridDim.x);
-    const int p = lin / nrg, i0 = (lin % nrg) * RW;   // the row groups of one parent are consecutive
-    const int nr = min(RW, Lp - i0);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int c0 = wave * CPT;
-    const int us = RW * psn;                                            // one column's U block
-    C* U = reinterpret_cast<C*>(m2m_lds) + (size_t)wave * CPT * us;   // this wavefront's [CPT][RW][2 Lc]
-    // phi-pass outputs of this thread: row ir[jj] (relative), column jc[jj]
-    int ir[JJ], jc[JJ], pj[JJ][3];
+    const int cb = lin % ncb, g = (lin / ncb) % nrg, p = lin / (ncb * nrg);   // one parent's workgroups are consecutive
+    const int i0 = g * RW, nr = min(RW, Lp - i0);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int c0 = (cb * (int)(blockDim.x >> 6) + wave) * CPT;
+    C* U = reinterpret_cast<C*>(m2m_lds) + (size_t)wave * CPT * RW * psn;   // [CPT][RW][2 Lc]
+    // phi-pass outputs of this thread (t = lane + 64 jj, clamped past the last)
+    int pj[JJ][3];
     R wj[JJ][3];
-    bool ok[JJ];
+    C out[JJ][CPT];
 #pragma unroll
     for (int jj = 0; jj < JJ; ++jj) {
-        const int t = lane + 64 * jj;
-        ok[jj] = t < nr * pfn;
-        const int tc = min(t, nr * pfn - 1);
-        ir[jj] = tc / pfn;
-        jc[jj] = tc - ir[jj] * pfn;
+        const int t = min(lane + 64 * jj, nr * pfn - 1);
+        const int r = t / pfn, j = t - r * pfn;
 #pragma unroll
         for (int b = 0; b < 3; ++b) {
-            pj[jj][b] = ir[jj] * psn + ph_tap[3 * jc[jj] + b];
-            wj[jj][b] = ph_w[3 * jc[jj] + b];
+            pj[jj][b] = r * psn + ph_tap[3 * j + b];
+            wj[jj][b] = ph_w[3 * j + b];
         }
+#pragma unroll
+        for (int d = 0; d < CPT; ++d) out[jj][d] = C{0, 0};
     }
-    C acc[JJ][CPT];
+    const int k0 = win_ptr[g], k1 = win_ptr[g + 1];
+    const int s0 = son_ptr[p], s1 = son_ptr[p + 1];
+    if (s0 == s1) return;   // (every box of a parent level has a child)
+    auto load = [&](const C* S, int m, int k, C (&v)[CPT]) {
+        const int at = win_row[min(k, k1 - 1)] * psn + m;
 #pragma unroll
-    for (int jj = 0; jj < JJ; ++jj)
+        for (int d = 0; d < CPT; ++d) v[d] = S[(size_t)d * Kc + at];
+    };
+    auto block = [&](int s) { return Smc + ((size_t)son_idx[s] * nc * 3 + c0) * Kc; };
+    // four rows in flight; the first two of the next 64 columns or child are
+    // loaded before this one's phi pass
+    C va[CPT], vb[CPT], vc[CPT], vd[CPT];
+    const C* S = block(s0);
+    load(S, min(lane, psn - 1), k0, va);
+    load(S, min(lane, psn - 1), k0 + 1, vb);
+    for (int s = s0; s < s1; ++s) {
+        const C* Sn = block(min(s + 1, s1 - 1));
+        for (int mb = 0; mb < psn; mb += 64) {
+            const int m = min(mb + lane, psn - 1);
+            C acc[RW][CPT];
 #pragma unroll
-        for (int d = 0; d < CPT; ++d) acc[jj][d] = C{0, 0};
-    // theta-pass items of this thread (t = lane + 64 k < RW 2 Lc <= 192 with the
-    // launch's LDS bound): child offsets and weights, the same for every child
-    constexpr int KT = 3;
-    int ti[KT][3];
-    R lt[KT][3];
+            for (int r = 0; r < RW; ++r)
 #pragma unroll
-    for (int k = 0; k < KT; ++k) {
-        const int t = min(lane + 64 * k, nr * psn - 1);
-        const int r = t / psn, m = t - r * psn;
+                for (int d = 0; d < CPT; ++d) acc[r][d] = C{0, 0};
+            auto add = [&](int k, const C (&v)[CPT]) {
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            ti[k][a] = th_tap[3 * (i0 + r) + a] * psn + m;
-            lt[k][a] = th_w[3 * (i0 + r) + a];
-        }
-    }
-    for (int s = son_ptr[p]; s < son_ptr[p + 1]; ++s) {
-        const int c = son_idx[s];
-        const C* S = Smc + ((size_t)c * NC * 3 + c0) * Kc;
+                for (int r = 0; r < RW; ++r) {
+                    const R w = win_w[(size_t)k * RW + r];
 #pragma unroll
-        for (int k = 0; k < KT; ++k) {
-            const int t = lane + 64 * k;
-            if (t < nr * psn) {
-#pragma unroll
-                for (int d = 0; d < CPT; ++d) {
-                    const C* sd = S + (size_t)d * Kc;
-                    const C f0 = sd[ti[k][0]], f1 = sd[ti[k][1]], f2 = sd[ti[k][2]];
-                    C u;
-                    u.x = f0.x * lt[k][0] + f1.x * lt[k][1] + f2.x * lt[k][2];
-                    u.y = f0.y * lt[k][0] + f1.y * lt[k][1] + f2.y * lt[k][2];
-                    U[d * us + t] = u;
+                    for (int d = 0; d < CPT; ++d) {
+                        acc[r][d].x = fma(w, v[d].x, acc[r][d].x);
+                        acc[r][d].y = fma(w, v[d].y, acc[r][d].y);
+                    }
                 }
+            };
+            for (int k = k0; k < k1; k += 4) {
+                load(S, m, k + 2, vc);
+                load(S, m, k + 3, vd);
+                __builtin_amdgcn_sched_barrier(0);
+                add(k, va);
+                if (k + 1 < k1) add(k + 1, vb);
+                const bool more = k + 4 < k1, same = mb + 64 < psn;   // uniform
+                const C* Sl = more || same ? S : Sn;
+                const int ml = more ? m : min((same ? mb + 64 : 0) + lane, psn - 1);
+                load(Sl, ml, more ? k + 4 : k0, va);
+                load(Sl, ml, more ? k + 5 : k0 + 1, vb);
+                __builtin_amdgcn_sched_barrier(0);
+                if (k + 2 < k1) add(k + 2, vc);
+                if (k + 3 < k1) add(k + 3, vd);
             }
+            if (mb + lane < psn)
+#pragma unroll
+                for (int d = 0; d < CPT; ++d)
+#pragma unroll
+                    for (int r = 0; r < RW; ++r) U[(d * RW + r) * psn + m] = acc[r][d];
         }
-        __syncthreads();
-        const C* sh = shup + (size_t)oct_child[c] * Kp + (size_t)i0 * pfn;
+        S = Sn;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // other lanes of this wavefront wrote U
+        const C* sh = shup + (size_t)oct_child[son_idx[s]] * Kp + (size_t)i0 * pfn;
 #pragma unroll
         for (int jj = 0; jj < JJ; ++jj) {
-            if (ok[jj]) {
-                const C e = sh[ir[jj] * pfn + jc[jj]];
+            const C e = sh[min(lane + 64 * jj, nr * pfn - 1)];
 #pragma unroll
-                for (int d = 0; d < CPT; ++d) {
-                    const C u0 = U[d * us + pj[jj][0]], u1 = U[d * us + pj[jj][1]], u2 = U[d * us + pj[jj][2]];
-                    C r;
-                    r.x = u0.x * wj[jj][0] + u1.x * wj[jj][1] + u2.x * wj[jj][2];
-                    r.y = u0.y * wj[jj][0] + u1.y * wj[jj][1] + u2.y * wj[jj][2];
-                    cfma(acc[jj][d], e, r);
-                }
+            for (int d = 0; d < CPT; ++d) {
+                const C u0 = U[d * RW * psn + pj[jj][0]], u1 = U[d * RW * psn + pj[jj][1]],
+                        u2 = U[d * RW * psn + pj[jj][2]];
+                C r;
+                r.x = u0.x * wj[jj][0] + u1.x * wj[jj][1] + u2.x * wj[jj][2];
+                r.y = u0.y * wj[jj][0] + u1.y * wj[jj][1] + u2.y * wj[jj][2];
+                cfma(out[jj][d], e, r);
             }
         }
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // U is read before the next child's rows replace it
     }
-    C* o = Smp + ((size_t)p * NC * 3 + c0) * Kp + (size_t)i0 * pfn;
+    C* o = Smp + ((size_t)p * nc * 3 + c0) * Kp + (size_t)i0 * pfn;
 #pragma unroll
     for (int jj = 0; jj < JJ; ++jj)
-        if (ok[jj])
+        if (lane + 64 * jj < nr * pfn)
 #pragma unroll
-            for (int d = 0; d < CPT; ++d) o[(size_t)d * Kp + ir[jj] * pfn + jc[jj]] = acc[jj][d];
+            for (int d = 0; d < CPT; ++d) o[(size_t)d * Kp + lane + 64 * jj] = out[jj][d];
 }
 
-// The separable interpolation when a parent row has at most 256 samples and
-// one row of every column fits in LDS (64 KB per workgroup); false otherwise
-// (the caller takes the 9-tap kernel).  A workgroup takes as many rows as fit
-// both (RW 2 Lp <= 256 outputs per lane group, RW rows of LDS).
+// Parent rows per group: 4 up to rows of 64 samples, 2 up to 192, then 1 (with
+// 4 outputs per thread; 6 for 2 rows).  4 rows of 65 to 96 samples take 6
+// outputs as well and run slower (FP64: one wavefront per SIMD, 76 against 45
+// us at 2 rows; FP32 39 against 34), 1 row of 129 to 192 slower than 2 (64.5
+// against 51).  0 (the caller takes the 9-tap kernel) where a row has more than
+// 256 samples or does not fit 64 KB of LDS.
+int m2m_rows(int Lp, int Lc) {
+    const size_t row = (size_t)3 * 2 * Lc * sizeof(double2);
+    if (2 * Lp > 256 || row > 64 * 1024) return 0;
+    if (2 * Lp <= 64 && 4 * row <= 64 * 1024) return 4;
+    if (2 * Lp <= 192 && 2 * row <= 64 * 1024) return 2;
+    return 1;
+}
+
 template <typename R>
-bool launch_m2m_sep(hipStream_t st, int ncur, int nparent, int Lp, int Lc, const int* son_ptr, const int* son_idx,
-                    const int* octant_child, const int* th_tap, const R* th_w, const int* ph_tap, const R* ph_w,
-                    const cplx_t<R>* shift_up, const cplx_t<R>* Sm_child, cplx_t<R>* Sm_parent) {
-    if (nparent == 0) return true;
-    const size_t row_lds = (size_t)ncur * 3 * 2 * Lc * sizeof(cplx_t<R>);   // one row of all column groups
-    if (2 * Lp > 256 || row_lds > 64 * 1024) return false;
-    if (2 * Lc > 192) return false;   // theta-pass items per lane (KT = 3)
-    const int RW = std::max(1, std::min({Lp, (int)(64 * 1024 / row_lds), 256 / (2 * Lp), 192 / (2 * Lc)}));
-    const int JJ = (RW * 2 * Lp + 63) / 64;
-    const size_t lds = row_lds * RW;
-    const unsigned grid = (unsigned)nparent * ((Lp + RW - 1) / RW);
-#define M2MS(NC, CPT, J)                                                                                              \
-    k_m2m_sep<R, NC, CPT, J><<<grid, 64 * NC * 3 / CPT, lds, st>>>(Lp, Lc, RW, son_ptr, son_idx, octant_child,      \
-                                                                    th_tap, th_w, ph_tap, ph_w, shift_up, Sm_child, \
-                                                                    Sm_parent)
-#define M2MS_J(NC, CPT)                                                                                               \
-    if (JJ == 1) M2MS(NC, CPT, 1);                                                                                    \
-    else if (JJ == 2) M2MS(NC, CPT, 2);                                                                               \
-    else if (JJ == 3) M2MS(NC, CPT, 3);                                                                               \
-    else M2MS(NC, CPT, 4);
-    if (ncur == 1) {
-        M2MS_J(1, 3)
-    } else if (ncur == 2) {
-        M2MS_J(2, 3)
-    } else if (ncur == 4) {
-        M2MS_J(4, 3)
-    } else if (ncur == 8) {
-        M2MS_J(8, 3)
-    } else if constexpr (sizeof(R) == 4) {
-        M2MS_J(16, 6)
+void launch_m2m_row(hipStream_t st, int ncur, int nparent, int Lp, int Lc, int rw, const int* son_ptr,
+                    const int* son_idx, const int* octant_child, const int* win_ptr, const int* win_row,
+                    const R* win_w, const int* ph_tap, const R* ph_w, const cplx_t<R>* shift_up,
+                    const cplx_t<R>* Sm_child, cplx_t<R>* Sm_parent) {
+    if (nparent == 0) return;
+    constexpr int CPT = 3;
+    const size_t lds = (size_t)CPT * rw * 2 * Lc * sizeof(cplx_t<R>);   // per wavefront
+    const int JJ = (rw * 2 * Lp + 63) / 64;
+    if ((rw != 1 && rw != 2 && rw != 4) || JJ > (rw == 2 ? 6 : 4) || lds > 64 * 1024)
+        throw std::invalid_argument("separable interpolation: rows per wavefront out of range");
+    int G = std::min(4, ncur);   // wavefronts (column groups) per workgroup
+    while (G > 1 && G * lds > 64 * 1024) G /= 2;
+    const int ncb = ncur / G;
+    const unsigned grid = (unsigned)nparent * ((Lp + rw - 1) / rw) * ncb;
+#define M2MR(RW, J)                                                                                                   \
+    k_m2m_row<R, CPT, RW, J><<<grid, 64 * G, G * lds, st>>>(ncur, Lp, Lc, ncb, son_ptr, son_idx, octant_child,        \
+                                                            win_ptr, win_row, win_w, ph_tap, ph_w, shift_up,          \
+                                                            Sm_child, Sm_parent)
+    if (rw == 4) {
+        if (JJ <= 2) M2MR(4, 2);
+        else if (JJ == 3) M2MR(4, 3);
+        else M2MR(4, 4);
+    } else if (rw == 2) {
+        if (JJ <= 3) M2MR(2, 3);
+        else if (JJ == 4) M2MR(2, 4);
+        else M2MR(2, 6);
     } else {
-        throw std::invalid_argument("FP64 far field: at most 8 workspace currents per pass");
+        M2MR(1, 4);
     }
-#undef M2MS_J
-#undef M2MS
-    return true;
+#undef M2MR
 }
 
 // Anterpolation from the parent level as a separable pass (the transpose of
-// k_m2m_sep): for box b with parent P and octant o, child sample (i, j) gets
+// k_m2m_row): for box b with parent P and octant o, child sample (i, j) gets
 //   sum over (parent row ip, wt) with th_tap[ip][a] = i, (parent column jp, wp)
 //   with ph_tap[jp][b] = j of  wt wp shift_o(ip, jp) P(ip, jp),
 // the same products as the fused gather (Code/ProcessMLFMM.h:152-202) with the
-// sums regrouped (theta first, into LDS), which changes only rounding.  A
-// workgroup takes RW consecutive child rows of one box; the theta pass goes
-// row by row with lanes over parent columns, the phi pass has lanes over
-// (row, child column) pairs and adds into Bm (the translation wrote it before).
-template <typename R, int NC, int CPT, int JJ>
-__global__ __launch_bounds__(64 * NC * 3 / CPT) void k_l2l_sep(int Lp, int Lc, int RW, const int* __restrict__ parent,
-                                                        const int* __restrict__ oct, const int* __restrict__ at_ptr,
-                                                        const int* __restrict__ at_idx, const R* __restrict__ at_w,
-                                                        const int* __restrict__ ap_ptr, const int* __restrict__ ap_idx,
-                                                        const R* __restrict__ ap_w, const cplx_t<R>* __restrict__ shdn,
-                                                        const cplx_t<R>* __restrict__ Bmp, cplx_t<R>* __restrict__ Bm) {
+// sums regrouped (theta first), which changes only rounding; it adds into Bm,
+// which the translation wrote before.  A wavefront takes RW child rows of one
+// box and CPT of the nc x 3 columns.  Theta: its lanes run over the parent's
+// columns and it walks the window of parent rows that touch its child rows
+// (win_*: per group of RW rows the parent rows, ascending, with RW weights
+// each), so every parent sample is loaded and shifted once per group and
+// added to the RW rows in registers, the next row's loads in flight.  (Child
+// row by child row, each parent sample was loaded three times behind scalar
+// table loads: C5, 64 right-hand sides, 6.0 ms per matvec, now 4.5.)  Phi: the
+// rows go through the wavefront's own LDS (no barrier), lanes over (row, child
+// column) pairs, MT taps per child column padded with weight 0.
+template <typename R, int CPT, int RW, int MT>
+__global__ __launch_bounds__(256) void k_l2l_row(int nc, int Lp, int Lc, int ncb, const int* __restrict__ parent,
+                                                 const int* __restrict__ oct, const int* __restrict__ win_ptr,
+                                                 const int* __restrict__ win_row, const R* __restrict__ win_w,
+                                                 const int* __restrict__ ap_tap, const R* __restrict__ ap_w,
+                                                 const cplx_t<R>* __restrict__ shdn,
+                                                 const cplx_t<R>* __restrict__ Bmp, cplx_t<R>* __restrict__ Bm) {
     using C = cplx_t<R>;
     extern __shared__ __align__(16) unsigned char l2l_lds[];
     const int pfn = 2 * Lp, psn = 2 * Lc, Kp = Lp * pfn, Kc = Lc * psn;
     const int nrg = (Lc + RW - 1) / RW;   // row groups per box
     const int lin = xcd_remap(blockIdx.x, (int)gridDim.x);
-    const int b = lin / nrg, r0 = (lin % nrg) * RW;   // the row groups of one box are consecutive
-    const int nr = min(RW, Lc - r0);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int c0 = wave * CPT;
-    const int us = RW * pfn;                                             // one column's block
-    C* V = reinterpret_cast<C*>(l2l_lds) + (size_t)wave * CPT * us;    // this wavefront's [CPT][RW][2 Lp]
-    const C* P = Bmp + ((size_t)parent[b] * NC * 3 + c0) * Kp;
+    const int cb = lin % ncb, g = (lin / ncb) % nrg, b = lin / (ncb * nrg);   // one box's workgroups are consecutive
+    const int r0 = g * RW, nr = min(RW, Lc - r0);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int c0 = (cb * (int)(blockDim.x >> 6) + wave) * CPT;
+    C* V = reinterpret_cast<C*>(l2l_lds) + (size_t)wave * CPT * RW * pfn;   // [CPT][RW][2 Lp]
+    const C* P = Bmp + ((size_t)parent[b] * nc * 3 + c0) * Kp;
     const C* sh = shdn + (size_t)oct[b] * Kp;
-    // rows one after another, so a row's taps are the same for every lane
-    // (scalar loads) and each parent sample load depends on nothing per lane
-    for (int r = 0; r < nr; ++r) {
-        const int k0 = at_ptr[r0 + r], k1 = at_ptr[r0 + r + 1];
-        for (int jp = lane; jp < pfn; jp += 64) {
-            C acc[CPT];
+    const int k0 = win_ptr[g], k1 = win_ptr[g + 1];
+    for (int jb = 0; jb < pfn; jb += 64) {
+        const int jp = min(jb + lane, pfn - 1);
+        C acc[RW][CPT];
 #pragma unroll
-            for (int d = 0; d < CPT; ++d) acc[d] = C{0, 0};
-            for (int k = k0; k < k1; ++k) {
-                const int kp = at_idx[k] * pfn + jp;
-                const R w = at_w[k];
-                C e = sh[kp];
-                e.x *= w;
-                e.y *= w;
+        for (int r = 0; r < RW; ++r)
 #pragma unroll
-                for (int d = 0; d < CPT; ++d) cfma(acc[d], e, P[(size_t)d * Kp + kp]);
-            }
+            for (int d = 0; d < CPT; ++d) acc[r][d] = C{0, 0};
+        auto load = [&](int k, C& e, C (&v)[CPT]) {
+            const int kp = win_row[min(k, k1 - 1)] * pfn + jp;
+            e = sh[kp];
 #pragma unroll
-            for (int d = 0; d < CPT; ++d) V[d * us + r * pfn + jp] = acc[d];
-        }
-    }
-    __syncthreads();
-    C* O = Bm + ((size_t)b * NC * 3 + c0) * Kc + (size_t)r0 * psn;
+            for (int d = 0; d < CPT; ++d) v[d] = P[(size_t)d * Kp + kp];
+        };
+        auto add = [&](int k, const C& e, const C (&v)[CPT]) {
+            R w[RW];
 #pragma unroll
-    for (int jj = 0; jj < JJ; ++jj) {
-        const int t = lane + 64 * jj;
-        if (t < nr * psn) {
-            const int r = t / psn, jc = t - r * psn;
-            C s[CPT];
-#pragma unroll
-            for (int d = 0; d < CPT; ++d) s[d] = C{0, 0};
-            for (int k = ap_ptr[jc]; k < ap_ptr[jc + 1]; ++k) {
-                const int vi = r * pfn + ap_idx[k];
-                const R w = ap_w[k];
-#pragma unroll
-                for (int d = 0; d < CPT; ++d) {
-                    const C v = V[d * us + vi];
-                    s[d].x += w * v.x;
-                    s[d].y += w * v.y;
-                }
-            }
+            for (int r = 0; r < RW; ++r) w[r] = win_w[(size_t)k * RW + r];
 #pragma unroll
             for (int d = 0; d < CPT; ++d) {
-                C o = O[(size_t)d * Kc + t];
-                o.x += s[d].x;
-                o.y += s[d].y;
-                O[(size_t)d * Kc + t] = o;
+                const C t = cmul(e, v[d]);
+#pragma unroll
+                for (int r = 0; r < RW; ++r) {
+                    acc[r][d].x = fma(w[r], t.x, acc[r][d].x);
+                    acc[r][d].y = fma(w[r], t.y, acc[r][d].y);
+                }
             }
+        };
+        C ea, eb, va[CPT], vb[CPT];
+        load(k0, ea, va);
+        for (int k = k0; k < k1; k += 2) {
+            load(k + 1, eb, vb);
+            __builtin_amdgcn_sched_barrier(0);
+            add(k, ea, va);
+            load(k + 2, ea, va);
+            __builtin_amdgcn_sched_barrier(0);
+            if (k + 1 < k1) add(k + 1, eb, vb);
+        }
+        if (jb + lane < pfn)
+#pragma unroll
+            for (int d = 0; d < CPT; ++d)
+#pragma unroll
+                for (int r = 0; r < RW; ++r) V[(d * RW + r) * pfn + jp] = acc[r][d];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // other lanes of this wavefront wrote V
+    C* O = Bm + ((size_t)b * nc * 3 + c0) * Kc + (size_t)r0 * psn;
+    for (int t = lane; t < nr * psn; t += 64) {
+        const int r = t / psn, jc = t - r * psn;
+        C o[CPT];
+#pragma unroll
+        for (int d = 0; d < CPT; ++d) o[d] = O[(size_t)d * Kc + t];
+        int ti[MT];
+        R tw[MT];
+#pragma unroll
+        for (int k = 0; k < MT; ++k) {
+            ti[k] = r * pfn + ap_tap[k * psn + jc];
+            tw[k] = ap_w[k * psn + jc];
+        }
+#pragma unroll
+        for (int d = 0; d < CPT; ++d) {
+            C s = C{0, 0};
+#pragma unroll
+            for (int k = 0; k < MT; ++k) {
+                const C v = V[d * RW * pfn + ti[k]];
+                s.x = fma(tw[k], v.x, s.x);
+                s.y = fma(tw[k], v.y, s.y);
+            }
+            o[d].x += s.x;
+            o[d].y += s.y;
+            O[(size_t)d * Kc + t] = o[d];
         }
     }
 }
 
-// child rows per workgroup: as many as fit 64 KB of LDS (the theta pass's rows
-// of every column) and 256 outputs per lane group (JJ <= 4); 0 if none fits
-int l2l_sep_rows(int ncur, int Lp, int Lc, size_t csize) {
-    const size_t row_lds = (size_t)ncur * 3 * 2 * Lp * csize;
-    if (row_lds > 64 * 1024 || 2 * Lc > 256) return 0;
-    return std::max(1, std::min({Lc, (int)(64 * 1024 / row_lds), 256 / (2 * Lc)}));
+// Child rows per group and the LDS of one wavefront (3 columns, FP64) decide
+// whether the pass applies: 4 rows up to 2 Lp = 340, 2 up to 682, else none
+// (0: the translation then fuses the anterpolation), and at most 8 taps.
+int l2l_rows(int Lp, int taps) {
+    if (taps > 8) return 0;
+    const size_t row = (size_t)3 * 2 * Lp * sizeof(double2);
+    return 4 * row <= 64 * 1024 ? 4 : (2 * row <= 64 * 1024 ? 2 : 0);
 }
 
+// taps that the phi pass is compiled for
+int l2l_taps(int rw, int taps) { return rw == 2 || taps > 6 ? 8 : std::max(taps, 5); }
+
 template <typename R>
-void launch_l2l_sep(hipStream_t st, int ncur, int nbox, int Lp, int Lc, int rw, const int* parent, const int* oct,
-                    const int* at_ptr, const int* at_idx, const R* at_w, const int* ap_ptr, const int* ap_idx,
+void launch_l2l_row(hipStream_t st, int ncur, int nbox, int Lp, int Lc, int rw, int taps, const int* parent,
+                    const int* oct, const int* win_ptr, const int* win_row, const R* win_w, const int* ap_tap,
                     const R* ap_w, const cplx_t<R>* shift_dn, const cplx_t<R>* Bm_parent, cplx_t<R>* Bm) {
     if (nbox == 0) return;
-    const int JJ = (rw * 2 * Lc + 63) / 64;
-    if (rw < 1 || rw > Lc || JJ > 4 || (size_t)ncur * 3 * 2 * Lp * sizeof(cplx_t<R>) * rw > 64 * 1024)
-        throw std::invalid_argument("separable anterpolation: rows per workgroup out of range");
-    const size_t lds = (size_t)ncur * 3 * 2 * Lp * sizeof(cplx_t<R>) * rw;
-    const unsigned grid = (unsigned)nbox * ((Lc + rw - 1) / rw);
-#define L2LS(NC, CPT, J)                                                                                              \
-    k_l2l_sep<R, NC, CPT, J><<<grid, 64 * NC * 3 / CPT, lds, st>>>(Lp, Lc, rw, parent, oct, at_ptr, at_idx, at_w,    \
-                                                                    ap_ptr, ap_idx, ap_w, shift_dn, Bm_parent, Bm)
-#define L2LS_J(NC, CPT)                                                                                               \
-    if (JJ == 1) L2LS(NC, CPT, 1);                                                                                    \
-    else if (JJ == 2) L2LS(NC, CPT, 2);                                                                               \
-    else if (JJ == 3) L2LS(NC, CPT, 3);                                                                               \
-    else L2LS(NC, CPT, 4);
-    if (ncur == 1) {
-        L2LS_J(1, 3)
-    } else if (ncur == 2) {
-        L2LS_J(2, 3)
-    } else if (ncur == 4) {
-        L2LS_J(4, 3)
-    } else if (ncur == 8) {
-        L2LS_J(8, 3)
-    } else if constexpr (sizeof(R) == 4) {
-        L2LS_J(16, 6)
-    } else {
-        throw std::invalid_argument("FP64 far field: at most 8 workspace currents per pass");
-    }
-#undef L2LS_J
-#undef L2LS
+    constexpr int CPT = 3;
+    const size_t lds = (size_t)CPT * rw * 2 * Lp * sizeof(cplx_t<R>);   // per wavefront
+    if ((rw != 2 && rw != 4) || lds > 64 * 1024 || taps != l2l_taps(rw, taps))
+        throw std::invalid_argument("separable anterpolation: rows per wavefront out of range");
+    int G = std::min(4, ncur);   // wavefronts (column groups) per workgroup
+    while (G > 1 && G * lds > 64 * 1024) G /= 2;
+    const int ncb = ncur / G;
+    const unsigned grid = (unsigned)nbox * ((Lc + rw - 1) / rw) * ncb;
+#define L2LR(RW, MT)                                                                                                  \
+    k_l2l_row<R, CPT, RW, MT><<<grid, 64 * G, G * lds, st>>>(ncur, Lp, Lc, ncb, parent, oct, win_ptr, win_row, win_w, \
+                                                             ap_tap, ap_w, shift_dn, Bm_parent, Bm)
+    if (rw == 2) L2LR(2, 8);
+    else if (taps == 5) L2LR(4, 5);
+    else if (taps == 6) L2LR(4, 6);
+    else L2LR(4, 8);
+#undef L2LR
 }
 
 // ---------------------------------------------------------------- translation + anterpolation
@@ -1355,17 +1396,17 @@ void launch_narrow(hipStream_t st, size_t n, const double2* in, float2* out) {
                                          const cplx_t<R>*, const cplx_t<R>*, double2, double2*);                  \
     template void launch_disagg_pmchwt_b<R>(hipStream_t, int, int, int, const int*, const int*,                    \
                                             const PmchwtFarArgs<R>&, double2*);                                   \
-    template bool launch_m2m_sep<R>(hipStream_t, int, int, int, int, const int*, const int*, const int*, const int*, \
-                                    const R*, const int*, const R*, const cplx_t<R>*, const cplx_t<R>*,           \
-                                    cplx_t<R>*);                                                                  \
+    template void launch_m2m_row<R>(hipStream_t, int, int, int, int, int, const int*, const int*, const int*,      \
+                                    const int*, const int*, const R*, const int*, const R*, const cplx_t<R>*,     \
+                                    const cplx_t<R>*, cplx_t<R>*);                                                \
     template void launch_m2l_cls<R>(hipStream_t, int, int, int, const int*, const int*, const int*, const int*,      \
                                     const cplx_t<R>*, const cplx_t<R>*, int, const int*, const int*, const int*,  \
                                     const int*, const R*, const cplx_t<R>*, const cplx_t<R>*, cplx_t<R>*);        \
     template void launch_m2l_cl<R>(hipStream_t, int, int, int, int, const int*, const int*, const int*, const int*,  \
                                    const cplx_t<R>*, const cplx_t<R>*, int, const int*, const int*, const int*,   \
                                    const int*, const R*, const cplx_t<R>*, const cplx_t<R>*, cplx_t<R>*);       \
-    template void launch_l2l_sep<R>(hipStream_t, int, int, int, int, int, const int*, const int*, const int*,        \
-                                    const int*, const R*, const int*, const int*, const R*, const cplx_t<R>*,     \
+    template void launch_l2l_row<R>(hipStream_t, int, int, int, int, int, int, const int*, const int*, const int*,  \
+                                    const int*, const R*, const int*, const R*, const cplx_t<R>*,                 \
                                     const cplx_t<R>*, cplx_t<R>*);
 MLFMA_FAR_INSTANTIATE(double)
 MLFMA_FAR_INSTANTIATE(float)

@@ -38,24 +38,28 @@ void launch_m2m(hipStream_t st, int ncur, int nparent, int Kp, int Kc, const int
                 const int* octant_child, const int* tap, const R* w, const cplx_t<R>* shift_up, const cplx_t<R>* Sm_child,
                 cplx_t<R>* Sm_parent);
 
-// Separable (theta, then phi) form of launch_m2m from the direction tables of
-// the stencil; returns false when it does not apply (the caller then runs
-// launch_m2m).
+// Separable (theta, then phi) form of launch_m2m: m2m_rows gives the parent
+// rows per group (0 when it does not apply; the caller then runs launch_m2m),
+// win_* are the row_windows of the theta stencil, ph_* the phi stencil.
+int m2m_rows(int Lp, int Lc);
 template <typename R>
-bool launch_m2m_sep(hipStream_t st, int ncur, int nparent, int Lp, int Lc, const int* son_ptr, const int* son_idx,
-                    const int* octant_child, const int* th_tap, const R* th_w, const int* ph_tap, const R* ph_w,
-                    const cplx_t<R>* shift_up, const cplx_t<R>* Sm_child, cplx_t<R>* Sm_parent);
+void launch_m2m_row(hipStream_t st, int ncur, int nparent, int Lp, int Lc, int rw, const int* son_ptr,
+                    const int* son_idx, const int* octant_child, const int* win_ptr, const int* win_row,
+                    const R* win_w, const int* ph_tap, const R* ph_w, const cplx_t<R>* shift_up,
+                    const cplx_t<R>* Sm_child, cplx_t<R>* Sm_parent);
 
 // Separable anterpolation, after the translation of a level: for every box of
 // the level, Bm += the parent's local expansion shifted to the box and
-// anterpolated through the transposed direction stencils (theta rows into
-// LDS, then phi).  l2l_sep_rows gives the child rows per workgroup that fit
-// (0 when the pass does not apply; the translation then fuses the
-// anterpolation).
-int l2l_sep_rows(int ncur, int Lp, int Lc, size_t csize);
+// anterpolated through the transposed direction stencils.  l2l_rows: child
+// rows per group (0 when the pass does not apply; the translation then fuses
+// the anterpolation).  win_*: row_windows of the transposed theta stencil;
+// ap_tap / ap_w: the transposed phi stencil as [taps][2 Lc], padded with weight
+// 0 to the taps that l2l_taps gives.
+int l2l_rows(int Lp, int taps);
+int l2l_taps(int rw, int taps);
 template <typename R>
-void launch_l2l_sep(hipStream_t st, int ncur, int nbox, int Lp, int Lc, int rw, const int* parent, const int* oct,
-                    const int* at_ptr, const int* at_idx, const R* at_w, const int* ap_ptr, const int* ap_idx,
+void launch_l2l_row(hipStream_t st, int ncur, int nbox, int Lp, int Lc, int rw, int taps, const int* parent,
+                    const int* oct, const int* win_ptr, const int* win_row, const R* win_w, const int* ap_tap,
                     const R* ap_w, const cplx_t<R>* shift_dn, const cplx_t<R>* Bm_parent, cplx_t<R>* Bm);
 
 // Bm[b][..][q] = sum_dr TFw[vec][q] * Sm[dr][..][q]

@@ -112,6 +112,15 @@ struct Medium {
 };
 
 // ------------------------------------------------------------------ builders (host)
+// Windows of a row stencil (CSR: row r takes source rows idx[ptr[r]..] with
+// weights w): per group of rw consecutive rows the source rows that any of them
+// takes, ascending, with rw weights each (0 where a row does not take it).
+void row_windows(const std::vector<int>& ptr, const std::vector<int>& idx, const std::vector<double>& w, int rw,
+                 std::vector<int>& win_ptr, std::vector<int>& win_row, std::vector<double>& win_w);
+// The same stencil as [taps][rows], padded with (idx 0, weight 0); taps is the
+// largest row's count, at least `least`.
+int padded_taps(const std::vector<int>& ptr, const std::vector<int>& idx, const std::vector<double>& w, int least,
+                std::vector<int>& tap, std::vector<double>& tw);
 int read_nas(const std::string& path, std::vector<int>& ids, std::vector<double>& xyz, std::vector<int>& fids,
              std::vector<int>& fvid, std::string& err);
 bool build_mesh(int np, const int* ids, const double* xyz, int nf, const int* fids, const int* fvid, Mesh& m,

@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <map>
 
 #include "mlfma.h"
 #include "model.hpp"
@@ -187,6 +188,43 @@ static void stencil(double t, const std::vector<double>& a, int out[3]) {
 
 static double lagrange(double x0, double x1, double x2, double x3) {
     return ((x0 - x2) * (x0 - x3)) / ((x1 - x2) * (x1 - x3));
+}
+
+void row_windows(const std::vector<int>& ptr, const std::vector<int>& idx, const std::vector<double>& w, int rw,
+                 std::vector<int>& win_ptr, std::vector<int>& win_row, std::vector<double>& win_w) {
+    const int rows = (int)ptr.size() - 1;
+    win_ptr.assign(1, 0);
+    win_row.clear();
+    win_w.clear();
+    for (int r0 = 0; r0 < rows; r0 += rw) {
+        std::map<int, std::vector<double>> window;
+        for (int r = r0; r < std::min(rows, r0 + rw); ++r)
+            for (int k = ptr[r]; k < ptr[r + 1]; ++k) {
+                std::vector<double>& v = window[idx[k]];
+                v.resize(rw, 0.0);
+                v[r - r0] += w[k];
+            }
+        for (const auto& e : window) {
+            win_row.push_back(e.first);
+            win_w.insert(win_w.end(), e.second.begin(), e.second.end());
+        }
+        win_ptr.push_back((int)win_row.size());
+    }
+}
+
+int padded_taps(const std::vector<int>& ptr, const std::vector<int>& idx, const std::vector<double>& w, int least,
+                std::vector<int>& tap, std::vector<double>& tw) {
+    const int rows = (int)ptr.size() - 1;
+    int taps = least;
+    for (int r = 0; r < rows; ++r) taps = std::max(taps, ptr[r + 1] - ptr[r]);
+    tap.assign((size_t)taps * rows, 0);
+    tw.assign((size_t)taps * rows, 0.0);
+    for (int r = 0; r < rows; ++r)
+        for (int k = ptr[r]; k < ptr[r + 1]; ++k) {
+            tap[(size_t)(k - ptr[r]) * rows + r] = idx[k];
+            tw[(size_t)(k - ptr[r]) * rows + r] = w[k];
+        }
+    return taps;
 }
 
 void build_wave_tables(const Octree& t, cplx k, double kabs, int tf_mode, WaveTables& W) {
