@@ -146,11 +146,9 @@ int mlfma_set_graphs(mlfma_handle* h, int on);
  * vector units and the translation by sibling clusters or per box; keeps the
  * choice for this handle.  out4 = {rhs per pass, choice bits (bit 0 near on
  * the matrix cores, bit 1 disaggregation on the matrix cores, bit 2 cluster
- * translation, bit 3 cluster translation with 12 workspace columns per thread
- * (FP32), bit 4 cluster translation over every child of a parent (up to 8)
- * with the members' translation samples staged in LDS (FP32; takes precedence
- * over bit 3)), ms per batched matvec of the choice, ms of the slowest
- * configuration timed}.  No reference counterpart. */
+ * translation, bit 4 cluster translation over every child of a parent (up to
+ * 8) with the members' translation samples staged in LDS (FP32)), ms per
+ * batched matvec of the choice, ms of the slowest configuration timed}.  No reference counterpart. */
 int mlfma_autotune(mlfma_handle* h, int nrhs, int precision, double* out4);
 
 /* Sets the launch configuration directly (e.g. one that mlfma_autotune chose
@@ -159,9 +157,9 @@ int mlfma_autotune(mlfma_handle* h, int nrhs, int precision, double* out4);
  * choice bits of mlfma_autotune's out4[1]: bit 0 near field on the matrix
  * cores, bit 1 disaggregation on the matrix cores, bit 2 translation by
  * sibling clusters (up to 4 children of one parent share each source box,
- * read once), bit 3 12 instead of 6 workspace columns per thread in the FP32
- * cluster translation, bit 4 FP32 cluster translation over every child of a
- * parent with LDS-staged translation samples (takes precedence over bit 3).
+ * read once), bit 3 accepted without effect (earlier configurations hold it),
+ * bit 4 FP32 cluster translation over every child of a parent with LDS-staged
+ * translation samples.
  * No reference counterpart. */
 int mlfma_set_tuning(mlfma_handle* h, int precision, int rhs_per_pass, int bits);
 

@@ -781,12 +781,12 @@ void Engine::translate(int w, int l, int nc) {
     // (gather over the 9-tap stencil's transpose) or as a separable pass after it
     const bool sep = l > 2 && l2l_separable_ && D.dn_rows[l] > 0;
     const bool up = l > 2 && !sep;
-    if (m2l_cluster_ && m2l_variant_ == 2 && std::is_same<R, float>::value && (nc == 4 || nc == 8 || nc == 16))
+    if (m2l_cluster_ && m2l_staged_ && std::is_same<R, float>::value && (nc == 4 || nc == 8 || nc == 16))
         launch_m2l_cls<R>(st, nc, v.ncl8, D.K[l], v.cl8_child, v.cl8_ptr, v.cl8_src, v.cl8_vec, F.TFw[l], F.Sm[l],
                           up ? D.K[l - 1] : 0, v.parent, v.oct, D.t_ptr[l], D.t_kp[l], F.t_w[l], F.sh_dn[l],
                           up ? F.Bm[l - 1] : nullptr, F.Bm[l]);
     else if (m2l_cluster_)
-        launch_m2l_cl<R>(st, m2l_variant_, nc, v.ncl, D.K[l], v.cl_child, v.cl_ptr, v.cl_src, v.cl_vec, F.TFw[l], F.Sm[l],
+        launch_m2l_cl<R>(st, nc, v.ncl, D.K[l], v.cl_child, v.cl_ptr, v.cl_src, v.cl_vec, F.TFw[l], F.Sm[l],
                          up ? D.K[l - 1] : 0, v.parent, v.oct, D.t_ptr[l], D.t_kp[l], F.t_w[l], F.sh_dn[l],
                          up ? F.Bm[l - 1] : nullptr, F.Bm[l]);
     else
@@ -1217,7 +1217,7 @@ void Engine::autotune(int R, int prec, double* out) {
         near_mfma_ = (m & 1) != 0;
         disagg_mfma_ = (m & 2) != 0;
         m2l_cluster_ = (m & 4) != 0;
-        m2l_variant_ = (m & 16) ? 2 : ((m & 8) ? 1 : 0);
+        m2l_staged_ = (m & 16) != 0;
         rb_tuned_[f32 ? 1 : 0] = rb;
         float ms = 0;
         MLFMA_HIP(hipEventRecord(a, st));
@@ -1245,12 +1245,11 @@ void Engine::autotune(int R, int prec, double* out) {
         const double t = time(best_rb, best_m ^ bit);
         if (t < best) best = t, best_m ^= bit;
     }
-    if (f32 && (best_m & 4))   // the cluster translation's forms: two samples (start), twelve columns, six
-        for (int v : {8, 0}) {
-            const int m = (best_m & ~24) | v;
-            const double t = time(best_rb, m);
-            if (t < best) best = t, best_m = m;
-        }
+    if (f32 && (best_m & 4)) {   // the cluster translation's forms: all-sibling LDS-staged (start), four children
+        const int m = best_m & ~16;
+        const double t = time(best_rb, m);
+        if (t < best) best = t, best_m = m;
+    }
     for (int rb = rbmax / 2; rb >= std::max(1, rbmax / 4); rb /= 2) {
         const double t = time(rb, best_m);
         if (t < best) best = t, best_rb = rb;
@@ -1262,7 +1261,7 @@ void Engine::autotune(int R, int prec, double* out) {
     near_mfma_ = (best_m & 1) != 0;
     disagg_mfma_ = (best_m & 2) != 0;
     m2l_cluster_ = (best_m & 4) != 0;
-    m2l_variant_ = (best_m & 16) ? 2 : ((best_m & 8) ? 1 : 0);
+    m2l_staged_ = (best_m & 16) != 0;
     clear_graphs();   // recorded sequences follow the tuned configuration
     if (out) out[0] = best_rb, out[1] = best_m, out[2] = best, out[3] = worst;
 }
@@ -1274,7 +1273,7 @@ void Engine::set_tuning(int prec, int rb, int bits) {
     near_mfma_ = (bits & 1) != 0;
     disagg_mfma_ = (bits & 2) != 0;
     m2l_cluster_ = (bits & 4) != 0;
-    m2l_variant_ = (bits & 16) ? 2 : ((bits & 8) ? 1 : 0);
+    m2l_staged_ = (bits & 16) != 0;
     clear_graphs();
 }
 

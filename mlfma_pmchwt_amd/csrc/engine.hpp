@@ -385,7 +385,7 @@ private:
     bool m2l_cluster_ = true;   // translation by sibling clusters
     bool m2m_separable_ = true;  // interpolation: separable (theta, then phi) form where it applies
     bool l2l_separable_ = true;  // anterpolation: separable pass after the translation where it applies
-    int m2l_variant_ = 0;       // FP32 cluster translation: 1 twelve columns per thread, 2 all-sibling clusters, LDS-staged samples
+    bool m2l_staged_ = false;   // FP32 cluster translation by all-sibling clusters with LDS-staged samples
     double2* d_Dinv_ = nullptr;
     long long* d_Doff_ = nullptr;
 };

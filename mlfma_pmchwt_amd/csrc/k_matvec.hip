@@ -698,10 +698,25 @@ void launch_m2l_l2l(hipStream_t st, int ncur, int nbox, int K, const int* dr_ptr
 // list reads the all-zero row the table keeps after its last vector, so the
 // member loop has no branches (a member's sum thus runs over its own list in
 // ascending box order, plus exact zeros).  The interpolation from the parent
-// reads each parent value once for all members.  G = nc x 3 / CPT wavefronts
-// per workgroup, one per column group; no LDS and no barriers.
-template <typename R, int NC, int G, int NM>
-__device__ __forceinline__ void m2l_cl_body(int cl, int K, int q, int c0, const int* __restrict__ cl_child,
+// reads each parent value once for all members.  No LDS and no barriers.
+// SP = 2 (FP32): a lane owns two neighbouring samples and loads both with one
+// 16-byte load.  An 8-byte load keeps the L1 busy as long as a 16-byte one (16
+// against 18 to 20 cycles per wavefront and CU, measured on 64 consecutive
+// values), and that data path bounds this kernel.
+template <typename R, int SP>
+struct SampleVec {
+    using type = cplx_t<R>;
+};
+template <>
+struct SampleVec<float, 2> {
+    using type = float4;
+};
+__device__ __forceinline__ float2 sample_of(float4 v, int s) { return s ? make_float2(v.z, v.w) : make_float2(v.x, v.y); }
+__device__ __forceinline__ float2 sample_of(float2 v, int) { return v; }
+__device__ __forceinline__ double2 sample_of(double2 v, int) { return v; }
+
+template <typename R, int CPT, int SP, int NM>
+__device__ __forceinline__ void m2l_cl_body(int nc, int cl, int K, int q, int c0, const int* __restrict__ cl_child,
                                             const int* __restrict__ cl_ptr, const int* __restrict__ cl_src,
                                             const int* __restrict__ cl_vec, const cplx_t<R>* __restrict__ TFw,
                                             const cplx_t<R>* __restrict__ Sm, int Kp, const int* __restrict__ parent,
@@ -710,34 +725,38 @@ __device__ __forceinline__ void m2l_cl_body(int cl, int K, int q, int c0, const 
                                             const cplx_t<R>* __restrict__ shdn, const cplx_t<R>* __restrict__ Bmp,
                                             cplx_t<R>* __restrict__ Bm) {
     using C = cplx_t<R>;
-    constexpr int CPT = NC * 3 / G;
+    using V = typename SampleVec<R, SP>::type;   // SP samples (q is a multiple of SP, K is even: aligned)
     int child[NM];
 #pragma unroll
     for (int k = 0; k < NM; ++k) child[k] = cl_child[cl * 4 + k];
-    C acc[NM][CPT];
+    C acc[NM][CPT][SP];
 #pragma unroll
     for (int k = 0; k < NM; ++k)
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) acc[k][j] = C{0, 0};
+        for (int j = 0; j < CPT; ++j)
+#pragma unroll
+            for (int p = 0; p < SP; ++p) acc[k][j][p] = C{0, 0};
     const int u0 = cl_ptr[cl], u1 = cl_ptr[cl + 1];
     // software pipeline over two register sets: the next source's values and
     // its members' translation samples are loaded into one set while the
     // other is applied
-    C sa[CPT], sb[CPT], ta[NM], tb[NM];
-    auto fetch = [&](C (&s)[CPT], C (&t)[NM], int u) {
+    V sa[CPT], sb[CPT], ta[NM], tb[NM];
+    auto fetch = [&](V (&s)[CPT], V (&t)[NM], int u) {
         const int4 v = *reinterpret_cast<const int4*>(cl_vec + (size_t)u * 4);
         const int vk[4] = {v.x, v.y, v.z, v.w};
-        const C* S = Sm + ((size_t)cl_src[u] * NC * 3 + c0) * K + q;
+        const C* S = Sm + ((size_t)cl_src[u] * nc * 3 + c0) * K + q;
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) s[j] = S[(size_t)j * K];
+        for (int j = 0; j < CPT; ++j) s[j] = *reinterpret_cast<const V*>(S + (size_t)j * K);
 #pragma unroll
-        for (int k = 0; k < NM; ++k) t[k] = TFw[(size_t)vk[k] * K + q];
+        for (int k = 0; k < NM; ++k) t[k] = *reinterpret_cast<const V*>(TFw + (size_t)vk[k] * K + q);
     };
-    auto apply = [&](const C (&s)[CPT], const C (&t)[NM]) {
+    auto apply = [&](const V (&s)[CPT], const V (&t)[NM]) {
 #pragma unroll
         for (int k = 0; k < NM; ++k)
 #pragma unroll
-            for (int j = 0; j < CPT; ++j) cmac(acc[k][j], t[k], s[j]);
+            for (int j = 0; j < CPT; ++j)
+#pragma unroll
+                for (int p = 0; p < SP; ++p) cmac(acc[k][j][p], sample_of(t[k], p), sample_of(s[j], p));
     };
     // Sources go in pairs, so that every apply has the other set's loads in
     // flight; the prefetch after a pair is unconditional (the last source is
@@ -756,31 +775,39 @@ __device__ __forceinline__ void m2l_cl_body(int cl, int K, int q, int c0, const 
     }
     if (u < u1) apply(sa, ta);
     if (Bmp != nullptr) {
-        const C* P = Bmp + ((size_t)parent[child[0]] * NC * 3 + c0) * Kp;   // siblings share the parent
+        const C* P = Bmp + ((size_t)parent[child[0]] * nc * 3 + c0) * Kp;   // siblings share the parent
         const C* sh[NM];
 #pragma unroll
         for (int k = 0; k < NM; ++k) sh[k] = shdn + (size_t)oct[child[k]] * Kp;
-        for (int j = t_ptr[q]; j < t_ptr[q + 1]; ++j) {
-            const int kp = t_kp[j];
-            const R w = t_w[j];
-            C pv[CPT];
 #pragma unroll
-            for (int jj = 0; jj < CPT; ++jj) pv[jj] = P[(size_t)jj * Kp + kp];
+        for (int p = 0; p < SP; ++p)
+            for (int j = t_ptr[q + p]; j < t_ptr[q + p + 1]; ++j) {
+                const int kp = t_kp[j];
+                const R w = t_w[j];
+                C pv[CPT];
 #pragma unroll
-            for (int k = 0; k < NM; ++k) {
-                C e = sh[k][kp];
-                e.x *= w;
-                e.y *= w;
+                for (int jj = 0; jj < CPT; ++jj) pv[jj] = P[(size_t)jj * Kp + kp];
 #pragma unroll
-                for (int jj = 0; jj < CPT; ++jj) cfma(acc[k][jj], e, pv[jj]);
+                for (int k = 0; k < NM; ++k) {
+                    C e = sh[k][kp];
+                    e.x *= w;
+                    e.y *= w;
+#pragma unroll
+                    for (int jj = 0; jj < CPT; ++jj) cfma(acc[k][jj][p], e, pv[jj]);
+                }
             }
-        }
     }
 #pragma unroll
     for (int k = 0; k < NM; ++k) {
-        C* o = Bm + ((size_t)child[k] * NC * 3 + c0) * K + q;
+        C* o = Bm + ((size_t)child[k] * nc * 3 + c0) * K + q;
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) o[(size_t)j * K] = acc[k][j];
+        for (int j = 0; j < CPT; ++j) {
+            if constexpr (SP == 2)
+                *reinterpret_cast<V*>(o + (size_t)j * K) =
+                    make_float4(acc[k][j][0].x, acc[k][j][0].y, acc[k][j][SP - 1].x, acc[k][j][SP - 1].y);
+            else
+                o[(size_t)j * K] = acc[k][j][0];
+        }
     }
 }
 
@@ -972,27 +999,39 @@ void launch_m2l_cls(hipStream_t st, int ncur, int ncl, int K, const int* cl_chil
     }
 }
 
-template <typename R, int NC, int G>
-__global__ __launch_bounds__(64 * G) void k_m2l_cl(int ncl, int K, int ktiles, int wc, const int* __restrict__ cl_child,
-                                                   const int* __restrict__ cl_ptr, const int* __restrict__ cl_src,
-                                                   const int* __restrict__ cl_vec, const cplx_t<R>* __restrict__ TFw,
-                                                   const cplx_t<R>* __restrict__ Sm, int Kp,
-                                                   const int* __restrict__ parent, const int* __restrict__ oct,
-                                                   const int* __restrict__ t_ptr, const int* __restrict__ t_kp,
-                                                   const R* __restrict__ t_w, const cplx_t<R>* __restrict__ shdn,
-                                                   const cplx_t<R>* __restrict__ Bmp, cplx_t<R>* __restrict__ Bm) {
-    constexpr int CPT = NC * 3 / G;
-    int cl, kt;
-    window_order(xcd_remap(blockIdx.x, ncl * ktiles), ncl, ktiles, wc, cl, kt);
-    const int c0 = (threadIdx.x >> 6) * CPT;
-    const int q = kt * 64 + (threadIdx.x & 63);
-    if (q >= K) return;
-    // members are packed first; the count is uniform over the workgroup
+// A workgroup's wavefronts take consecutive clusters, all with one sample tile
+// and one group of CPT columns, and the launch goes window by window of wc
+// workgroups: tile, then column group, then clusters.  The wavefronts that run
+// at once on one XCD so read 64 samples x CPT columns of the boxes around wc
+// neighbouring clusters, which its L2 holds, and neighbouring clusters share
+// sources in the L1.  With a cluster's column groups as the wavefronts of one
+// workgroup the tile's boxes took four times that and a quarter of the reads
+// missed the L2: C5 at 64 right-hand sides 30.2 ms per matvec, 29.3 in this
+// order, 27.5 with two samples per lane as well.  What is left is shared by the
+// L1 (10 loads of 18 cycles per source) and the vector unit (192 cycles of FMA).
+template <typename R, int CPT, int SP>
+__global__ __launch_bounds__(256) void k_m2l_cl(int nc, int ncl, int K, int ktiles, int wc,
+                                                const int* __restrict__ cl_child,
+                                                const int* __restrict__ cl_ptr, const int* __restrict__ cl_src,
+                                                const int* __restrict__ cl_vec, const cplx_t<R>* __restrict__ TFw,
+                                                const cplx_t<R>* __restrict__ Sm, int Kp,
+                                                const int* __restrict__ parent, const int* __restrict__ oct,
+                                                const int* __restrict__ t_ptr, const int* __restrict__ t_kp,
+                                                const R* __restrict__ t_w, const cplx_t<R>* __restrict__ shdn,
+                                                const cplx_t<R>* __restrict__ Bmp, cplx_t<R>* __restrict__ Bm) {
+    const int W = blockDim.x >> 6, ncg = nc * 3 / CPT, nq = (ncl + W - 1) / W;
+    int quad, tile;
+    window_order(xcd_remap(blockIdx.x, (int)gridDim.x), nq, ktiles * ncg, wc, quad, tile);
+    const int kt = tile / ncg, c0 = (tile - kt * ncg) * CPT;
+    const int cl = quad * W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = (kt * 64 + (threadIdx.x & 63)) * SP;
+    if (cl >= ncl || q >= K) return;
+    // members are packed first; the count is uniform over the wavefront
     const int4 ch = *reinterpret_cast<const int4*>(cl_child + (size_t)cl * 4);
     const int nm = (ch.y >= 0) + (ch.z >= 0) + (ch.w >= 0) + 1;
 #define M2LB(NM)                                                                                                      \
-    m2l_cl_body<R, NC, G, NM>(cl, K, q, c0, cl_child, cl_ptr, cl_src, cl_vec, TFw, Sm, Kp, parent, oct, t_ptr, t_kp, \
-                              t_w, shdn, Bmp, Bm)
+    m2l_cl_body<R, CPT, SP, NM>(nc, cl, K, q, c0, cl_child, cl_ptr, cl_src, cl_vec, TFw, Sm, Kp, parent, oct, t_ptr,     \
+                            t_kp, t_w, shdn, Bmp, Bm)
     if (nm == 4) M2LB(4);
     else if (nm == 3) M2LB(3);
     else if (nm == 2) M2LB(2);
@@ -1001,41 +1040,39 @@ __global__ __launch_bounds__(64 * G) void k_m2l_cl(int ncl, int K, int ktiles, i
 }
 
 template <typename R>
-void launch_m2l_cl(hipStream_t st, int variant, int ncur, int ncl, int K, const int* cl_child, const int* cl_ptr,
+void launch_m2l_cl(hipStream_t st, int ncur, int ncl, int K, const int* cl_child, const int* cl_ptr,
                    const int* cl_src, const int* cl_vec, const cplx_t<R>* TFw, const cplx_t<R>* Sm, int Kp,
                    const int* parent, const int* octant, const int* t_ptr, const int* t_kp, const R* t_w,
                    const cplx_t<R>* shift_down, const cplx_t<R>* Bm_parent, cplx_t<R>* Bm) {
     if (ncl == 0) return;
-    const int kt = (K + 63) / 64;
-    // windows of 128 clusters: the fetch from memory drops from about 7.6 to
-    // 4.5 times the level's workspaces (the kernel's time does not change)
-    constexpr int wc = 128;
-    // columns per thread: 3 in FP64, 6 in FP32 (3 when there are only 3)
+    if (ncur != 1 && ncur != 2 && ncur != 4 && ncur != 8 && (ncur != 16 || sizeof(R) == 8))
+        throw std::invalid_argument("FP64 far field: at most 8 workspace currents per pass");
+    // Columns x samples per thread.  From 4 currents 6 x 2 in FP32 and 6 x 1 in
+    // FP64 (16-byte loads both): whole matvec of C5 at 64 right-hand sides, FP32:
+    // 6 x 2 27.5 ms, 6 x 1 29.3, 12 x 1 28.5, 3 x 2 28.4, 8 x 2 31.8 (spills into
+    // the accumulator file); FP64 lossy sphere at 13: 6 x 1 5.57, 3 x 1 5.77.
+    // Below 4 the level has too few wavefronts to lose any: PMCHWT of 15k unknowns,
+    // one vector: 401 us as here, 409 with the wide form.
     constexpr bool f64 = sizeof(R) == 8;
-#define M2LC_G(NC, G)                                                                                                 \
-    k_m2l_cl<R, NC, G><<<ncl * kt, 64 * G, 0, st>>>(ncl, K, kt, wc, cl_child, cl_ptr, cl_src, cl_vec, TFw, Sm, Kp, \
-                                                    parent, octant, t_ptr, t_kp, t_w, shift_down, Bm_parent, Bm)
-#define M2LC(NC)                                                                                                      \
-    {                                                                                                                 \
-        if constexpr (!f64 && NC >= 4) {                                                                              \
-            if (variant == 1) {                                                                                       \
-                M2LC_G(NC, NC / 4);                                                                                   \
-            } else {                                                                                                  \
-                M2LC_G(NC, NC / 2);                                                                                   \
-            }                                                                                                         \
-        } else {                                                                                                      \
-            constexpr int G = f64 ? NC : (NC == 1 ? 1 : NC / 2);                                                      \
-            M2LC_G(NC, G);                                                                                            \
-        }                                                                                                             \
-    }
-    if (ncur == 1) M2LC(1)
-    else if (ncur == 2) M2LC(2)
-    else if (ncur == 4) M2LC(4)
-    else if (ncur == 8) M2LC(8)
-    else if constexpr (sizeof(R) == 4) M2LC(16)
-    else throw std::invalid_argument("FP64 far field: at most 8 workspace currents per pass");
+    const bool wide = ncur >= 4;
+    const int sp = !f64 && wide && (K & 1) == 0 ? 2 : 1;   // pairs need rows of whole pairs (K = 2 L^2 is even)
+    const int kt = (K + 64 * sp - 1) / (64 * sp);
+    const int cpt = wide || (!f64 && ncur == 2) ? 6 : 3;
+    const int ncg = ncur * 3 / cpt;
+    // Wavefronts (neighbouring clusters) per workgroup; single ones where a level
+    // does not give each SIMD four wavefronts.
+    const int W = !wide || (long long)ncl * kt * ncg < 4096 ? 1 : 4;
+    const int nq = (ncl + W - 1) / W;
+    // clusters per window: 512 (measured 27.5 at 512 and 1024, 27.9 at 256), 128 below 4 currents
+    const int wc = wide ? 512 / W : 128;
+#define M2LC(CPT, SP)                                                                                                 \
+    k_m2l_cl<R, CPT, SP><<<nq * kt * ncg, 64 * W, 0, st>>>(ncur, ncl, K, kt, wc, cl_child, cl_ptr, cl_src, cl_vec,   \
+                                                           TFw, Sm, Kp, parent, octant, t_ptr, t_kp, t_w,             \
+                                                           shift_down, Bm_parent, Bm)
+    if (cpt == 3) M2LC(3, 1);
+    else if (sp == 1) M2LC(6, 1);
+    else if constexpr (!f64) M2LC(6, 2);
 #undef M2LC
-#undef M2LC_G
 }
 
 // ---------------------------------------------------------------- disaggregation
@@ -1402,7 +1439,7 @@ void launch_narrow(hipStream_t st, size_t n, const double2* in, float2* out) {
     template void launch_m2l_cls<R>(hipStream_t, int, int, int, const int*, const int*, const int*, const int*,      \
                                     const cplx_t<R>*, const cplx_t<R>*, int, const int*, const int*, const int*,  \
                                     const int*, const R*, const cplx_t<R>*, const cplx_t<R>*, cplx_t<R>*);        \
-    template void launch_m2l_cl<R>(hipStream_t, int, int, int, int, const int*, const int*, const int*, const int*,  \
+    template void launch_m2l_cl<R>(hipStream_t, int, int, int, const int*, const int*, const int*, const int*,      \
                                    const cplx_t<R>*, const cplx_t<R>*, int, const int*, const int*, const int*,   \
                                    const int*, const R*, const cplx_t<R>*, const cplx_t<R>*, cplx_t<R>*);       \
     template void launch_l2l_row<R>(hipStream_t, int, int, int, int, int, int, const int*, const int*, const int*,  \
