@@ -378,7 +378,7 @@ private:
     double2* d_iW_ = nullptr;
     double2* d_ipart_ = nullptr;
     double2* d_ismall_ = nullptr;
-    double* d_iscale_ = nullptr;
+    double2* d_ih_ = nullptr;   // every step's coefficients and norms
     int inner_cap_R_ = 0, inner_cap_k_ = 0;
     bool near_mfma_ = true;     // batched near product on the matrix cores (FP32 copy or FP64 entries)
     bool disagg_mfma_ = true;   // batched disaggregation on the matrix cores

@@ -322,6 +322,23 @@ void launch_scale_copy_b(hipStream_t st, int n, int R, const double* a, const do
     k_scale_copy_b<float2><<<(unsigned)((nR + 255) / 256), 256, 0, st>>>(nR, R, a, x, y);
 }
 
+// y[u][r] = x[u][r] / |x_r| with the squared norms n2 where a reduction left
+// them; zero where |x_r| is zero or below eps |v_r| (v2 likewise)
+__global__ void k_unit_copy_b(size_t nR, int R, const double2* __restrict__ n2, const double2* __restrict__ v2,
+                              double eps, const double2* __restrict__ x, double2* __restrict__ y) {
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= nR) return;
+    const int r = (int)(e % R);
+    const double nv = sqrt(n2[r].x), lim = eps * sqrt(v2[r].x);
+    y[e] = cscale(x[e], nv > 0 && !(nv < lim) ? 1.0 / nv : 0.0);
+}
+
+void launch_unit_copy_b(hipStream_t st, int n, int R, const double2* n2, const double2* v2, double eps,
+                        const double2* x, double2* y) {
+    const size_t nR = (size_t)n * R;
+    k_unit_copy_b<<<(unsigned)((nR + 255) / 256), 256, 0, st>>>(nR, R, n2, v2, eps, x, y);
+}
+
 // FP32 -> FP64 (exact)
 __global__ void k_widen(size_t n, const float2* __restrict__ in, double2* __restrict__ out) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -73,6 +73,8 @@ void launch_sub_combination_b(hipStream_t st, int n, int R, int m, const double2
 void launch_add_combination_b(hipStream_t st, int n, int R, int m, const double2* V, size_t ldv, const double2* y,
                               double2* x);
 void launch_scale_copy_b(hipStream_t st, int n, int R, const double* a, const double2* x, double2* y);
+void launch_unit_copy_b(hipStream_t st, int n, int R, const double2* n2, const double2* v2, double eps,
+                        const double2* x, double2* y);
 // the same with an FP32 basis V (FP32-mode batched solves): V is widened exactly
 // and the sums stay in FP64; scale_copy rounds its output to FP32
 void launch_multidot_b(hipStream_t st, int n, int R, int m, const float2* V, size_t ldv, const double2* w,
