@@ -502,14 +502,22 @@ void launch_split_rows(hipStream_t st, int N, int Q, int Qp, const float2* V, un
     k_split_rows<<<(unsigned)((total + 255) / 256), 256, 0, st>>>(N, Q, Qp, V, planes);
 }
 
-template <int NO, int CT>
+// KS (few items): a workgroup owns one row tile and its wavefronts each take a
+// quarter of every chunk's q; their sums are added once, in wavefront order.
+template <int NO, int CT, bool KS>
 __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, int nw, int K1,
                                                     const unsigned short* __restrict__ P1,
                                                     const uint2* __restrict__ E1, int K2,
                                                     const unsigned short* __restrict__ P2,
                                                     const uint2* __restrict__ E2, double2* __restrict__ y) {
     constexpr int RT = 8 * CT;
-    constexpr int kQ = 32, kP = kQ + 8;   // staged q per chunk, padded LDS row (80 B)
+    // Staged q per chunk and padded LDS row.  A chunk costs a memory round trip
+    // behind two barriers, so with few right-hand sides, where it holds little
+    // work, it is longer: 128 q at 8 of them, which also gives every thread a
+    // staging unit.  With 32 q for all the product with 8 took 205 us on a
+    // 15,870-RWG ellipsoid, with 128 it takes 182.
+    constexpr int kQ = 128 / CT, NS = KS ? 1 : kQ / 32, kP = kQ + 8;   // NS: steps of a wavefront
+    static_assert(!KS || kQ == 128, "a step per wavefront");
     // staging units: a thread loads 8 consecutive q of one (output, rhs) and
     // stores their split pairs with four 16-byte writes, which 8 consecutive
     // lanes (consecutive rhs, rows 80 B apart) spread over all banks
@@ -524,18 +532,22 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
     // read the same pattern planes) run together on one XCD
     const int ny = (R + RT - 1) / RT;
     int it, gy;
-    xcd_chunk(blockIdx.x, 4, ny, it, gy);
+    xcd_chunk(blockIdx.x, KS ? 16 : 4, ny, it, gy);
+    const int rt = KS ? it & 3 : 0;   // this workgroup's row tile of the item
+    if (KS) it >>= 2;
     if (it >= nd.nitem) return;
     const int2 item = nd.items[it];
-    const int t = item.x, rp = item.y;
+    const int t = item.x, rp = item.y + rt;
     const int i0 = nd.leaf_ptr[t], nt = nd.leaf_ptr[t + 1] - i0;
-    const int nrp = min(4, ((nt + 15) >> 4) - rp);
+    const int nrp = min(4 - rt, ((nt + 15) >> 4) - rp);
+    if (KS && nrp < 1) return;   // the whole workgroup
     const int rb0 = gy * RT;
     const int rv = min(RT, R - rb0);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int part = li >> 3;
-    const WaveShare<CT> ws(wave, nrp);
+    const WaveShare<CT> ws(KS ? 0 : wave, KS ? 4 : nrp);   // KS: one row tile, every column tile
+    const int qw = KS ? 32 * wave : 0;                     // first q of this wavefront's steps in a chunk
     const int arow = min((rp + (ws.on ? ws.tile : 0)) * 16 + li, nt - 1);
     // the rest for this item's number of column tiles per wavefront
     ws.each([&](auto cnt) {
@@ -557,9 +569,12 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
         const unsigned short* arow_p = Pl + ((size_t)i0 + arow) * Qp + 8 * lk;   // this lane's 8 q of plane 0
         const uint2* E = (w ? E2 : E1) + (size_t)t * NO * Q * lde;
         auto load_a = [&](int q0, uint4* a) {
-            const int qc = min(q0, Qp - kQ);
 #pragma unroll
-            for (int p = 0; p < 4; ++p) a[p] = *reinterpret_cast<const uint4*>(arow_p + p * plane + qc);
+            for (int s = 0; s < NS; ++s) {
+                const int qc = min(q0 + qw + 32 * s, Qp - 32);
+#pragma unroll
+                for (int p = 0; p < 4; ++p) a[4 * s + p] = *reinterpret_cast<const uint4*>(arow_p + p * plane + qc);
+            }
         };
         auto load_e = [&](int q0) {
             pmask = 0;
@@ -571,7 +586,7 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
                 pmask |= (unsigned)((q < Q) & (sr < rv)) << i;
             }
         };
-        // one 32-q chunk: stage Eall's (split when stored), then the next
+        // one chunk: stage Eall's (split when stored), then the next
         // chunk's loads, then the products from the current patterns (cur);
         // chunks alternate between two register sets, so nothing is copied
         // and the next patterns stay in flight during the products
@@ -598,21 +613,24 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
                 for (int o = 0; o < NO; ++o) {
                     floatx4 d = acc[ct][o];
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {   // E part: hi, then lo (lo meets only the hi patterns)
-                        const uint4 b1 = *reinterpret_cast<const uint4*>(&es[h][o][2 * part][rc][8 * lk]);
-                        const uint4 b2 = *reinterpret_cast<const uint4*>(&es[h][o][1 - part][rc][8 * lk]);
-                        d = mfb(cur[0], b1, d);
-                        d = mfb(cur[1], b2, d);
-                        if (h == 0) {
-                            d = mfb(cur[2], b1, d);
-                            d = mfb(cur[3], b2, d);
+                    for (int s = 0; s < NS; ++s)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {   // E part: hi, then lo (lo meets only the hi patterns)
+                            const int q = qw + 32 * s + 8 * lk;
+                            const uint4 b1 = *reinterpret_cast<const uint4*>(&es[h][o][2 * part][rc][q]);
+                            const uint4 b2 = *reinterpret_cast<const uint4*>(&es[h][o][1 - part][rc][q]);
+                            d = mfb(cur[4 * s], b1, d);
+                            d = mfb(cur[4 * s + 1], b2, d);
+                            if (h == 0) {
+                                d = mfb(cur[4 * s + 2], b1, d);
+                                d = mfb(cur[4 * s + 3], b2, d);
+                            }
                         }
-                    }
                     acc[ct][o] = d;
                 }
             }
         };
-        uint4 aa[4], ab[4];
+        uint4 aa[4 * NS], ab[4 * NS];
         load_e(0);
         load_a(0, aa);
         // chunks in pairs (a chunk past Qp reads clamped patterns and meets zero-staged Eall)
@@ -620,6 +638,20 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
             chunk(q0, aa, ab);
             chunk(q0 + kQ, ab, aa);
         }
+    }
+    if (KS) {
+        static_assert(!KS || sizeof(es) >= 3 * NC * NO * 64 * sizeof(floatx4), "partial sums in the staging area");
+        floatx4* rs = reinterpret_cast<floatx4*>(&es[0][0][0][0][0]);
+        __syncthreads();
+        if (wave > 0)
+#pragma unroll
+            for (int c = 0; c < NC * NO; ++c) rs[((wave - 1) * NC * NO + c) * 64 + lane] = acc[c / NO][c % NO];
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 0; w < 3; ++w)
+#pragma unroll
+            for (int c = 0; c < NC * NO; ++c) acc[c / NO][c % NO] += rs[(w * NC * NO + c) * 64 + lane];
     }
     if (!ws.on) return;
 #pragma unroll
@@ -646,14 +678,20 @@ __global__ __launch_bounds__(256) void k_disagg_bf3(NearDev nd, int R, int lde, 
 void launch_disagg_bf3(hipStream_t st, int R, int lde, const NearDev& nd, bool pmchwt, int K1, const unsigned short* P1,
                        const uint2* E1, int K2, const unsigned short* P2, const uint2* E2, double2* y) {
     if (nd.nitem == 0 || R < 1) return;
-    const int ct = R > 16 ? 4 : (R > 8 ? 2 : 1);
+    // Fewer workgroups of four row tiles than CUs: one row tile and 8 right-hand
+    // sides per workgroup, the wavefronts along q.  64 items at 8 right-hand sides
+    // (a 1,368-RWG cylinder): matvec 215 us with four row tiles, 181 with one; at
+    // several hundred items the two are alike (30.4 ms for the ellipsoid's solve).
+    const bool ks = (long long)nd.nitem * ((R + 7) / 8) < 256;
+    const int ct = ks || R <= 8 ? 1 : (R > 16 ? 4 : 2);
     const int ny = (R + 8 * ct - 1) / (8 * ct);
-    const unsigned grid = xcd_chunk_grid(nd.nitem, 4, ny);
-#define DB(NO, CT) k_disagg_bf3<NO, CT><<<grid, 256, 0, st>>>(nd, R, lde, NO, K1, P1, E1, K2, P2, E2, y)
+    const unsigned grid = ks ? xcd_chunk_grid(4 * nd.nitem, 16, ny) : xcd_chunk_grid(nd.nitem, 4, ny);
+#define DB(NO, CT, KS) k_disagg_bf3<NO, CT, KS><<<grid, 256, 0, st>>>(nd, R, lde, NO, K1, P1, E1, K2, P2, E2, y)
 #define DBN(NO)                                                                                                       \
-    if (ct == 4) DB(NO, 4);                                                                                           \
-    else if (ct == 2) DB(NO, 2);                                                                                      \
-    else DB(NO, 1);
+    if (ks) DB(NO, 1, true);                                                                                          \
+    else if (ct == 4) DB(NO, 4, false);                                                                               \
+    else if (ct == 2) DB(NO, 2, false);                                                                               \
+    else DB(NO, 1, false);
     if (pmchwt) {
         DBN(2)
     } else {
