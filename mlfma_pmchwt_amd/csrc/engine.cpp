@@ -2595,25 +2595,22 @@ void Engine::precond_statistics(const double2* d_b, int steps, int degree, doubl
 }
 
 void Engine::excitation(double pol, double th, double ph, double2* d_v) {
-    ExcitationArgs a;
-    double vth[3], vph[3];
-    plane_wave(pol, th, ph, a.kinc, a.einc, a.hinc, vth, vph);
-    a.k = d2(med.k1);
-    a.alpha = P.cfie_alpha;
-    launch_excitation(st, N, ie, d_geo_, d_perm_, gauss_, a, d_v);
-    MLFMA_HIP(hipGetLastError());
-    MLFMA_HIP(hipStreamSynchronize(st));
+    excitation_batch(1, &pol, &th, &ph, d_v);
 }
 
 // Right-hand sides of n_inc plane waves into column-major d_V (column j at d_V + j * nunk).
 void Engine::excitation_batch(int n_inc, const double* pol, const double* th, const double* ph, double2* d_V) {
-    for (int j = 0; j < n_inc; ++j) {
-        ExcitationArgs a;
-        double vth[3], vph[3];
-        plane_wave(pol[j], th[j], ph[j], a.kinc, a.einc, a.hinc, vth, vph);
-        a.k = d2(med.k1);
-        a.alpha = P.cfie_alpha;
-        launch_excitation(st, N, ie, d_geo_, d_perm_, gauss_, a, d_V + (size_t)j * nunk);
+    for (int j0 = 0; j0 < n_inc; j0 += kExcitationBatch) {
+        ExcitationBatch b{};
+        b.n = std::min(kExcitationBatch, n_inc - j0);
+        for (int j = 0; j < b.n; ++j) {
+            ExcitationArgs& a = b.a[j];
+            double vth[3], vph[3];
+            plane_wave(pol[j0 + j], th[j0 + j], ph[j0 + j], a.kinc, a.einc, a.hinc, vth, vph);
+            a.k = d2(med.k1);
+            a.alpha = P.cfie_alpha;
+        }
+        launch_excitation(st, N, ie, d_geo_, d_perm_, gauss_, b, (size_t)nunk, d_V + (size_t)j0 * nunk);
     }
     MLFMA_HIP(hipGetLastError());
     MLFMA_HIP(hipStreamSynchronize(st));

@@ -16,6 +16,11 @@ struct ExcitationArgs {
     double2 k;
     double alpha;
 };
+constexpr int kExcitationBatch = 8;
+struct ExcitationBatch {   // n <= kExcitationBatch incidences, column j at v + j * ld
+    int n;
+    ExcitationArgs a[kExcitationBatch];
+};
 
 // mode 0 EFIE, 1 CFIE, 2 PMCHWT.  One batch of blocks of the near field: the
 // face-pair integrals (pair_items: block, chunk of 64 face pairs; same: block,
@@ -28,7 +33,7 @@ void launch_patterns(hipStream_t st, bool cfie, int N, int K, const RwgGeo* geo,
                      const double* centre, const double* kp, double2 k, const GaussRule& g, double alpha, double2* Vs,
                      double2* Vf);
 void launch_excitation(hipStream_t st, int N, int mode, const RwgGeo* geo, const int* perm, const GaussRule& g,
-                       const ExcitationArgs& a, double2* v);
+                       const ExcitationBatch& b, size_t ld, double2* v);
 // istride: offset between the current vectors of consecutive angles (0: one vector for all angles)
 void launch_farfield(hipStream_t st, int N, int pmchwt, const RwgGeo* geo, const int* perm, const GaussRule& g,
                      double2 k, int nang, const double* dirs, const double2* I, size_t istride, double2* partial,
