@@ -1143,26 +1143,49 @@ __global__ __launch_bounds__(256) void k_disagg_pec(int N, int K, int ldr, int r
 // sum (-khat x V).B with khat = -kp is sum V.(kp x B)) for the J and M outputs
 //   E_J = a B_J - c kp x B_M,   E_M = c kp x B_J + b B_M
 // with a, b, c the wavenumber's constants over the common factor `scale`, which
-// multiplies the sums in FP64 (k1: a = b = c = 1).  Forming E once per ROWS rows in
-// place of one row's L and K sums cuts the L2 reads of B, which bounded the
-// row-per-wavefront form (7,680 RWG, 346 MB of patterns: 98 us, now 76).  KS = 4:
-// the block's wavefronts split the samples of the same rows instead, for few
-// rows (480 RWG, PEC: 11.7 us with four rows a wavefront, 4.1 with one a block).
+// multiplies the sums in FP64 (k1: a = b = c = 1).  In FP32 mode the constants
+// keep their FP64 value as two FP32 parts, and each wavenumber's sums are added
+// in FP64: constants rounded to FP32 scaled every row of an output alike, by up
+// to 2^-24, which sums of independent roundings stay below.  216,000 PMCHWT
+// unknowns, FP32 product: rounded constants 2.23 ms, as here 2.25, E formed in
+// FP64 2.29, and the four sums with B_J, B_M and their curls kept apart 2.57.
+// Forming E once per ROWS rows in place of one row's L and K sums cuts the L2
+// reads of B, which bounded the row-per-wavefront form (7,680 RWG, 346 MB of
+// patterns: 98 us, now 76).  KS = 4: the block's wavefronts split the samples of
+// the same rows instead, for few rows (480 RWG, PEC: 11.7 us with four rows a
+// wavefront, 4.1 with one a block).
+template <typename R>
+struct WideConst {   // an FP64 constant, as the sum of two FP32 ones in FP32 mode
+    cplx_t<R> hi, lo;
+    WideConst(double2 v) {
+        hi = cplx_t<R>{(R)v.x, (R)v.y};
+        lo = cplx_t<R>{(R)(v.x - (double)hi.x), (R)(v.y - (double)hi.y)};
+    }
+    __device__ __forceinline__ cplx_t<R> times(cplx_t<R> x) const {
+        if constexpr (sizeof(R) == 8) return cmul(hi, x);
+        cplx_t<R> p = cmul(lo, x);
+        cmac(p, hi, x);   // the low part is added before the product is rounded
+        return p;
+    }
+};
+
 template <typename R>
 struct DisaggWave {
     int K;
     const cplx_t<R>*Vf, *Bm;
     const R* kp;
-    double2 a, b, c;
+    WideConst<R> a, b, c;
 };
 
+// (FP32 PMCHWT by whole rows: three wavefronts per SIMD asked for, 181 registers without)
 template <typename R, bool PM, int ROWS, int KS>
-__global__ __launch_bounds__(256) void k_disagg_one(int N, int nw, int ldr, int r0, const int* __restrict__ leaf_of,
-                                                    const int* __restrict__ perm, DisaggWave<R> w0, DisaggWave<R> w1,
-                                                    double2 scale, double2* __restrict__ y) {
+__global__ __launch_bounds__(256, sizeof(R) == 4 && PM && ROWS == 4 && KS == 1 ? 3 : 1) void k_disagg_one(
+    int N, int nw, int ldr, int r0, const int* __restrict__ leaf_of, const int* __restrict__ perm, DisaggWave<R> w0,
+    DisaggWave<R> w1, double2 scale, double2* __restrict__ y) {
     using C = cplx_t<R>;
     constexpr int NO = PM ? 2 : 1;
-    __shared__ C red[KS == 1 ? 1 : 4][ROWS * NO];
+    constexpr bool APART = PM && sizeof(R) == 4;   // each wavenumber's sums are added in FP64
+    __shared__ double2 red[4][ROWS * NO];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int i00 = (KS == 1 ? blockIdx.x * 4 + wave : blockIdx.x) * ROWS;
     if (KS == 1 && i00 >= N) return;
@@ -1174,10 +1197,22 @@ __global__ __launch_bounds__(256) void k_disagg_one(int N, int nw, int ldr, int 
     for (int u = 0; u < ROWS; ++u)
 #pragma unroll
         for (int o = 0; o < NO; ++o) s[u][o] = C{0, 0};
+    auto leave = [&](bool add) {   // the sums so far into red, or added to what is there
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+            for (int o = 0; o < NO; ++o) {
+                double2 f = widen(wave_sum(s[u][o]));
+                s[u][o] = C{0, 0};
+                if (lane == 0) {
+                    if (add) f = cadd(red[wave][u * NO + o], f);
+                    red[wave][u * NO + o] = f;
+                }
+            }
+    };
     for (int w = 0; w < nw; ++w) {
         const DisaggWave<R> W = w == 0 ? w0 : w1;
         const int K = W.K;
-        const C ca = C{(R)W.a.x, (R)W.a.y}, cb = C{(R)W.b.x, (R)W.b.y}, cc = C{(R)W.c.x, (R)W.c.y};
         for (int q = lane + (KS == 1 ? 0 : 64 * wave); q < K; q += 64 * KS) {
             C v[ROWS][3];
 #pragma unroll
@@ -1205,8 +1240,8 @@ __global__ __launch_bounds__(256) void k_disagg_one(int N, int nw, int ldr, int 
                         const C m[3] = {m0, m1, m2};
 #pragma unroll
                         for (int d = 0; d < 3; ++d) {
-                            e[0][d] = csub(cmul(ca, e[0][d]), cmul(cc, cm[d]));
-                            e[NO - 1][d] = cadd(cmul(cc, cj[d]), cmul(cb, m[d]));
+                            e[0][d] = csub(W.a.times(e[0][d]), W.c.times(cm[d]));
+                            e[NO - 1][d] = cadd(W.c.times(cj[d]), W.b.times(m[d]));
                         }
                     }
                 }
@@ -1216,37 +1251,24 @@ __global__ __launch_bounds__(256) void k_disagg_one(int N, int nw, int ldr, int 
                     for (int d = 0; d < 3; ++d) cfma(s[u][o], v[u][d], e[o][d]);
             }
         }
+        if (APART && w == 0) leave(false);
     }
-#pragma unroll
-    for (int u = 0; u < ROWS; ++u)
-#pragma unroll
-        for (int o = 0; o < NO; ++o) s[u][o] = wave_sum(s[u][o]);
+    leave(APART);
     if (KS > 1) {
-        if (lane == 0)
-#pragma unroll
-            for (int u = 0; u < ROWS; ++u)
-#pragma unroll
-                for (int o = 0; o < NO; ++o) red[wave][u * NO + o] = s[u][o];
         __syncthreads();
         if (wave > 0) return;
+    } else {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // lane 0 of this wavefront wrote red
     }
     if (lane < ROWS * NO) {   // lane u * NO + o writes row u, output o
         const int u = lane / NO, o = lane - u * NO;
-        C v = s[0][0];
-        if (KS > 1) {
-            v = red[0][lane];
-            for (int k = 1; k < 4; ++k) v.x += red[k][lane].x, v.y += red[k][lane].y;
-        } else {
-#pragma unroll
-            for (int uu = 0; uu < ROWS; ++uu)
-#pragma unroll
-                for (int oo = 0; oo < NO; ++oo)
-                    if (uu == u && oo == o) v = s[uu][oo];
-        }
+        double2 v = red[wave][lane];
+        if (KS > 1)
+            for (int k = 1; k < 4; ++k) v = cadd(v, red[k][lane]);
         if (i00 + u < N) {
             double2* yp = y + ((size_t)o * N + perm[i00 + u]) * ldr + r0;
             double2 t = *yp;
-            cfma(t, scale, widen(v));
+            cfma(t, scale, v);
             *yp = t;
         }
     }

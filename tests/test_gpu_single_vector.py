@@ -72,3 +72,48 @@ def test_disaggregation_rows(freq, radius, ie):
         # sums of 3K products in two orders, a few roundings per product
         bound = (6 * v.size + 64) * np.finfo(float).eps * size
         assert np.all(np.abs(np.array(got) - want[:len(got)]) <= bound[:len(got)]), i
+
+
+# the three forms of the disaggregation again, in FP32
+@pytest.mark.parametrize("freq,radius", [(8, 0.9), (16, 1.1), (26, 1.4)])
+def test_fp32_disaggregation_keeps_its_constants(freq, radius):
+    """FP32 sums of the second wavenumber meet their constants in FP64.  The constants c, c z and c / z of this
+    permittivity round to FP32 by 0.98 units u = 2^-24 of either sign, which would scale the two outputs of one
+    current apart by 1.96 u in every row alike.  The scales of the two outputs' errors along their exact parts
+    come from one workspace, so what its own rounding adds to both cancels; the rest is 2,000 rows' independent
+    errors of about 3 u, 0.07 u of each scale."""
+    eps = 4.0322144
+    op = api.Operator(geometry.geodesic_sphere(freq, radius), integral_equation=api.PMCHWT, eps_r_re=eps,
+                      far_precision=api.FP32)
+    n = op.n_rwg
+    assert {8: n < 2048, 16: 2048 <= n < 16384, 26: n >= 16384}[freq]
+    rng = np.random.default_rng(freq)
+    ptr, rwg = op.level_list(op.max_level, 4)
+    box = np.empty(n, dtype=int)
+    for t in range(len(ptr) - 1):
+        box[rwg[ptr[t]:ptr[t + 1]]] = t
+    rows = rng.permutation(n)[:2000]
+    v = np.stack([op.pattern(2, 1, int(i)) for i in rows])
+    _, th, ph, _, _ = op.grid(2, op.max_level)
+    T, P = np.meshgrid(th, ph, indexing="ij")
+    kp = np.stack([np.sin(T) * np.cos(P), np.sin(T) * np.sin(P), np.cos(T)], -1).reshape(-1, 3)
+    for cur in (0, 1):
+        x = np.zeros(op.n, dtype=complex)
+        x[cur * n:(cur + 1) * n] = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+        op.set_apply_precision(api.FP64)
+        y = op.apply(x)
+        far = y - op.stage(api.STAGE_NEAR, x)
+        op.set_apply_precision(api.FP32)
+        err = op.apply(x) - y      # the near product is the same FP64 one
+        assert np.linalg.norm(err) <= 2e-6 * np.linalg.norm(far)   # FP32 sums throughout
+        op.stage(api.STAGE_AGGREGATE, x)
+        op.stage(api.STAGE_M2M)
+        op.stage(api.STAGE_M2L_L2L)
+        b = np.stack([op.workspace(2, cur, 1, op.max_level, t) for t in range(len(ptr) - 1)])[box[rows]]
+        c, z = eps / 4.0, np.sqrt(1.0 / eps)
+        lin, curl = c * np.einsum("nqx,nqx->n", v, b), c * np.einsum("nqx,nqx->n", v, np.cross(kp, b))
+        parts = (lin * z, curl) if cur == 0 else (-curl, lin / z)
+        scale = [np.vdot(p, e) / np.vdot(p, p).real for p, e in zip(parts, (err[rows], err[n + rows]))]
+        print(f"[constants] {n} RWG current {cur}: {scale[0] * 2**24:.2f} {scale[1] * 2**24:.2f} u", flush=True)
+        assert abs(scale[0] - scale[1]) <= 0.5 * 2.0**-24
+    op.close()
