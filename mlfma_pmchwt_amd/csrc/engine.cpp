@@ -88,7 +88,9 @@ T* Engine::dalloc(size_t count) {
     if (capturing_) throw Error(MLFMA_ERR_STATE, "device allocation inside a recorded matvec");
     if (count == 0) count = 1;
     void* p = nullptr;
-    MLFMA_HIP(hipMalloc(&p, count * sizeof(T)));
+    const hipError_t e = hipMalloc(&p, count * sizeof(T));
+    if (e != hipSuccess) (void)hipGetLastError();   // thrown here, not seen again by the next launch's check
+    MLFMA_HIP(e);
     allocs_[p] = count * sizeof(T);
     dev_bytes += count * sizeof(T);
     return static_cast<T*>(p);
@@ -660,7 +662,7 @@ void Engine::fill_near(int planes, const NearConsts& c) {
     for (const void* q : {(const void*)nf.faces, (const void*)nf.face_ptr, (const void*)nf.face_idx,
                           (const void*)nf.row_ptr, (const void*)nf.side, (const void*)nf.len, (const void*)nf.blocks,
                           (const void*)d_pairs, (const void*)d_same, (const void*)d_entries, (const void*)scr})
-        dfree(const_cast<void*>(q));
+        release(const_cast<void*>(q));
 }
 
 // Items of the single-vector near product when the leaves alone do not fill
@@ -1079,7 +1081,6 @@ void Engine::ensure_eall(int R) {
     for (int w = 0; w < nw; ++w) {
         dfree(d_Eall_[w]);
         dfree(d_Sall_[w]);
-        d_Eall_[w] = d_Sall_[w] = nullptr;
     }
     const int c32 = P.far_precision == MLFMA_FP32 ? eall_ld(R) : 0;
     auto take = [&](int cols) {   // cols of FP32
@@ -1102,7 +1103,6 @@ void Engine::ensure_eall(int R) {
     for (int w = 0; w < nw; ++w) {
         dfree(d_Eall_[w]);
         dfree(d_Sall_[w]);
-        d_Eall_[w] = d_Sall_[w] = nullptr;
     }
     if (c32 > 0) {
         take(c32);
@@ -1136,6 +1136,7 @@ void Engine::ensure_block(int R) {
     ensure_eall(R);
     if (R <= block_cap_) return;
     clear_graphs();
+    block_cap_ = 0;
     dfree(d_bx_);
     dfree(d_by_);
     d_bx_ = dalloc<double2>((size_t)nunk * R);
@@ -1278,7 +1279,7 @@ void Engine::set_tuning(int prec, int rb, int bits) {
     clear_graphs();
 }
 
-void Engine::dfree(void* p) {
+void Engine::release(void* p) {
     if (!p) return;
     if (capturing_) throw Error(MLFMA_ERR_STATE, "device free inside a recorded matvec");
     auto it = allocs_.find(p);
@@ -1377,14 +1378,17 @@ void Engine::solve(const mlfma_solve_params& sp, const double2* d_b, double2* d_
     const int m = std::max(1, sp.restart);
     const double eps = 1e-16;
     if (V_cols_ < std::max(m + 1, 10)) {
-        V_cols_ = std::max(m + 1, 10);
-        d_V_ = dalloc<double2>((size_t)V_cols_ * n);
+        const int cols = std::max(m + 1, 10);
+        V_cols_ = 0;
+        dfree(d_V_, d_w_, d_r_, d_t_, d_part_, d_small_, d_rpart_);
+        d_V_ = dalloc<double2>((size_t)cols * n);
         d_w_ = dalloc<double2>(n);
         d_r_ = dalloc<double2>(n);
         d_t_ = dalloc<double2>(n);
-        d_part_ = dalloc<double2>((size_t)V_cols_ * kRedBlocks);
-        d_small_ = dalloc<double2>(V_cols_);
+        d_part_ = dalloc<double2>((size_t)cols * kRedBlocks);
+        d_small_ = dalloc<double2>(cols);
         d_rpart_ = dalloc<double>(kRedBlocks);
+        V_cols_ = cols;
     }
     if (sp.precond < 0 || sp.precond > 3) throw Error(MLFMA_ERR_ARG, "precond must be 0, 1, 2 or 3");
     stats_fallbacks_ = 0;
@@ -1393,6 +1397,7 @@ void Engine::solve(const mlfma_solve_params& sp, const double2* d_b, double2* d_
     precond_kind_ = sp.precond;
     if (sp.precond == 1) precond_setup();
     if (pc && sp.solver == MLFMA_SOLVER_GMRES && Zf_cols_ < m) {
+        Zf_cols_ = 0;
         dfree(d_Zf_);
         d_Zf_ = dalloc<double2>((size_t)m * n);
         Zf_cols_ = m;
@@ -1698,11 +1703,9 @@ void Engine::bs_start(BlockState& s, const mlfma_solve_params& sp, const double2
     ensure_pinned((size_t)(2 * m + 3) * R);
     const size_t nR = s.nR;
     if (bV_cols_ < m + 1 || bV_R_ != R) {
-        for (void* p : {(void*)d_bV_, (void*)d_bW_, (void*)d_bRr_, (void*)d_bpart_, (void*)d_bsmall_, (void*)d_bscale_,
-                        (void*)d_bZ_, (void*)d_bG_})
-            dfree(p);
-        bV_cols_ = m + 1;
-        bV_R_ = R;
+        clear_graphs();   // recorded sequences refer to these buffers
+        bV_cols_ = 0;
+        dfree(d_bV_, d_bW_, d_bRr_, d_bpart_, d_bsmall_, d_bscale_, d_bZ_, d_bG_);
         d_bV_ = dalloc<double2>(nR * (m + 1));
         d_bW_ = dalloc<double2>(nR);
         d_bRr_ = dalloc<double2>(nR);
@@ -1711,11 +1714,13 @@ void Engine::bs_start(BlockState& s, const mlfma_solve_params& sp, const double2
         d_bscale_ = dalloc<double>(R);
         d_bZ_ = dalloc<double2>(nR);
         d_bG_ = dalloc<double2>(nR);
-        clear_graphs();   // recorded sequences refer to the freed block buffers
+        bV_cols_ = m + 1;
+        bV_R_ = R;
     }
     // the flexible basis z_k = M^-1 v_k is sized whenever a preconditioner may run
     // (a stalling polynomial falls back to the block-diagonal one mid-solve)
     if (s.pc && (bZf_cols_ < m || bZf_nR_ != nR)) {
+        bZf_cols_ = 0;
         dfree(d_bZf_);
         d_bZf_ = dalloc<double2>(nR * m);
         bZf_cols_ = m;
@@ -1725,12 +1730,14 @@ void Engine::bs_start(BlockState& s, const mlfma_solve_params& sp, const double2
     // Gram-Schmidt passes); the reductions, W and the solution stay FP64
     s.vf = apply_prec == MLFMA_FP32;
     if (s.vf && (bVf_cols_ < m + 1 || bVf_nR_ != nR)) {
+        bVf_cols_ = 0;
         dfree(d_bVf_);
         d_bVf_ = dalloc<float2>(nR * (m + 1));
         bVf_cols_ = m + 1;
         bVf_nR_ = nR;
     }
     if (s.vf && s.pc && (bZff_cols_ < m || bZff_nR_ != nR)) {
+        bZff_cols_ = 0;
         dfree(d_bZff_);
         d_bZff_ = dalloc<float2>(nR * m);
         bZff_cols_ = m;
@@ -2264,8 +2271,9 @@ void Engine::ensure_inner(int R) {
     const int k = inner_steps_;
     if (R <= inner_cap_R_ && k <= inner_cap_k_) return;
     clear_graphs();
-    for (void* p : {(void*)d_iU_, (void*)d_iW_, (void*)d_ipart_, (void*)d_ismall_, (void*)d_ih_}) dfree(p);
     const int Rc = std::max(R, inner_cap_R_), kc = std::max(k, inner_cap_k_);
+    inner_cap_R_ = inner_cap_k_ = 0;
+    dfree(d_iU_, d_iW_, d_ipart_, d_ismall_, d_ih_);
     d_iU_ = dalloc<double2>((size_t)nunk * Rc * (kc + 1));
     d_iW_ = dalloc<double2>((size_t)nunk * Rc);
     d_ipart_ = dalloc<double2>((size_t)(kc + 1) * kRedBlocks * Rc);
@@ -2395,6 +2403,7 @@ void Engine::set_poly(const std::vector<cplx>& alpha) {
 void Engine::ensure_xf(int R) {
     if (!d_Z32_ || R <= xf_cap_) return;
     clear_graphs();
+    xf_cap_ = 0;
     dfree(d_xf_);
     d_xf_ = dalloc<float2>((size_t)nunk * R);
     xf_cap_ = R;
@@ -2408,14 +2417,11 @@ void Engine::ensure_poly(int R) {
     if (P.far_precision == MLFMA_FP32) ensure_eall(R);
     if (R <= poly_cap_) return;
     clear_graphs();
-    dfree(d_pt_);
-    dfree(d_pu_);
+    poly_cap_ = 0;
+    dfree(d_pt_, d_pu_, d_xb_);
     d_pt_ = dalloc<double2>((size_t)nunk * R);
     d_pu_ = dalloc<double2>((size_t)nunk * R);
-    if (d_Zbf_) {
-        dfree(d_xb_);
-        d_xb_ = dalloc<unsigned>((size_t)nunk * R);
-    }
+    if (d_Zbf_) d_xb_ = dalloc<unsigned>((size_t)nunk * R);
     poly_cap_ = R;
 }
 
@@ -2590,8 +2596,7 @@ void Engine::precond_statistics(const double2* d_b, int steps, int degree, doubl
     block_dots(E, col);
     for (int j = 0; j < m; ++j) h[j] = d2(col[j]);
     *c = (double)R;   // unit basis vectors
-    for (void* q : {(void*)V, (void*)W, (void*)part, (void*)small, (void*)E, (void*)T, (void*)bpart, (void*)bsmall})
-        dfree(q);
+    dfree(V, W, part, small, E, T, bpart, bsmall);
 }
 
 void Engine::excitation(double pol, double th, double ph, double2* d_v) {

@@ -229,7 +229,14 @@ private:
     T* dalloc(size_t count);
     template <typename T>
     T* upload(const std::vector<T>& v);
-    void dfree(void* p);
+    void release(void* p);
+    // every pointer freed and forgotten.  A caller that replaces buffers also
+    // forgets their capacity first, so that a failed allocation leaves neither a
+    // freed pointer nor a size that a later call would take as there
+    template <typename... T>
+    void dfree(T*&... p) {
+        ((release(p), p = nullptr), ...);
+    }
     struct GraphKey {
         int kind, R, prec;
         bool operator<(const GraphKey& o) const {
