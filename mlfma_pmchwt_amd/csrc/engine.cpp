@@ -88,8 +88,15 @@ T* Engine::dalloc(size_t count) {
     if (capturing_) throw Error(MLFMA_ERR_STATE, "device allocation inside a recorded matvec");
     if (count == 0) count = 1;
     void* p = nullptr;
-    const hipError_t e = hipMalloc(&p, count * sizeof(T));
+    hipError_t e = hipMalloc(&p, count * sizeof(T));
     if (e != hipSuccess) (void)hipGetLastError();   // thrown here, not seen again by the next launch's check
+    if (e == hipErrorOutOfMemory && drop_eall64()) {
+        e = hipMalloc(&p, count * sizeof(T));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            eall64_asked_ = 0;   // given back in vain: the next product may take them again
+        }
+    }
     MLFMA_HIP(e);
     allocs_[p] = count * sizeof(T);
     dev_bytes += count * sizeof(T);
@@ -995,7 +1002,7 @@ void Engine::apply_block(const double2* X, double2* Y, int R, int prec, const fl
     // and disaggregation groups)
     if (!f32 && !capturing_) ensure_eall(R);
     // columns per all-RHS product: whole passes, so that the passes are the same either way
-    const int width = f32 ? R : std::min({R, kAll64, all64_cols_});
+    const int width = f32 ? R : std::min({R, kAll64, eall_cols_ / 2 & ~7});   // whole padded columns (eall_ld)
     const int step = width >= R ? R : width / cap * cap;
     const bool all = mfma_near && disagg_mfma_ && step > 0;
     const int L = tree.max_level;
@@ -1072,44 +1079,61 @@ void Engine::apply_block(const double2* X, double2* Y, int R, int prec, const fl
 // All-RHS leaf workspaces and effective matrices (sized before any recording:
 // the recorded sequences hold their addresses): R columns of FP32 for the FP32
 // far field, and of FP64 for up to kAll64 columns, in the same buffers (64
-// columns of FP32 hold 32 of FP64).  Where the FP64 columns do not fit the
-// device, the FP64 matvec keeps to passes.
+// columns of FP32 hold 32 of FP64).  The FP64 columns are a matter of speed
+// only: they are taken where the matrix-core products that use them are on and
+// they need at most an eighth of the device's free memory, and given back when
+// another allocation of the handle does not fit (drop_eall64).  The FP64 matvec
+// then keeps to passes.
 void Engine::ensure_eall(int R) {
-    if (R <= eall_cap_ || R < 2) return;
-    clear_graphs();
-    const int L = tree.max_level, no = ie == MLFMA_PMCHWT ? 2 : 1;
-    for (int w = 0; w < nw; ++w) {
-        dfree(d_Eall_[w]);
-        dfree(d_Sall_[w]);
+    if (R < 2) return;
+    const int need = std::max(eall_need_, P.far_precision == MLFMA_FP32 ? eall_ld(R) : 0);
+    const int r64 = near_mfma_ && disagg_mfma_ ? std::min(R, kAll64) : 0;
+    int cols = need;
+    if (r64 > eall64_asked_) {
+        const int want = std::max(need, 2 * eall_ld(r64));
+        size_t free = 0, total = 0;
+        MLFMA_HIP(hipMemGetInfo(&free, &total));
+        const size_t more = eall_bytes(want) - eall_bytes(std::max(need, std::min(eall_cols_, want)));
+        if (more <= free / 8) cols = want;
     }
-    const int c32 = P.far_precision == MLFMA_FP32 ? eall_ld(R) : 0;
-    auto take = [&](int cols) {   // cols of FP32
+    eall_need_ = need;
+    eall64_asked_ = std::max(eall64_asked_, r64);
+    if (cols <= eall_cols_) return;
+    take_eall(cols);
+}
+
+size_t Engine::eall_bytes(int cols) const {   // cols of FP32, a multiple of 8
+    const int L = tree.max_level, no = ie == MLFMA_PMCHWT ? 2 : 1;
+    size_t n = 0;
+    for (int w = 0; w < nw; ++w) n += (size_t)nleaf * (no + ncur) * 3 * wd_[w].K[L] * cols * sizeof(float2);
+    return n;
+}
+
+void Engine::take_eall(int cols) {
+    clear_graphs();
+    eall_cols_ = 0;
+    dfree(d_Eall_[0], d_Eall_[1], d_Sall_[0], d_Sall_[1]);
+    if (cols == 0) return;
+    const int L = tree.max_level, no = ie == MLFMA_PMCHWT ? 2 : 1;
+    try {
         for (int w = 0; w < nw; ++w) {
-            d_Eall_[w] = dalloc<float2>((size_t)nleaf * no * 3 * wd_[w].K[L] * cols);   // cols: a multiple of 8
+            d_Eall_[w] = dalloc<float2>((size_t)nleaf * no * 3 * wd_[w].K[L] * cols);
             d_Sall_[w] = dalloc<float2>((size_t)nleaf * ncur * 3 * wd_[w].K[L] * cols);
         }
-        all64_cols_ = cols / 2 & ~7;   // whole padded columns (eall_ld)
-        eall_cap_ = R;
-    };
-    eall_cap_ = all64_cols_ = 0;
-    const int cols = std::max(c32, 2 * eall_ld(std::min(R, kAll64)));
-    try {
-        take(cols);
-        return;
     } catch (const Error& e) {
-        if (e.code != MLFMA_ERR_OOM || cols == c32) throw;
-        (void)hipGetLastError();
+        if (e.code != MLFMA_ERR_OOM || cols == eall_need_) throw;
+        take_eall(eall_need_);   // without the FP64 columns
+        return;
     }
-    for (int w = 0; w < nw; ++w) {
-        dfree(d_Eall_[w]);
-        dfree(d_Sall_[w]);
-    }
-    if (c32 > 0) {
-        take(c32);
-    } else {
-        all64_cols_ = 0;
-        eall_cap_ = R;
-    }
+    eall_cols_ = cols;
+}
+
+// Gives back what only the FP64 columns take; false where there is nothing, or
+// where a matvec under way uses it.
+bool Engine::drop_eall64() {
+    if (capturing_ || eall_R_ > 0 || eall_cols_ <= eall_need_) return false;
+    take_eall(eall_need_);
+    return true;
 }
 
 // Column-major device vectors (vector j at x + j * nunk), as the C ABI passes them.
@@ -1176,6 +1200,7 @@ void Engine::run_graph(const GraphKey& key, const std::function<void()>& body) {
 
 void Engine::clear_graphs() {
     if (capturing_) throw Error(MLFMA_ERR_STATE, "workspace resize inside a recorded matvec");
+    ++graph_epoch_;
     if (!graphs_.empty()) hipStreamSynchronize(st);
     for (auto& kv : graphs_) hipGraphExecDestroy(kv.second);
     graphs_.clear();

@@ -170,6 +170,8 @@ public:
     // a capture of several operators' matvecs into one graph (solve_multi)
     void set_capturing(bool on) { capturing_ = on; }
     bool graphs_on() const { return use_graphs_ && !prof_on_; }
+    // changes whenever sequences recorded before no longer hold (buffers moved, tuning changed)
+    int graph_epoch() const { return graph_epoch_; }
     // hipGraph replay of batched matvecs; launch-configuration autotuner
     void set_graphs(bool on);
     void autotune(int R, int prec, double* out);
@@ -247,6 +249,7 @@ private:
     void clear_graphs();
     std::map<GraphKey, hipGraphExec_t> graphs_;
     bool use_graphs_ = false;
+    int graph_epoch_ = 0;
     int rb_tuned_[2] = {0, 0};   // tuned right-hand sides per far pass (FP64, FP32); 0: widest
     void build_device_tree();
     void build_wave(int w);
@@ -285,6 +288,9 @@ private:
     void ensure_poly(int R);
     void ensure_xf(int R);
     void ensure_eall(int R);
+    size_t eall_bytes(int cols) const;
+    void take_eall(int cols);
+    bool drop_eall64();
     void near_block(const double2* X, double2* Y, int R, int prec, bool precond = false);
     double norm(const double2* v, int n);
 
@@ -306,20 +312,21 @@ private:
     long long* d_bsoff_ = nullptr;
     uint4* d_Zbf_ = nullptr;    // BF16 record copy for the preconditioner (precond_precision = MLFMA_BF16)
     long long* d_bfoff_ = nullptr;
-    float2* d_Eall_[2] = {nullptr, nullptr};   // all-RHS effective matrices (FP32), nleaf x no x 3K x eall_cap_
+    float2* d_Eall_[2] = {nullptr, nullptr};   // all-RHS effective matrices (FP32), nleaf x no x 3K x eall_cols_
     unsigned short* d_Vb_[2] = {nullptr, nullptr};   // split-pair BF16 receive-pattern planes (near_precision = MLFMA_BF16)
     unsigned short* d_Va_[2] = {nullptr, nullptr};   // split-pair BF16 radiation-pattern planes, transposed [4][Qa][Np]
     int Qa_[2] = {0, 0};                             // their sample rows (3 K rounded up to 64)
     int Np_ = 0;                                     // their RWG columns (every leaf rounded up to 32)
     int* d_joff_ = nullptr;                          // first column of each leaf
     int* d_jmap_ = nullptr;                          // RWG of each column, -1 for padding
-    float2* d_Sall_[2] = {nullptr, nullptr};   // all-RHS leaf radiation workspaces of the passes, nleaf x ncur x 3K x eall_cap_
-    int eall_cap_ = 0;
+    float2* d_Sall_[2] = {nullptr, nullptr};   // all-RHS leaf radiation workspaces of the passes, nleaf x ncur x 3K x eall_cols_
+    int eall_cols_ = 0;      // columns of FP32 in both
+    int eall_need_ = 0;      // of them, those that the FP32 far field cannot do without
+    int eall64_asked_ = 0;   // FP64 columns that were taken or did not fit
     int eall_R_ = 0;   // > 0 while a batched matvec defers its disaggregation to one all-RHS product
     static constexpr int kAll64 = 32;   // FP64 columns of an all-RHS product
     // columns of Eall, padded so that the passes' 2 to 8 columns start on 64-byte boundaries
     static int eall_ld(int R) { return (R + 7) & ~7; }
-    int all64_cols_ = 0;                // FP64 columns that the all-RHS buffers hold
     float2* d_xf_ = nullptr;    // FP32 copy of the matrix-core near product's input, nunk x xf_cap_
     int xf_cap_ = 0;
     unsigned* d_xb_ = nullptr;  // BF16 copy of the preconditioner's near-product input, nunk x poly_cap_

@@ -12,9 +12,9 @@
 // quarter of its columns has converged), so each object's iterates equal a
 // solve of that object alone.  The orthogonalisation of all objects is issued
 // together and shares one synchronisation per step.  Graphs are recorded per set of
-// (object, graph kind, right-hand sides, precision) taking part in a step, so
-// an object that finishes or falls back to a plainer preconditioner leads to
-// a new recording; the recordings live for the call.
+// (object, graph kind, right-hand sides, precision, buffers) taking part in a
+// step, so an object that finishes or falls back to a plainer preconditioner
+// leads to a new recording; the recordings live for the call.
 #include <algorithm>
 #include <map>
 #include <vector>
@@ -86,6 +86,7 @@ void solve_multi(const std::vector<Engine*>& es, const mlfma_solve_params& sp, c
             key.push_back(es[k]->bs_graph_kind(top(k)));
             key.push_back(top(k).R);
             key.push_back(es[k]->apply_prec);
+            key.push_back(es[k]->graph_epoch());
         }
         // the inputs each object staged on its own stream come first
         for (int k : open) {
