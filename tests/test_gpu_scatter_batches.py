@@ -4,7 +4,8 @@ Excitation columns equal single excitations: the same sums per column, so up to 
 product and a sum, one rounding for each of the 2 n quadrature terms of a function.  The far field of
 many directions (four per thread) equals that of few (one per thread) up to where the projection is
 taken: about eight roundings for each of T = 2 n N terms, independent, so 8 sqrt(T) u of the summed
-magnitudes, which are at most some ten times the largest field of an open angle range."""
+magnitudes, which are at most some ten times the largest field of an open angle range.  The same with
+a current per direction, as in a monostatic sweep."""
 import numpy as np
 import pytest
 
@@ -46,5 +47,26 @@ def test_many_directions_match_few(name, nang):
     err = np.abs(field(many) - field(few)).max() / field(few).max()
     bound = 10 * 8 * np.sqrt(2 * POINTS * op.n_rwg) * U
     print(f"[directions] {name} x{nang}: {err:.2e} bound {bound:.2e}", flush=True)
+    assert err <= bound
+    op.close()
+
+
+@pytest.mark.parametrize("name", ["cfie", "pmchwt"])
+def test_many_directions_with_a_current_each(name):
+    """The monostatic sweep's far field (a current per direction, four directions per thread, a count that four
+    does not divide) against one direction at a time of the same solutions."""
+    op = api.Operator(geometry.icosphere(4, 0.9), integral_equation=CASES[name], eps_r_re=3.0, max_rhs=8)
+    nang = 141
+    assert -(-op.n_rwg // 256) * nang >= 4096
+    th, ph = np.linspace(3.0, 177.0, nang), np.linspace(0.0, 90.0, nang)
+    how = dict(restart=50, tol_rel=1e-12, tol_abs=0.0, itr_max=2)   # solutions of two steps
+    many, _ = op.monostatic(th, ph, pol=0.0, **how)
+    x, _ = op.solve_batch(op.excitation_batch(np.zeros(nang), th, ph), **how)
+    few = np.concatenate([np.asarray(op.rcs(np.ascontiguousarray(x[:, a]), th[a:a + 1], ph[a:a + 1]))
+                          for a in range(nang)])
+    field = lambda db: 10.0 ** (db / 20.0)
+    err = np.abs(field(np.asarray(many)) - field(few)).max() / field(few).max()
+    bound = 10 * 8 * np.sqrt(2 * POINTS * op.n_rwg) * U
+    print(f"[currents] {name}: {err:.2e} bound {bound:.2e}", flush=True)
     assert err <= bound
     op.close()
