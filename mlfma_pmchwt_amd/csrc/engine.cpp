@@ -156,7 +156,6 @@ void Engine::build(int np, const int* ids, const double* xyz, int nf, const int*
             g.vf[s][0] = fv.x, g.vf[s][1] = fv.y, g.vf[s][2] = fv.z;
             g.nrm[s][0] = mesh.normal[f].x, g.nrm[s][1] = mesh.normal[f].y, g.nrm[s][2] = mesh.normal[f].z;
             g.area[s] = mesh.area[f];
-            g.face[s] = mesh.face_id[f];
         }
         g.len = basis.len[r];
     }

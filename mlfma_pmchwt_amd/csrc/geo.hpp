@@ -12,7 +12,6 @@ struct RwgGeo {
     double nrm[2][3];    // unit normal (snapped, Code/NASReader.cpp:52-56)
     double area[2];
     double len;          // common edge length
-    int face[2];         // face ids, for the identical-triangle test
 };
 
 struct GaussRule {       // Dunavant rule, weights sum to 0.5
