@@ -677,8 +677,11 @@ void Engine::fill_near(int planes, const NearConsts& c) {
 // PMCHWT unknowns in 56 leaves of 25 MB took 1.27 ms (1.1 TB/s).  With column
 // ranges of about 1/1024 of all entries (at least 128 KB, at least 16 columns)
 // every CU holds several (the same product: 0.19 ms); their partial sums cost
-// a second, small launch (about 4 us), so leaves under 512 KB (or 2,048 and more of them: 300,000 RWG
-// in 3,200 leaves of 2.1 MB stream at 5.9 TB/s unsplit) stay whole.
+// a second, small launch (about 4 us), so leaves under 512 KB stay whole (FP64
+// PMCHWT: 768 leaves of 19 RWG whole 42 us, split 49; of 31 RWG, at the line, 102
+// and 104; 392 leaves of 48 RWG 165 and 142), and so do 2,048 and more leaves
+// (1,392 leaves 1,127 and 1,067 us, 1,968 leaves 796 and 791, 2,264 leaves 1,160
+// and 1,164; 300,000 RWG in 3,200 leaves of 2.1 MB stream at 5.9 TB/s unsplit).
 void Engine::build_near_split(int planes) {
     const std::vector<int>& lp = tree.leaf_ptr;
     const size_t esize = sizeof(double2);
@@ -1823,8 +1826,8 @@ bool Engine::bs_step_open(const BlockState& s) const {
 int Engine::bs_graph_kind(const BlockState& s) const { return s.pc && s.pkind != 3 ? (s.pkind == 2 ? 1 : 3) : 2; }
 
 // The matvec of step k.  recorded: the input goes to the fixed buffer G
-// (through the inner near-field solve first with precond 3, which synchronises
-// with the host and so is never recorded), and bs_body runs between fixed
+// (through the inner near-field solve first with precond 3, which waits for the
+// device once and so is never recorded), and bs_body runs between fixed
 // buffers.  Otherwise the whole step runs here.
 void Engine::bs_pre(BlockState& s, bool recorded) {
     ++s.total;
@@ -2318,9 +2321,11 @@ void Engine::inner_near_solve(const double2* V, double2* Z, int R, int prec) {
     // each, and the subtractions and the scaling read them there.  The host reads
     // all of it once, after the last step.  A column whose recurrence has ended
     // (v = 0, or breakdown) is scaled by zero and stays zero through the remaining
-    // steps, which the host leaves out.  With the host between the reductions
-    // (five waits per step) a 12-iteration solve of 8 right-hand sides at 31,740
-    // unknowns took 44.8 ms, so 30.8.
+    // steps, which the host leaves out.  (They still run where every column has
+    // ended: a solve's block has a live column, so only a zero block given to the
+    // preconditioner alone, or fewer unknowns than steps, pays for them.)  With the
+    // host between the reductions (five waits per step) a 12-iteration solve of 8
+    // right-hand sides at 31,740 unknowns took 44.8 ms, so 30.8.
     auto at = [&](int j) { return (size_t)R * (1 + (size_t)j * (j + 2)); };   // step j's block
     auto norm_to = [&](const double2* v, double2* out) {
         launch_norm2_partial_b(st, n, R, v, d_ipart_, kRedBlocks);

@@ -192,7 +192,11 @@ __global__ __launch_bounds__(256) void k_aggregate_t(int K, int N, int tiles, co
 // One workgroup per leaf needs enough leaves: 7,680 RWG in 56 leaves (PMCHWT,
 // FP64, both wavenumbers, 346 MB of patterns) take 310 us that way and 88 us in
 // sample tiles, 480 RWG 7.1 and 5.0 us.  With 3,200 leaves (300,000 RWG,
-// 4.9 GB) whole rows stream slightly better, 917 against 944 us.
+// 4.9 GB) whole rows stream slightly better, 917 against 944 us.  Near the line,
+// FP64 PMCHWT, whole rows and tiles in us: 512 leaves 309 and 252, 768 leaves
+// 235 and 232, 824 leaves 679 and 674, 1,272 leaves 209 and 223, 1,968 leaves
+// 967 and 1,046; FP32 with leaves of 19 RWG leans to whole rows earlier (768
+// leaves 27 and 32), with leaves of 90 later (1,392 leaves 520 and 484).
 constexpr int kAggTileLeaves = 1024;
 
 template <typename R>
@@ -1274,10 +1278,15 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 && PM && ROWS == 4 && KS == 1 ?
     }
 }
 
-// Rows per wavefront and sample split by the number of rows: from 16,384 rows
-// whole rows by fours give every SIMD four wavefronts and more (300,000 RWG:
-// 809 us, 6.0 TB/s), fewer take all four wavefronts of a block for the same
-// rows, very few one row a block.
+// Rows per wavefront and sample split by the number of rows: very few rows take
+// one row a block, more take four rows a block whose wavefronts split the
+// samples, and from 16,384 rows a wavefront takes four whole rows (300,000 RWG:
+// 809 us, 6.0 TB/s).  Measured, FP64, PEC and PMCHWT, in us: one row against four
+// rows split, 1,080 RWG 9.1 / 11.0 and 22 / 25, 3,000 RWG 14.9 / 16.5 and 47 / 49,
+// 7,680 RWG 30.6 / 31.3 and 103 / 91; four rows split against four whole rows,
+// 7,680 RWG 31.3 / 31.2 and 91 / 113, 18,750 RWG 64 / 68 and 176 / 196, 147,000
+// RWG 401 / 413 and 1,242 / 1,317 (FP32 690 / 671).  The split form loses only in
+// FP32 PMCHWT at large sizes, so the upper line could lie higher elsewhere.
 template <typename R, bool PM>
 void disagg_one(hipStream_t st, int N, int nw, int ldr, int r0, const int* leaf_of, const int* perm,
                 const DisaggWave<R>& w0, const DisaggWave<R>& w1, double2 scale, double2* y) {
