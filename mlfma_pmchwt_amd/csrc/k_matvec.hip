@@ -1205,14 +1205,15 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 && PM && ROWS == 4 && KS == 1 ?
 #pragma unroll
         for (int u = 0; u < ROWS; ++u)
 #pragma unroll
-            for (int o = 0; o < NO; ++o) {
-                double2 f = widen(wave_sum(s[u][o]));
-                s[u][o] = C{0, 0};
-                if (lane == 0) {
-                    if (add) f = cadd(red[wave][u * NO + o], f);
-                    red[wave][u * NO + o] = f;
+            for (int o = 0; o < NO; ++o) s[u][o] = wave_sum(s[u][o]);
+        if (lane == 0)
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+                for (int o = 0; o < NO; ++o) {
+                    double2& r = red[wave][u * NO + o];
+                    r = add ? cadd(r, widen(s[u][o])) : widen(s[u][o]);
                 }
-            }
     };
     for (int w = 0; w < nw; ++w) {
         const DisaggWave<R> W = w == 0 ? w0 : w1;
@@ -1255,7 +1256,13 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 && PM && ROWS == 4 && KS == 1 ?
                     for (int d = 0; d < 3; ++d) cfma(s[u][o], v[u][d], e[o][d]);
             }
         }
-        if (APART && w == 0) leave(false);
+        if (APART && w == 0) {
+            leave(false);
+#pragma unroll
+            for (int u = 0; u < ROWS; ++u)
+#pragma unroll
+                for (int o = 0; o < NO; ++o) s[u][o] = C{0, 0};
+        }
     }
     leave(APART);
     if (KS > 1) {
