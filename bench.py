@@ -117,8 +117,9 @@ def group_roofline(op, R, dom, groups):
         kern = "k_m2l_cl + k_l2l_row (sibling-cluster translation, then separable anterpolation; FP32 vector ALUs)"
         work, unit, peak, bound = translation_flops(op, R, 2) / launches, "TFLOP/s", FP32_PEAK_TFS, "mfma"
         note = ("compute roofline at the FP32 dense peak; the kernel does its FP32 FMAs on the vector ALUs, where "
-                "packed FP32 instructions are disabled in this build (half that rate); counters: the vector-memory "
-                "address unit is busy about 60% of the kernel's time, VALU issue about 38%")
+                "packed FP32 instructions are disabled in this build (half that rate); counters of the kernels: the "
+                "vector-memory address unit is busy about 57% (translation) and 66% (anterpolation) of their time, "
+                "VALU issue about 46% and 41%")
     elif dom == "aggregate" and op.params.near_precision == 2:
         kern = "k_aggregate_bf3 (split-pair BF16 matrix cores, all right-hand sides)"
         work, unit, peak, bound = far_flops(op, R, dom) / launches, "TFLOP/s", 2500.0, "mfma"
