@@ -97,7 +97,9 @@ T* Engine::dalloc(size_t count) {
             eall64_asked_ = 0;   // given back in vain: the next product may take them again
         }
     }
-    MLFMA_HIP(e);
+    if (e != hipSuccess)
+        throw Error(e == hipErrorOutOfMemory ? MLFMA_ERR_OOM : MLFMA_ERR_HIP,
+                    "hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes: " + hipGetErrorString(e));
     allocs_[p] = count * sizeof(T);
     dev_bytes += count * sizeof(T);
     return static_cast<T*>(p);
@@ -1123,9 +1125,13 @@ void Engine::take_eall(int cols) {
             d_Sall_[w] = dalloc<float2>((size_t)nleaf * ncur * 3 * wd_[w].K[L] * cols);
         }
     } catch (const Error& e) {
-        if (e.code != MLFMA_ERR_OOM || cols == eall_need_) throw;
-        take_eall(eall_need_);   // without the FP64 columns
-        return;
+        if (e.code == MLFMA_ERR_OOM && cols > eall_need_) {
+            take_eall(eall_need_);   // without the FP64 columns
+            return;
+        }
+        eall_need_ = 0;   // fewer right-hand sides may fit
+        dfree(d_Eall_[0], d_Eall_[1], d_Sall_[0], d_Sall_[1]);
+        throw;
     }
     eall_cols_ = cols;
 }

@@ -88,14 +88,15 @@ def test_fp64_buffers_give_way_to_a_basis(mode):
         op.set_apply_precision(api.FP64)
     op.set_tuning(api.FP64, 0, 7)
     taken = _taken(lambda: op.apply(x))
-    assert taken >= 100 * MIB, taken
+    print(f"[buffers] {mode}: {taken // MIB} MiB", flush=True)
+    assert taken >= 192 * MIB      # half of it stands out against what only_free may be off
     all_rhs = op.apply(x)
     if mode == "fp32":
         op.set_apply_precision(api.FP32)
         x32 = op.apply(x)
         op.set_apply_precision(api.FP64)
     op.set_tuning(api.FP64, 0, 5)
-    assert _taken(lambda: op.apply(x)) <= MIB
+    assert _taken(lambda: op.apply(x)) <= 32 * MIB
     op.set_tuning(api.FP64, 0, 7)
     free = 256 * MIB
     basis = op.n * R * 16
@@ -134,7 +135,14 @@ def test_fp64_buffers_are_left_where_little_is_free():
             cases.append((op, x, want))
     with only_free(400 * MIB):
         for op, x, want in cases:
-            assert _taken(lambda: op.apply(x)) <= MIB
+            assert _taken(lambda: op.apply(x)) <= 32 * MIB
             assert relerr(op.apply(x), want) <= 1e-13
+        op, x, want = cases[-1]    # FP32 products of more right-hand sides than fit, then of as many as before
+        op.set_apply_precision(api.FP32)
+        y = op.apply(x)
+        with pytest.raises(api.MlfmaError, match="memory"):
+            op.apply(_block(op, 256))
+        same = np.array_equal(op.apply(x), y)
+        assert same
     for op, _, _ in cases:
         op.close()
