@@ -5,6 +5,7 @@
 #include "setup.hpp"
 
 #include <stdexcept>
+#include <type_traits>
 
 namespace mlfma {
 
@@ -563,6 +564,14 @@ void launch_excitation(hipStream_t st, int N, int mode, const RwgGeo* geo, const
 // follow once per direction instead of once per point.  Bound by the FP64 sine
 // and cosine of every (point, direction).  181 directions of 75,000 RWG: 879 us
 // with one direction per thread and projected points, now 636.
+// One direction per thread is for launches too small to fill the chip with four,
+// and a single chain of latency: it takes its record into registers at once (138
+// of them; with four directions there is no room) and hides the phase's origin
+// from the compiler, which otherwise computes the sine's reduction of huge
+// arguments for every point instead of branching round it.  Without the two, 361
+// directions of 2,430 RWG took 91 us and 37 of 12,000 took 48, now 54 and 30;
+// four directions are faster without them (189 us, 203 with the hidden phase:
+// 361 of 12,000).
 template <int NA>
 __global__ __launch_bounds__(256) void k_farfield(int N, int pmchwt, const RwgGeo* __restrict__ geo,
                                                   const int* __restrict__ perm, GaussRule g, double2 k, int nang,
@@ -582,7 +591,7 @@ __global__ __launch_bounds__(256) void k_farfield(int N, int pmchwt, const RwgGe
     for (int a = 0; a < NA; ++a) V[a][0] = V[a][1] = V[a][2] = make_double2(0, 0);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < N) {
-        const RwgGeo& G = geo[i];
+        std::conditional_t<NA == 1, const RwgGeo, const RwgGeo&> G = geo[i];
         for (int q = 0; q < g.n; ++q) {
             const double wl = G.len * g.w[q];
             for (int side = 1; side >= 0; --side) {
@@ -590,8 +599,9 @@ __global__ __launch_bounds__(256) void k_farfield(int N, int pmchwt, const RwgGe
                 const R3 rho = scl3(side == 1 ? sub3(r, mk(G.vf[1])) : sub3(mk(G.vf[0]), r), wl);
 #pragma unroll
                 for (int a = 0; a < NA; ++a) {
-                    // e^{+jk r.p}
-                    const double2 e = expmjk(make_double2(-k.x, -k.y), dot3(r, rd[a]));
+                    double rp = dot3(r, rd[a]);
+                    if (NA == 1) asm("" : "+v"(rp));
+                    const double2 e = expmjk(make_double2(-k.x, -k.y), rp);   // e^{+jk r.p}
                     V[a][0] = cadd(V[a][0], cscale(e, rho.x));
                     V[a][1] = cadd(V[a][1], cscale(e, rho.y));
                     V[a][2] = cadd(V[a][2], cscale(e, rho.z));
@@ -637,7 +647,9 @@ void launch_farfield(hipStream_t st, int N, int pmchwt, const RwgGeo* geo, const
                      double2 k, int nang, const double* dirs, const double2* I, size_t istride, double2* partial,
                      int nblocks) {
     // four directions per thread from 16 workgroups per CU of one each, so that a
-    // quarter of them still fills the chip
+    // quarter of them still fills the chip.  Near the line the two are alike
+    // (12,000 RWG: 84 directions one by one 57.6 us, 88 and 100 by fours 61.8 and
+    // 62.6); below it one by one wins (60: 45.3), above it fours do (361: 189).
     if ((long long)nblocks * nang >= 4096)
         k_farfield<4><<<dim3(nblocks, (nang + 3) / 4), 256, 0, st>>>(N, pmchwt, geo, perm, g, k, nang, dirs, I, istride,
                                                                      partial);
