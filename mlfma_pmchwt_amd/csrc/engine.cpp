@@ -2328,10 +2328,10 @@ void Engine::inner_near_solve(const double2* V, double2* Z, int R, int prec) {
     // all of it once, after the last step.  A column whose recurrence has ended
     // (v = 0, or breakdown) is scaled by zero and stays zero through the remaining
     // steps, which the host leaves out.  (They still run where every column has
-    // ended: a solve's block has a live column, so only a zero block given to the
-    // preconditioner alone, or fewer unknowns than steps, pays for them.)  With the
-    // host between the reductions (five waits per step) a 12-iteration solve of 8
-    // right-hand sides at 31,740 unknowns took 44.8 ms, so 30.8.
+    // ended; a solve's block has a live column, so only fewer unknowns than steps
+    // bring that about.)  With the host between the reductions (five waits per
+    // step) a 12-iteration solve of 8 right-hand sides at 31,740 unknowns took
+    // 44.8 ms, so 30.8.
     auto at = [&](int j) { return (size_t)R * (1 + (size_t)j * (j + 2)); };   // step j's block
     auto norm_to = [&](const double2* v, double2* out) {
         launch_norm2_partial_b(st, n, R, v, d_ipart_, kRedBlocks);
