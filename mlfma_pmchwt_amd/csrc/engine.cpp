@@ -679,11 +679,15 @@ void Engine::fill_near(int planes, const NearConsts& c) {
 // PMCHWT unknowns in 56 leaves of 25 MB took 1.27 ms (1.1 TB/s).  With column
 // ranges of about 1/1024 of all entries (at least 128 KB, at least 16 columns)
 // every CU holds several (the same product: 0.19 ms); their partial sums cost
-// a second, small launch (about 4 us), so leaves under 512 KB stay whole (FP64
-// PMCHWT: 768 leaves of 19 RWG whole 42 us, split 49; of 31 RWG, at the line, 102
-// and 104; 392 leaves of 48 RWG 165 and 142), and so do 2,048 and more leaves
-// (1,392 leaves 1,127 and 1,067 us, 1,968 leaves 796 and 791, 2,264 leaves 1,160
-// and 1,164; 300,000 RWG in 3,200 leaves of 2.1 MB stream at 5.9 TB/s unsplit).
+// a second, small launch and traffic of their own, so a product stays whole
+// while its largest leaf, as stored, is under 1.25 MB, or half that with at most
+// 128 leaves, half as many as CUs.  Whole and split, us: FP64 392 leaves of 0.87
+// MB 47 and 59, 584 of 1.20 MB 67 and 71, 392 of 1.29 MB 67 and 67, 584 of 1.70 MB
+// 96 and 91; FP32 584 of 0.60 MB 40 and 51, 392 of 0.94 MB 56 and 56, 272 of 1.23
+// MB 60 and 56; 128 leaves of 0.50 MB (FP64) 14.4 and 15.6, of 0.71 MB 28 and 20.
+// 2,048 and more leaves stay whole too (1,392 leaves 1,127 and 1,067 us, 1,968
+// leaves 796 and 791, 2,264 leaves 1,160 and 1,164; 300,000 RWG in 3,200 leaves of
+// 2.1 MB stream at 5.9 TB/s unsplit).
 void Engine::build_near_split(int planes) {
     const std::vector<int>& lp = tree.leaf_ptr;
     const size_t esize = sizeof(double2);
@@ -693,8 +697,9 @@ void Engine::build_near_split(int planes) {
         total += b;
         most = std::max(most, b);
     }
-    nd_.nsplit = 0;
-    if (nleaf >= 2048 || most < (512u << 10)) return;
+    nd_.nsplit = nd_.nsplit32 = 0;
+    const size_t line = nleaf <= 128 ? 640u << 10 : 1280u << 10;
+    if (nleaf >= 2048 || most < line) return;
     const size_t target = std::max<size_t>(total / 1024, 128u << 10);
     std::vector<int4> split;
     std::vector<long long> part_ptr(nleaf + 1, 0);
@@ -711,6 +716,7 @@ void Engine::build_near_split(int planes) {
         return (long long)(a.z - a.y) * (lp[a.x + 1] - lp[a.x]) > (long long)(b.z - b.y) * (lp[b.x + 1] - lp[b.x]);
     });
     nd_.nsplit = (int)split.size();
+    nd_.nsplit32 = most / 2 < line ? 0 : nd_.nsplit;
     nd_.split = upload(split);
     nd_.part_ptr = upload(part_ptr);
     nd_.part = dalloc<double2>((size_t)part_ptr[nleaf]);

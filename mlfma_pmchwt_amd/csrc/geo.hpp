@@ -60,8 +60,9 @@ struct NearDev {
     const int* colref;        // caller-order index of x for every column
     int nitem;                // matrix-core work items: (target, first 16-row tile), <= 4 tiles each,
     const int2* items;        // by decreasing rows * C_t
-    int nsplit;               // column-range items of the single-vector product (0: one workgroup per leaf):
-    const int4* split;        // (target, first column, end column, index among the target's items), largest first
+    int nsplit;               // column-range items of the single-vector product (0: one workgroup per leaf)
+    int nsplit32;             // the same for entries stored in FP32: nsplit or 0
+    const int4* split;        // items: (target, first column, end column, index among the target's items), largest first
     const long long* part_ptr;   // per target, first of its items' partial sums in part: [item][current][row]
     double2* part;
     const int* leaf_of;       // leaf of every internal row

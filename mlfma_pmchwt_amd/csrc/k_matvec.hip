@@ -1635,13 +1635,14 @@ __global__ __launch_bounds__(256) void k_near_fold(NearDev nd, const int* __rest
 template <typename S>
 void launch_near(hipStream_t st, const NearDev& nd, const cplx_t<S>* Z, const double2* x, double2* y) {
     if (nd.nleaf == 0) return;
-    if (nd.nsplit > 0) {   // few or large leaves (Engine::build_near)
+    const int nsplit = sizeof(S) == 8 ? nd.nsplit : nd.nsplit32;
+    if (nsplit > 0) {   // few or large leaves (Engine::build_near_split)
         const int NX = nd.planes == 1 ? 1 : 2, fb = (NX * nd.N + 255) / 256;
         if (nd.planes == 1) {
-            k_near<S, 1, 512, 8, 1024, true><<<nd.nsplit, 512, 0, st>>>(nd, Z, x, y, nd.part);
+            k_near<S, 1, 512, 8, 1024, true><<<nsplit, 512, 0, st>>>(nd, Z, x, y, nd.part);
             k_near_fold<1><<<fb, 256, 0, st>>>(nd, nd.leaf_of, nd.part, y);
         } else {
-            k_near<S, 3, 512, 4, 512, true><<<nd.nsplit, 512, 0, st>>>(nd, Z, x, y, nd.part);
+            k_near<S, 3, 512, 4, 512, true><<<nsplit, 512, 0, st>>>(nd, Z, x, y, nd.part);
             k_near_fold<3><<<fb, 256, 0, st>>>(nd, nd.leaf_of, nd.part, y);
         }
         return;

@@ -8,11 +8,13 @@ from mlfma_pmchwt_amd import api, geometry
 pytestmark = pytest.mark.gpu
 
 # leaves of 13 to 50 rows (kept whole), of about 100 (several column groups per workgroup), and of
-# more than 512 (several row passes of a workgroup, one column group); one and three planes, both storages
+# more than 512 (several row passes of a workgroup, one column group); one and three planes, both storages;
+# the last pair has 392 leaves of up to 1.3 MB in FP64: column ranges there, whole in FP32
 CASES = [("whole", 4, 0.5, 0.3, api.PMCHWT, api.FP64), ("groups", 12, 0.4, 0.3, api.EFIE, api.FP64),
          ("groups", 9, 0.4, 0.3, api.PMCHWT, api.FP64), ("rows", 17, 0.45, 0.45, api.EFIE, api.FP64),
          ("rows", 17, 0.45, 0.45, api.PMCHWT, api.FP64), ("groups", 11, 0.4, 0.3, api.CFIE, api.FP32),
-         ("groups", 9, 0.4, 0.3, api.PMCHWT, api.FP32)]
+         ("groups", 9, 0.4, 0.3, api.PMCHWT, api.FP32),
+         ("whole", 20, 1.4, 0.3, api.PMCHWT, api.FP64), ("whole", 20, 1.4, 0.3, api.PMCHWT, api.FP32)]
 
 
 @pytest.mark.parametrize("kind,freq,radius,leaf,ie,near", CASES)
