@@ -826,7 +826,7 @@ void Engine::disaggregate(double2* y, int ldr, int r0, int rb) {
         const bool pm = ie == MLFMA_PMCHWT;
         // the split-pair product reads Eall as BF16 pairs
         const bool split = std::is_same<R, float>::value && d_Vb_[0] != nullptr;
-        const int lde = eall_ld(eall_R_);
+        const int lde = eall_stride(eall_R_);
         cplx_t<R>* E[2] = {reinterpret_cast<cplx_t<R>*>(d_Eall_[0]), reinterpret_cast<cplx_t<R>*>(d_Eall_[1])};
         const FarDev<R>& F1 = far<R>(0);
         if (!pm) {
@@ -1071,16 +1071,16 @@ void Engine::apply_block(const double2* X, double2* Y, int R, int prec, const fl
         eall_R_ = 0;
         timed(4, 1, [&] {
             if (!f32)
-                launch_disagg_all<double>(st, n, eall_ld(n), R, nd_, pm, wd_[0].K[L], far<double>(0).Vf,
+                launch_disagg_all<double>(st, n, eall_stride(n), R, nd_, pm, wd_[0].K[L], far<double>(0).Vf,
                                           reinterpret_cast<const double2*>(d_Eall_[0]), pm ? wd_[1].K[L] : 0,
                                           pm ? far<double>(1).Vf : nullptr,
                                           reinterpret_cast<const double2*>(d_Eall_[1]), Y + s0);
             else if (d_Vb_[0])   // split-pair BF16 (near_precision = MLFMA_BF16)
-                launch_disagg_bf3(st, R, eall_ld(R), nd_, pm, wd_[0].K[L], d_Vb_[0], reinterpret_cast<const uint2*>(d_Eall_[0]),
+                launch_disagg_bf3(st, R, eall_stride(R), nd_, pm, wd_[0].K[L], d_Vb_[0], reinterpret_cast<const uint2*>(d_Eall_[0]),
                                   pm ? wd_[1].K[L] : 0, pm ? d_Vb_[1] : nullptr,
                                   reinterpret_cast<const uint2*>(d_Eall_[1]), Y);
             else
-                launch_disagg_all<float>(st, R, eall_ld(R), R, nd_, pm, wd_[0].K[L], far<float>(0).Vf, d_Eall_[0],
+                launch_disagg_all<float>(st, R, eall_stride(R), R, nd_, pm, wd_[0].K[L], far<float>(0).Vf, d_Eall_[0],
                                          pm ? wd_[1].K[L] : 0, pm ? far<float>(1).Vf : nullptr, d_Eall_[1], Y);
         });
     }

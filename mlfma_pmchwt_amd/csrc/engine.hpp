@@ -325,8 +325,12 @@ private:
     int eall64_asked_ = 0;   // FP64 columns that were taken or did not fit
     int eall_R_ = 0;   // > 0 while a batched matvec defers its disaggregation to one all-RHS product
     static constexpr int kAll64 = 32;   // FP64 columns of an all-RHS product
-    // columns of Eall, padded so that the passes' 2 to 8 columns start on 64-byte boundaries
+    // columns taken for R of Eall, and from one row of it to the next: padded so that the passes'
+    // 2 to 8 columns start on 64-byte boundaries, but not below 8, where the padding would be most of
+    // it (61,440 FP32 PMCHWT unknowns, 2 right-hand sides: folding and disaggregation 587 us padded,
+    // 386 not; 5: 790 and 622)
     static int eall_ld(int R) { return (R + 7) & ~7; }
+    static int eall_stride(int R) { return R < 8 ? R : eall_ld(R); }
     float2* d_xf_ = nullptr;    // FP32 copy of the matrix-core near product's input, nunk x xf_cap_
     int xf_cap_ = 0;
     unsigned* d_xb_ = nullptr;  // BF16 copy of the preconditioner's near-product input, nunk x poly_cap_

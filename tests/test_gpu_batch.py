@@ -195,7 +195,7 @@ def test_cluster_translation_matches_per_box(name):
 
 
 @pytest.mark.parametrize("name", ["efie_ml", "pmchwt_lossy_ml", "pmchwt_1lvl"])
-@pytest.mark.parametrize("R", [5, 13, 21])
+@pytest.mark.parametrize("R", [2, 5, 7, 13, 21])
 def test_all_rhs_far_ends_match_per_pass(name, R):
     """FP32 batched matvecs aggregate all right-hand sides into every pass's
     leaf workspaces in one matrix-core product and disaggregate them in
