@@ -1055,13 +1055,19 @@ void launch_m2l_cl(hipStream_t st, int ncur, int ncl, int K, const int* cl_child
     // FP64 (16-byte loads both): whole matvec of C5 at 64 right-hand sides, FP32:
     // 6 x 2 27.5 ms, 6 x 1 29.3, 12 x 1 28.5, 3 x 2 28.4, 8 x 2 31.8 (spills into
     // the accumulator file); FP64 lossy sphere at 13: 6 x 1 5.57, 3 x 1 5.77.
-    // Below 4 the level has too few wavefronts to lose any: PMCHWT of 15k unknowns,
-    // one vector: 401 us as here, 409 with the wide form.
+    // A level that so has fewer than 1024 wavefronts, one per SIMD, takes one
+    // sample per lane, and below 512 of those 3 columns: a wavefront's walk through
+    // its sources then bounds the time (5,070 EFIE unknowns in 56 leaves, 64
+    // right-hand sides in passes of 8: 236 us of translation with 6 x 2, 180 with 6
+    // x 1, 143 with 3 x 1; 52,920 in 824 leaves, 4 of them: 216, 161, 161).  One
+    // vector: PMCHWT of 15k unknowns 401 us with 3 columns, 409 with the wide form.
     constexpr bool f64 = sizeof(R) == 8;
+    const long long cols = (long long)ncl * ncur / 2;   // wavefronts per sample tile, 6 columns each
     const bool wide = ncur >= 4;
-    const int sp = !f64 && wide && (K & 1) == 0 ? 2 : 1;   // pairs need rows of whole pairs (K = 2 L^2 is even)
+    // pairs need rows of whole pairs (K = 2 L^2 is even)
+    const int sp = !f64 && wide && (K & 1) == 0 && cols * ((K + 127) / 128) >= 1024 ? 2 : 1;
     const int kt = (K + 64 * sp - 1) / (64 * sp);
-    const int cpt = wide || (!f64 && ncur == 2) ? 6 : 3;
+    const int cpt = (wide || (!f64 && ncur == 2)) && cols * kt >= 512 ? 6 : 3;
     const int ncg = ncur * 3 / cpt;
     // Wavefronts (neighbouring clusters) per workgroup; single ones where a level
     // does not give each SIMD four wavefronts.

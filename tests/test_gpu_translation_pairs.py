@@ -47,6 +47,25 @@ def _uneven_level(op, currents, samples):
     return False
 
 
+def _forms(op, currents, f64):
+    """(columns, samples) per lane that the levels of one pass take, by the wavefronts they give."""
+    out = set()
+    for level in range(2, op.max_level + 1):
+        clusters = int(((np.unique(op.level(level)[3], return_counts=True)[1] + 3) // 4).sum())
+        tiles = -(-2 * op.grid(1, level)[0] ** 2 // 64)
+        pairs = not f64 and currents >= 4 and clusters * (currents // 2) * (-(-tiles // 2)) >= 1024
+        waves = clusters * currents / 2 * (-(-tiles // 2) if pairs else tiles)
+        out.add((6 if currents >= (4 if f64 else 2) and waves >= 512 else 3, 2 if pairs else 1))
+    return out
+
+
+@pytest.mark.parametrize("cur,f64,forms", [(4, False, {(3, 1), (6, 1)}), (8, False, {(6, 1), (6, 2)}),
+                                           (4, True, {(3, 1), (6, 1)})])
+def test_forms_reached(cur, f64, forms):
+    """The meshes of this file take every form of the kernel (passes of 4 and 8 vectors of one current)."""
+    assert _forms(_operator("cfie"), cur, f64) | _forms(_operator("cfie_four"), cur, f64) >= forms
+
+
 @pytest.mark.parametrize("name", list(CASES))
 @pytest.mark.parametrize("nrhs", [1, 2, 4, 8, 15])
 def test_translation_pairs_match_per_box(name, nrhs):
